@@ -84,6 +84,18 @@ int ensure_scratch(pargo_ctx *ctx, size_t bytes)
     return PARGO_OK;
 }
 
+int ensure_report(pargo_ctx *ctx)
+{
+    if (ctx->report) return PARGO_OK;
+    hipError_t e = alloc_should_fail("report words") ? hipErrorOutOfMemory
+                                                     : hipHostMalloc(&ctx->report, 64, hipHostMallocDefault);
+    if (e != hipSuccess) {
+        ctx->report = nullptr;
+        return fail(ctx, PARGO_E_NOMEM, "hipHostMalloc of the report words: %s%s", hipGetErrorString(e), injected_note());
+    }
+    return PARGO_OK;
+}
+
 // The reference tests NoData per window value as fabs(d - noData) < eps in
 // double (slopeOperator.cpp:68, d8Operator.cpp:46).  d is a float widened to
 // double, and |RN(d - noData)| is unimodal in d, so the floats passing the
@@ -190,6 +202,7 @@ int pargo_destroy(pargo_ctx *ctx)
     if (ctx->own_stream) hipStreamSynchronize(ctx->own_stream);
     if (ctx->stream && ctx->stream != ctx->own_stream) hipStreamSynchronize(ctx->stream);
     if (ctx->scratch) hipFree(ctx->scratch);
+    if (ctx->report) hipHostFree(ctx->report);
     pargo::free_batch_plan(ctx);
     if (ctx->fix_mem) hipFree(ctx->fix_mem);
     if (ctx->switch_event) hipEventDestroy(ctx->switch_event);

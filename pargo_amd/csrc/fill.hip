@@ -82,7 +82,7 @@ struct FillParams {
     unsigned *__restrict__ flags;    // [2][tiles]: what the tile's next visit starts from (even, odd passes)
     unsigned *__restrict__ count;    // [3]: entries of the worklists, pass p's in count[p % 3]
     int *__restrict__ list;          // [2][tiles]: tiles of the pass (even, odd)
-    double *__restrict__ edge;       // [tiles][2][kTH]: W of each tile's first and last column
+    double *__restrict__ edge;       // [tiles][2][kTH]: W of each tile's first and last column, NoData as +infinity
     unsigned *__restrict__ range;    // [0] smallest valid elevation (ordered bits), [1] NaN cells
     long long pitch;
     int rows, cols, tiles_x, tiles_y;
@@ -167,34 +167,36 @@ __device__ __forceinline__ void append_tiles(const FillParams &p, int t, bool fi
 constexpr int kInitBatch = 8;  // rows whose loads are in flight together
 static_assert(kTH % kInitBatch == 0, "whole batches");
 
-__global__ __launch_bounds__(256) void fill_init_kernel(FillParams p)
+// What the walk over a tile's rows finds.
+struct InitSeen {
+    unsigned least = 0xffffffffu, nans = 0;            // per lane: smallest elevation (ordered bits), NaN cells
+    unsigned long long any = 0, top = 0, bottom = 0;  // opened or excluded cells: all rows, the first and the last row
+};
+
+// INNER: every cell of the tile and around it is an interior cell, so no row
+// or column is tested (all tiles but the border's; 0.92 -> INIT_MS ms at
+// 16384^2, the tests being scalar work for every row).
+template <bool INNER>
+__device__ __forceinline__ void fill_init_tile(const FillParams &p, int ty, int tx, int lane, double *edge, InitSeen &o)
 {
-    const int lane = threadIdx.x & 63;
-    const int tx = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-    const int ty = blockIdx.y;
-    if (tx >= p.tiles_x) return;  // the whole wave
     const int c = tx * kTW + lane, r0 = ty * kTH;
-    const int ce = lane == 0 ? c - 1 : c + 1;  // lanes 0 and 63: the column beside the tile
-    const bool cin = c >= 1 && c <= p.cols - 2;
-    const bool ein = (lane == 0 || lane == 63) && ce >= 1 && ce <= p.cols - 2;
+    // lanes 0 and 63: the column beside the tile (the others: their own)
+    const int ce = lane == 0 ? c - 1 : (lane == 63 ? c + 1 : c);
+    const bool cin = INNER || (c >= 1 && c <= p.cols - 2), ein = INNER || (ce >= 1 && ce <= p.cols - 2);
     const bool opens = p.opens != 0;
+    auto rin = [&](int r) { return INNER || (r >= 1 && r <= p.rows - 2); };
     auto load = [&](int r, float &f, float &e) {
-        const bool rin = r >= 1 && r <= p.rows - 2;
-        f = rin && cin ? p.dem[(long long)r * p.pitch + c] : 0.0f;
-        e = rin && ein ? p.dem[(long long)r * p.pitch + ce] : 0.0f;
+        const float *row = p.dem + (long long)r * p.pitch;
+        f = rin(r) && cin ? row[c] : 0.0f;
+        e = rin(r) && ein ? row[ce] : 0.0f;
     };
     // excluded cells of row r, and the same widened by a column
     auto excluded = [&](int r, float f) -> unsigned long long {
-        const bool rin = r >= 1 && r <= p.rows - 2;
-        return __builtin_amdgcn_ballot_w64(!(rin && cin) || is_nd(p, f));
+        return __builtin_amdgcn_ballot_w64(!(rin(r) && cin) || is_nd(p, f));
     };
     auto widened = [&](int r, unsigned long long m, float e) -> unsigned long long {
-        const bool rin = r >= 1 && r <= p.rows - 2;
-        const unsigned long long b = __builtin_amdgcn_ballot_w64((lane == 0 || lane == 63) && (!(rin && ein) || is_nd(p, e)));
-        return m | (m << 1) | (m >> 1) | b;
+        return m | (m << 1) | (m >> 1) | __builtin_amdgcn_ballot_w64(!(rin(r) && ein) || is_nd(p, e));
     };
-    unsigned least = 0xffffffffu, nans = 0;
-    unsigned long long any = 0, top = 0, bottom = 0;  // opened or excluded cells: all rows, the first and the last row
     float f, e;
     load(r0 - 1, f, e);
     unsigned long long above = widened(r0 - 1, excluded(r0 - 1, f), e);
@@ -202,7 +204,7 @@ __global__ __launch_bounds__(256) void fill_init_kernel(FillParams p)
     float cur = f;
     unsigned long long cur_m = excluded(r0, f), cur_w = widened(r0, cur_m, e);
     for (int b = 0; b < kTH; b += kInitBatch) {
-        if (r0 + b >= p.rows) break;
+        if (!INNER && r0 + b >= p.rows) break;
         float fn[kInitBatch], en[kInitBatch];  // the rows below each row of the batch
 #pragma unroll
         for (int k = 0; k < kInitBatch; k++) load(r0 + b + k + 1, fn[k], en[k]);
@@ -210,26 +212,26 @@ __global__ __launch_bounds__(256) void fill_init_kernel(FillParams p)
         for (int k = 0; k < kInitBatch; k++) {
             const int r = r0 + b + k;
             const unsigned long long next_m = excluded(r + 1, fn[k]), next_w = widened(r + 1, next_m, en[k]);
-            if (r < p.rows) {
+            if (INNER || r < p.rows) {
                 const unsigned long long open = above | cur_w | next_w;
                 const bool valid = !((cur_m >> lane) & 1ull);
                 double w0 = p.nodata;
                 if (valid) {
                     w0 = opens && ((open >> lane) & 1ull) ? fmin((double)cur, kStart) : kStart;
                     if (cur != cur) {
-                        nans++;
+                        o.nans++;
                     } else {
                         unsigned u = __float_as_uint(cur);  // order-preserving map of floats to unsigned
                         u = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-                        least = u < least ? u : least;
+                        o.least = u < o.least ? u : o.least;
                     }
                 }
                 // streamed past the caches: the passes read W back much later
-                if (c < p.cols) __builtin_nontemporal_store(w0, &p.w[(long long)r * p.pitch + c]);
-                if ((lane == 0 || lane == 63) && c < p.cols) p.edge[edge_index(p, ty, tx, lane != 0, b + k)] = w0;
-                any |= open;
-                if (b + k == 0) top = open;
-                if (b + k == kTH - 1) bottom = open;
+                if (INNER || c < p.cols) __builtin_nontemporal_store(w0, &p.w[(long long)r * p.pitch + c]);
+                if (lane == 0 || lane == 63) edge[(lane ? kTH : 0) + b + k] = valid ? w0 : __builtin_huge_val();
+                o.any |= open;
+                if (b + k == 0) o.top = open;
+                if (b + k == kTH - 1) o.bottom = open;
             }
             above = cur_w;
             cur_w = next_w;
@@ -237,20 +239,38 @@ __global__ __launch_bounds__(256) void fill_init_kernel(FillParams p)
             cur = fn[k];
         }
     }
+}
+
+__global__ __launch_bounds__(256) void fill_init_kernel(FillParams p)
+{
+    __shared__ double edges[4][2 * kTH];  // each wave's first and last column
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int tx = (int)blockIdx.x * 4 + wave, ty = blockIdx.y;
+    if (tx >= p.tiles_x) return;  // the whole wave
+    InitSeen o;
+    if (ty > 0 && tx > 0 && (ty + 1) * kTH + 1 < p.rows && (tx + 1) * kTW + 1 < p.cols)
+        fill_init_tile<true>(p, ty, tx, lane, edges[wave], o);
+    else
+        fill_init_tile<false>(p, ty, tx, lane, edges[wave], o);
+    // lanes 0-31 the first column, lanes 32-63 the last: one run of 512 bytes
+    // (rows and columns past the raster are never read)
+    p.edge[edge_index(p, ty, tx, 0, 0) + lane] = edges[wave][lane];
     // the tiles with an opened cell in them or around them
     {
         const int dy = lane / 3 - 1, dx = lane % 3 - 1;
         const int nty = ty + dy, ntx = tx + dx;
-        const unsigned long long m = dy < 0 ? top : (dy > 0 ? bottom : any);
+        const unsigned long long m = dy < 0 ? o.top : (dy > 0 ? o.bottom : o.any);
         const bool need = lane < 9 && (dx < 0 ? (m & 1ull) != 0 : (dx > 0 ? (m >> 63) != 0 : m != 0)) && nty >= 0 &&
                           nty < p.tiles_y && ntx >= 0 && ntx < p.tiles_x;
         const int t = nty * p.tiles_x + ntx;
         const bool first = need && flag_tile(p, t, kAll, 0);
         append_tiles(p, t, first, 0);
     }
+    unsigned least = o.least, nans = o.nans;
     for (int off = 32; off > 0; off >>= 1) {
-        const unsigned o = __shfl_xor(least, off);
-        least = o < least ? o : least;
+        const unsigned u = __shfl_xor(least, off);
+        least = u < least ? u : least;
         nans += __shfl_xor(nans, off);
     }
     if (lane == 0) {
@@ -319,54 +339,79 @@ __device__ __forceinline__ void fill_tile(const FillParams &p, int tile, int pas
     bool up_sent = false, down_sent = false;
     unsigned touched = 0;                              // bit k: row r0 + k changed
     unsigned long long cols = 0, first = 0, last = 0;  // columns that changed: any row, the first, the last row
-    unsigned lrows = 0, rrows = 0;                     // rows whose first / last column changed
     auto row_h = [&](double v, double e) -> double { return vmin(vmin(dpp_from_left(v, e), v), dpp_from_right(v, e)); };
     auto load = [&]() {
-        const bool cin = c < p.cols;
+        double eu = inf, ed = inf, wu = p.nodata, wd = p.nodata;
+        // the edge copies beside the tile: the left tile's last column (which
+        // precedes this tile's copies) and the right tile's first
         const bool ein = (lane == 0 && tx > 0) || (lane == 63 && tx + 1 < p.tiles_x);
-        // the edge copies beside the tile: the left tile's last column (right
-        // after it, in the copies' order, comes this tile's first), and the
-        // right tile's first
-        const int eoff = lane == 0 ? -kTH : 2 * kTH;
-        double eu = p.nodata, ed = p.nodata, wu = p.nodata, wd = p.nodata;
-        auto get = [&](int r, double &v, double &e) {
-            v = p.nodata;
-            e = p.nodata;
-            if (r >= 0 && r < p.rows) {
-                const double *row = p.w + ((long long)r * p.pitch + tx * kTW);
-                const double *edge = p.edge + edge_index(p, r / kTH, tx, 0, r % kTH);
-                if (cin) v = row[(unsigned)lane];
-                if (ein) e = edge[eoff];
-            }
-        };
+        const double *edge = p.edge + (edge_index(p, ty, tx, 0, wave * kRW) + (lane == 0 ? -kTH : 2 * kTH));
+        const double *row = p.w + ((long long)r0 * p.pitch + tx * kTW);
+        const float *drow = p.dem + ((long long)r0 * p.pitch + tx * kTW);
         // every load is issued before the first value is used
-        get(r0 - 1, wu, eu);
+        if (ty > 0 && r0 + kRW < p.rows && tx * kTW + kTW <= p.cols) {
+            // every row the wave reads lies in the raster, and so do its columns
+            const double *rw = row - p.pitch;
+            wu = rw[(unsigned)lane];
 #pragma unroll
-        for (int k = 0; k < kRW; k++) {
-            get(r0 + k, w[k], side[k]);
-            const float *drow = p.dem + ((long long)(r0 + k) * p.pitch + tx * kTW);
-            dem[k] = cin && r0 + k < p.rows ? drow[(unsigned)lane] : 0.0f;
+            for (int k = 0; k < kRW; k++) {
+                rw += p.pitch;
+                w[k] = rw[(unsigned)lane];
+                dem[k] = drow[(unsigned)lane];
+                drow += p.pitch;
+                side[k] = inf;
+            }
+            rw += p.pitch;
+            wd = rw[(unsigned)lane];
+            if (ein) {
+                // the tile rows above and below hold their own copies
+                const long long stride = (long long)p.tiles_x * 2 * kTH;
+                eu = wave > 0 ? edge[-1] : edge[kTH - 1 - stride];
+                ed = wave < kWaves - 1 ? edge[kRW] : edge[stride - (kTH - kRW)];
+#pragma unroll
+                for (int k = 0; k < kRW; k++) side[k] = edge[k];
+            }
+        } else {
+            const bool cin = c < p.cols;
+            auto get = [&](int r, double &v, double &e) {
+                v = p.nodata;
+                e = inf;
+                if (r >= 0 && r < p.rows) {
+                    if (cin) v = p.w[(long long)r * p.pitch + c];
+                    if (ein) e = p.edge[edge_index(p, r / kTH, tx, 0, r % kTH) + (lane == 0 ? -kTH : 2 * kTH)];
+                }
+            };
+            get(r0 - 1, wu, eu);
+#pragma unroll
+            for (int k = 0; k < kRW; k++) {
+                get(r0 + k, w[k], side[k]);
+                dem[k] = cin && r0 + k < p.rows ? p.dem[(long long)(r0 + k) * p.pitch + c] : 0.0f;
+            }
+            get(r0 + kRW, wd, ed);
         }
-        get(r0 + kRW, wd, ed);
         // NoData reads as +infinity: never a minimum, never lowered
         auto open = [&](double v) -> double { return v == p.nodata ? inf : v; };
 #pragma unroll
         for (int k = 0; k < kRW; k++) {
             w[k] = open(w[k]);
-            side[k] = open(side[k]);
             dem[k] = w[k] == inf ? __builtin_huge_valf() : dem[k];
             h[k] = row_h(w[k], side[k]);
         }
-        if (!up_sent) up = row_h(open(wu), open(eu));
-        if (!down_sent) down = row_h(open(wd), open(ed));
+        if (!up_sent) up = row_h(open(wu), eu);
+        if (!down_sent) down = row_h(open(wd), ed);
     };
     // One evaluation of row r0 + k by every lane.
     auto evaluate = [&](int k) {
         dirty &= ~(1u << k);
-        const double m = vmin(vmin(k == 0 ? up : h[k > 0 ? k - 1 : 0], h[k]), k == kRW - 1 ? down : h[k < kRW - 1 ? k + 1 : 0]);
-        double d;  // widened where it is used: kept widened, the rows would take 16 more registers
-        asm volatile("v_cvt_f64_f32 %0, %1" : "=v"(d) : "v"(dem[k]));
-        const double t = vmax(d, m + kGap);
+        const double above = k == 0 ? up : h[k > 0 ? k - 1 : 0], below = k == kRW - 1 ? down : h[k < kRW - 1 ? k + 1 : 0];
+        // t = max(dem, min(h(r-1), h(r), h(r+1)) + gap), as one block: the
+        // DEM value is widened where it is used (kept widened, the rows would
+        // take 16 more registers)
+        double t, d;
+        asm volatile("v_min_f64 %0, %2, %3\n\tv_cvt_f64_f32 %1, %5\n\tv_min_f64 %0, %0, %4\n\t"
+                     "v_add_f64 %0, %0, %6\n\tv_max_f64 %0, %1, %0"
+                     : "=&v"(t), "=&v"(d)
+                     : "v"(above), "v"(h[k]), "v"(below), "v"(dem[k]), "s"(kGap));
         const unsigned long long ch = __builtin_amdgcn_ballot_w64(t < w[k]);
         if (ch != 0) {
             w[k] = vmin(w[k], t);
@@ -374,8 +419,6 @@ __device__ __forceinline__ void fill_tile(const FillParams &p, int tile, int pas
             dirty |= (7u << k >> 1) & kRows;
             touched |= 1u << k;
             cols |= ch;
-            lrows |= (unsigned)(ch & 1ull) << k;
-            rrows |= (unsigned)(ch >> 63) << k;
             if (k == 0) first |= ch;
             if (k == kRW - 1) last |= ch;
         }
@@ -449,10 +492,8 @@ __device__ __forceinline__ void fill_tile(const FillParams &p, int tile, int pas
         if (lane == 0) {
             // a changed side row matters to the rows beside it and next to
             // that: the band's own and, from its first or last row, the next
-            const unsigned lb = (lrows ? 1u << wave : 0u) | ((lrows & 1u) << wave >> 1) |
-                                ((lrows >> (kRW - 1) & 1u) << wave << 1);
-            const unsigned rb = (rrows ? 1u << wave : 0u) | ((rrows & 1u) << wave >> 1) |
-                                ((rrows >> (kRW - 1) & 1u) << wave << 1);
+            const unsigned bands = 1u << wave | (touched & 1u) << wave >> 1 | (touched >> (kRW - 1) & 1u) << wave << 1;
+            const unsigned lb = cols & 1ull ? bands : 0u, rb = cols >> 63 ? bands : 0u;
             unsigned o = (lb & 15u) * kLeft | (rb & 15u) * kRight;
             if (wave == 0 && first) o |= kTop | (first & 1ull ? kTopLeft : 0u) | (first >> 63 ? kTopRight : 0u);
             if (wave == kWaves - 1 && last)
@@ -544,6 +585,8 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     const size_t edge_off = (sizeof(unsigned) * (counters + 4 * (size_t)ntiles) + 255) / 256 * 256;
     rc = pargo::ensure_scratch(ctx, edge_off + sizeof(double) * 2 * pargo::kTH * (size_t)ntiles);
     if (rc) return rc;
+    rc = pargo::ensure_report(ctx);
+    if (rc) return rc;
     unsigned *scr = static_cast<unsigned *>(ctx->scratch);
     p.range = scr;
     p.count = scr + 2;
@@ -565,8 +608,8 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     for (;;) {
         for (int k = 0; k < kBatch; k++)
             hipLaunchKernelGGL(pargo::fill_pass_kernel, dim3(pass_blocks), dim3(256), 0, ctx->stream, p, pass + k);
-        unsigned h[5];  // range, then the list counts
-        PARGO_HIP(ctx, hipMemcpyAsync(h, scr, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
+        const unsigned *h = static_cast<const unsigned *>(ctx->report);  // range, then the list counts
+        PARGO_HIP(ctx, hipMemcpyAsync(ctx->report, scr, 5 * sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
         PARGO_HIP(ctx, hipStreamSynchronize(ctx->stream));
         rc = pargo::check_launch(ctx, "pargo_pit_remove");
         if (rc) return rc;

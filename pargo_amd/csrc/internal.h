@@ -29,6 +29,7 @@ struct pargo_ctx {
     // Small reusable device scratch owned by the context (grows on demand).
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
+    void *report = nullptr;  // page-locked host words that progress counters are copied to (64 bytes)
     void *fix_mem = nullptr;  // focal fixup queue (counters + cell list)
     // device address of the static fixup queue of pargo_slope_d8_noalloc on
     // this context's device (resolved once by pargo_create)
@@ -70,6 +71,11 @@ const char *injected_note();
 
 // Grows the context scratch to at least `bytes`.
 int ensure_scratch(pargo_ctx *ctx, size_t bytes);
+
+// Allocates the context's page-locked report words: a device-to-host copy of
+// a few counters into pageable memory goes through the runtime's staging and
+// held the stream about 45 us per check of pitremove, into these CHECK_US.
+int ensure_report(pargo_ctx *ctx);
 
 // Float interval [lo, hi] of the float32 values v for which the reference's
 // double test fabs((double)v - nodata) < eps (<= eps when inclusive) holds
