@@ -264,9 +264,10 @@ int pargo_sca_d8(pargo_ctx *ctx, const pargo_grid *grid, const uint8_t *flow, co
  * [min(dem, 10000), 10000]) is refused with PARGO_E_UNSUPPORTED, as is a
  * DEM holding NaN (the reference never settles next to NoData there).
  * Synchronous.  *passes (host, may be NULL) receives the number of device
- * passes.  Working memory: the context's scratch grows to 524 bytes per
- * 64 x 32 tile (worklists, stamps and a copy of each tile's edge columns),
- * kept until pargo_destroy. */
+ * passes.  Working memory: the context's scratch grows to 528 bytes per
+ * 64 x 32 tile (worklists, flags and a copy of each tile's edge columns)
+ * plus 25 KB, kept until pargo_destroy.  A refused DEM leaves filled_out
+ * undefined. */
 int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *grid, const float *dem, double *filled_out, int *passes);
 
 /* ---- IDW ------------------------------------------------------------ */

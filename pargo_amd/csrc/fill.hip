@@ -52,6 +52,18 @@
 // flag.  Pass 0's list holds the tiles with a cell in or around them that
 // the init kernel opened: with every valid W at 10000, nothing else can
 // change.
+//
+// Measured at 16384^2 on the synthetic DEM: 6.8 ms (19.3 ms with nine-cell
+// windows swept over whole tiles, two launches per pass): 0.6 ms init, 6 ms
+// in 32 passes, 525,000 visits of which half change something and 3.3 waves
+// on average load.  A visit that changes nothing reads 26 KB at 5.1 TB/s
+// (0.67 ms for all 131,072 tiles), which is 2.2 ms of the passes; the rest is
+// the evaluations (3.4 rounds a visit), the rows written (4.8 GB) and the
+// 15-20 us a pass of few tiles takes.  Occupancy (4 to 6 waves per SIMD),
+// a tiled layout of W and 16- or 64-row tiles changed nothing or lost
+// (16 rows 11.2 ms, 64 rows 8.9 ms against 7.2); putting a visit off when a
+// neighbour has changed during the pass saved no visits and took 56 passes
+// instead of 32.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -76,16 +88,24 @@ constexpr unsigned kTop = 1u << 8, kBottom = 1u << 9;
 constexpr unsigned kTopLeft = 1u << 10, kTopRight = 1u << 11, kBottomLeft = 1u << 12, kBottomRight = 1u << 13;
 constexpr unsigned kAll = 1u << 15;  // never visited: every row is to be evaluated
 
+// A worklist is kSub lists, a tile's by its number modulo kSub, each with a
+// counter in a cache line of its own: returning atomics on one address take
+// about 11 ns each here whatever else runs, and with one counter the passes
+// at 16384^2 took as long as their 300,000 appends did.
+constexpr int kSub = 64, kSubStride = 32;  // stride in 4-byte words
+constexpr int kSetWords = kSub * kSubStride;
+
 struct FillParams {
     const float *__restrict__ dem;
     double *__restrict__ w;
     unsigned *__restrict__ flags;    // [2][tiles]: what the tile's next visit starts from (even, odd passes)
-    unsigned *__restrict__ count;    // [3]: entries of the worklists, pass p's in count[p % 3]
-    int *__restrict__ list;          // [2][tiles]: tiles of the pass (even, odd)
+    unsigned *__restrict__ count;    // [3][kSub]: entries of the worklists (kSubStride apart), pass p's in set p % 3
+    unsigned *__restrict__ total;    // entries of the last pass that ran
+    int *__restrict__ list;          // [2][kSub][sub_cap]: tiles of the pass (even, odd)
     double *__restrict__ edge;       // [tiles][2][kTH]: W of each tile's first and last column, NoData as +infinity
     unsigned *__restrict__ range;    // [0] smallest valid elevation (ordered bits), [1] NaN cells
     long long pitch;
-    int rows, cols, tiles_x, tiles_y;
+    int rows, cols, tiles_x, tiles_y, sub_cap;
     float nd_lo, nd_hi;  // float32 values with fabs((double)v - nodata) <= 1e-6
     int opens;           // a NoData neighbour opens a cell (not with NoData +infinity, which tests unequal to itself)
     double nodata;
@@ -134,26 +154,17 @@ __device__ __forceinline__ long long edge_index(const FillParams &p, int ty, int
     return (((long long)ty * p.tiles_x + tx) * 2 + right) * kTH + row_in_tile;
 }
 
-// Sets flags of tile t for pass `pass`; true for the first one, which puts
-// the tile on that pass's list (the caller appends it).
-__device__ __forceinline__ bool flag_tile(const FillParams &p, int t, unsigned f, int pass)
+// Sets flags of tile t for pass `pass`; 0 for the first ones, with which the
+// caller appends the tile to that pass's list.
+__device__ __forceinline__ unsigned flag_tile(const FillParams &p, int t, unsigned f, int pass)
 {
-    return atomicOr(&p.flags[(long long)(pass & 1) * p.tiles_x * p.tiles_y + t], f) == 0;
+    return atomicOr(&p.flags[(long long)(pass & 1) * p.tiles_x * p.tiles_y + t], f);
 }
-
-// Appends the tiles of the lanes with `first` set to pass `pass`'s list: one
-// atomic per wave (same-address atomics serialise).  Lane 0 must be active.
-__device__ __forceinline__ void append_tiles(const FillParams &p, int t, bool first, int pass)
+__device__ __forceinline__ void append_tile(const FillParams &p, int t, int pass)
 {
-    const unsigned long long m = __builtin_amdgcn_ballot_w64(first);
-    if (m == 0) return;
-    unsigned base = 0;
-    if ((threadIdx.x & 63) == 0) base = atomicAdd(&p.count[pass % 3], (unsigned)__builtin_popcountll(m));
-    base = (unsigned)__builtin_amdgcn_readfirstlane((int)base);
-    if (first) {
-        const unsigned k = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-        p.list[(long long)(pass & 1) * p.tiles_x * p.tiles_y + base + k] = t;
-    }
+    const int sub = t % kSub;
+    const unsigned k = atomicAdd(&p.count[(pass % 3) * kSetWords + sub * kSubStride], 1u);
+    p.list[((long long)(pass & 1) * kSub + sub) * p.sub_cap + k] = t;
 }
 
 // W before the first sweep (pitRemoveOperator.cpp:39-45 plus copyLayerInfo,
@@ -174,8 +185,8 @@ struct InitSeen {
 };
 
 // INNER: every cell of the tile and around it is an interior cell, so no row
-// or column is tested (all tiles but the border's; 0.92 -> INIT_MS ms at
-// 16384^2, the tests being scalar work for every row).
+// or column is tested (all tiles but the border's; the tests are scalar work
+// for every row).  0.62 ms at 16384^2 (3.2 GB moved, 5.2 TB/s).
 template <bool INNER>
 __device__ __forceinline__ void fill_init_tile(const FillParams &p, int ty, int tx, int lane, double *edge, InitSeen &o)
 {
@@ -264,8 +275,7 @@ __global__ __launch_bounds__(256) void fill_init_kernel(FillParams p)
         const bool need = lane < 9 && (dx < 0 ? (m & 1ull) != 0 : (dx > 0 ? (m >> 63) != 0 : m != 0)) && nty >= 0 &&
                           nty < p.tiles_y && ntx >= 0 && ntx < p.tiles_x;
         const int t = nty * p.tiles_x + ntx;
-        const bool first = need && flag_tile(p, t, kAll, 0);
-        append_tiles(p, t, first, 0);
+        if (need && flag_tile(p, t, kAll, 0) == 0) append_tile(p, t, 0);
     }
     unsigned least = o.least, nans = o.nans;
     for (int off = 32; off > 0; off >>= 1) {
@@ -286,7 +296,7 @@ __global__ void fill_reset_kernel(FillParams p, int n)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < n) p.flags[i] = 0;
-    if (i < 3) p.count[i] = 0;
+    if (i < 3 * kSetWords) p.count[i] = 0;
     if (i == 0) {
         p.range[0] = 0xffffffffu;
         p.range[1] = 0;
@@ -296,34 +306,36 @@ __global__ void fill_reset_kernel(FillParams p, int n)
 struct FillShared {
     double h[2][kWaves][2][kTW];  // per round parity and wave: h of its first and last row
     unsigned note[2][kWaves];     // per round parity and wave: kSentTop, kSentBottom, kGoing
-    unsigned start;               // the flags of this visit (0: none)
-    unsigned out;                 // which edges and corners changed
+    unsigned start[2];            // by parity of the visit: its flags (0: none)
+    unsigned out[2];              // by parity of the visit: which edges and corners changed
 };
 constexpr unsigned kSentTop = 1u, kSentBottom = 2u, kGoing = 4u;
 
+// The flags a visit starts from, requested a visit ahead by thread 0 so that
+// no wave waits for them (list entry, flags and barrier in turn cost a visit
+// about 2 us of its 15).
+__device__ __forceinline__ unsigned *visit_flags(const FillParams &p, int tile, int pass)
+{
+    return &p.flags[(long long)(pass & 1) * p.tiles_x * p.tiles_y + tile];
+}
+
+// Tiles flagged at the end of a visit and not on a list yet: wave 0 appends
+// them during the next visit, while that visit's loads are on their way.
+struct Flagged {
+    int tile = 0;
+    unsigned old = 1;  // the flags found (0: the lane's tile goes on the list)
+};
+
 // One visit of one tile (see the top of the file).
-__device__ __forceinline__ void fill_tile(const FillParams &p, int tile, int pass, FillShared &S)
+__device__ __forceinline__ void fill_tile(const FillParams &p, int tile, unsigned start, int parity, int pass,
+                                          FillShared &S, Flagged &flagged)
 {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const long long ntiles = (long long)p.tiles_x * p.tiles_y;
-    if (threadIdx.x == 0) {
-        unsigned *mine = &p.flags[(long long)(pass & 1) * ntiles + tile];
-        unsigned *next = &p.flags[(long long)((pass + 1) & 1) * ntiles + tile];
-        unsigned f = *mine;
-        *mine = 0;
-        // a neighbour has changed during this pass already: the visit waits
-        // for the next pass, where one visit serves both changes
-        if (__atomic_load_n(next, __ATOMIC_RELAXED) != 0) {
-            atomicOr(next, f);
-            f = 0;
-        }
-        S.start = f;
-        S.out = 0;
-    }
-    __syncthreads();
-    const unsigned start = (unsigned)__builtin_amdgcn_readfirstlane((int)S.start);
-    if (start == 0) return;
+    auto flush = [&]() {
+        if (flagged.old == 0) append_tile(p, flagged.tile, pass + 1);
+        flagged.old = 1;
+    };
     const int ty = tile / p.tiles_x, tx = tile - ty * p.tiles_x;
     const int r0 = ty * kTH + wave * kRW, c = tx * kTW + lane;  // the wave's first row, the lane's column
     constexpr unsigned kRows = (1u << kRW) - 1u;
@@ -389,6 +401,7 @@ __device__ __forceinline__ void fill_tile(const FillParams &p, int tile, int pas
             }
             get(r0 + kRW, wd, ed);
         }
+        if (wave == 0) flush();
         // NoData reads as +infinity: never a minimum, never lowered
         auto open = [&](double v) -> double { return v == p.nodata ? inf : v; };
 #pragma unroll
@@ -451,6 +464,7 @@ __device__ __forceinline__ void fill_tile(const FillParams &p, int tile, int pas
         return notes == 0;
     };
     bool settled = false;
+    if (wave == 0 && dirty == 0) flush();
     while (dirty == 0 && !settled) settled = exchange(0);  // nothing to load yet
     if (!settled) {
         load();
@@ -498,12 +512,17 @@ __device__ __forceinline__ void fill_tile(const FillParams &p, int tile, int pas
             if (wave == 0 && first) o |= kTop | (first & 1ull ? kTopLeft : 0u) | (first >> 63 ? kTopRight : 0u);
             if (wave == kWaves - 1 && last)
                 o |= kBottom | (last & 1ull ? kBottomLeft : 0u) | (last >> 63 ? kBottomRight : 0u);
-            if (o) atomicOr(&S.out, o);
+            if (o) atomicOr(&S.out[parity], o);
         }
     }
-    __syncthreads();
-    const unsigned out = S.out;
-    if (wave == 0 && out != 0) {
+}
+
+// After the barrier that ends a visit: flags the tiles around it (wave 0).
+__device__ __forceinline__ void flag_around(const FillParams &p, int tile, unsigned out, int pass, Flagged &flagged)
+{
+    const int lane = threadIdx.x & 63;
+    const int ty = tile / p.tiles_x, tx = tile - ty * p.tiles_x;
+    {
         // lanes 0-8: the tiles around, each with the side of it that changed
         const int dy = lane / 3 - 1, dx = lane % 3 - 1;
         unsigned f = 0;
@@ -518,27 +537,78 @@ __device__ __forceinline__ void fill_tile(const FillParams &p, int tile, int pas
         const int nty = ty + dy, ntx = tx + dx;
         const bool need = f != 0 && nty >= 0 && nty < p.tiles_y && ntx >= 0 && ntx < p.tiles_x;
         const int t = nty * p.tiles_x + ntx;
-        const bool fresh = need && flag_tile(p, t, f, pass + 1);
-        append_tiles(p, t, fresh, pass + 1);
+        if (need) {
+            flagged.tile = t;
+            flagged.old = flag_tile(p, t, f, pass + 1);
+        }
     }
 }
 
 __global__ __launch_bounds__(256, 5) void fill_pass_kernel(FillParams p, int pass)
 {
     __shared__ FillShared S;
-    const unsigned n = p.count[pass % 3];
-    // the list count that pass + 1 fills (pass - 1 read it)
-    if (blockIdx.x == 0 && threadIdx.x == 0) p.count[(pass + 2) % 3] = 0;
-    const int *list = p.list + (long long)(pass & 1) * p.tiles_x * p.tiles_y;
-    // A fixed stride over the list keeps the tiles in flight apart (tiles
-    // next to each other in the list are neighbours); taking them one at a
-    // time from a cursor ran neighbours together, which then revisited each
-    // other more (27 against 24 ms).  The grid is what fits on the GPU at
-    // once, so no workgroup starts late with a full share.
-    for (unsigned e = blockIdx.x; e < n; e += gridDim.x) {
-        fill_tile(p, __builtin_amdgcn_readfirstlane(list[e]), pass, S);
-        __syncthreads();  // the next tile reuses the LDS
+    const int lane = threadIdx.x & 63;
+    // the sublists' lengths, one per lane, and where each ends in the whole list
+    const unsigned len = p.count[(pass % 3) * kSetWords + lane * kSubStride];
+    unsigned end = len;
+#pragma unroll
+    for (int off = 1; off < kSub; off <<= 1) {
+        const unsigned o = (unsigned)__shfl_up((int)end, off);
+        if (lane >= off) end += o;
     }
+    const unsigned n = (unsigned)__builtin_amdgcn_readlane((int)end, kSub - 1);
+    if (blockIdx.x == 0 && threadIdx.x < kSub) {
+        // the counters that pass + 1 fills (pass - 1 read them)
+        p.count[((pass + 2) % 3) * kSetWords + lane * kSubStride] = 0;
+        if (lane == 0) *p.total = n;
+    }
+    // A fixed stride over the list, whose neighbours are tiles kSub apart.
+    // The grid is what fits on the GPU at once, so no workgroup starts late
+    // with a full share.
+    const unsigned stride = gridDim.x;
+    unsigned e = blockIdx.x;
+    if (e >= n) return;  // the whole workgroup
+    const int *list = p.list + (long long)(pass & 1) * kSub * p.sub_cap;
+    auto entry = [&](unsigned i) -> int {
+        const int sub = __builtin_popcountll(__builtin_amdgcn_ballot_w64(end <= i));  // sublists that end before i
+        const unsigned at = i - (unsigned)__builtin_amdgcn_readlane((int)(end - len), sub);
+        return list[(long long)sub * p.sub_cap + at];
+    };
+    int tile = __builtin_amdgcn_readfirstlane(entry(e));
+    int ahead = e + stride < n ? entry(e + stride) : 0;
+    if (threadIdx.x == 0) {
+        unsigned *f = visit_flags(p, tile, pass);
+        S.start[0] = *f;
+        S.out[0] = 0;
+        *f = 0;
+    }
+    __syncthreads();
+    Flagged flagged;
+    for (int parity = 0; e < n; e += stride, parity ^= 1) {
+        const unsigned start = (unsigned)__builtin_amdgcn_readfirstlane((int)S.start[parity]);
+        // the next visit's flags and the list entry of the one after are
+        // requested now, so that no visit waits for them
+        const bool more = e + stride < n;
+        const int next_tile = __builtin_amdgcn_readfirstlane(ahead);
+        unsigned next_start = 0;
+        if (more && threadIdx.x == 0) next_start = *visit_flags(p, next_tile, pass);
+        if (e + 2 * stride < n) ahead = entry(e + 2 * stride);
+        fill_tile(p, tile, start, parity, pass, S, flagged);
+        if (more && threadIdx.x == 0) {
+            S.start[parity ^ 1] = next_start;
+            S.out[parity ^ 1] = 0;
+            *visit_flags(p, next_tile, pass) = 0;
+        }
+        // the next visit reuses the LDS; what a visit leaves there is read
+        // right after the barrier and written again only after the next one
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            const unsigned out = (unsigned)__builtin_amdgcn_readfirstlane((int)S.out[parity]);
+            if (out != 0) flag_around(p, tile, out, pass, flagged);
+        }
+        tile = next_tile;
+    }
+    if (threadIdx.x < 64 && flagged.old == 0) append_tile(p, flagged.tile, pass + 1);
 }
 
 }  // namespace
@@ -579,22 +649,27 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     const int ntiles = p.tiles_x * p.tiles_y;
     constexpr int kBatch = 8;      // passes between checks
     constexpr int kMaxPasses = 1 << 20;
-    // scratch: the range check's two words and the three list counts, then
-    // the flags, the two worklists and the tiles' edge columns
-    const size_t counters = 8;
-    const size_t edge_off = (sizeof(unsigned) * (counters + 4 * (size_t)ntiles) + 255) / 256 * 256;
+    // scratch: the range check's two words and the last list's length, the
+    // list counters, then the flags, the two worklists and the tiles' edge
+    // columns
+    const size_t counters = 64 + 3 * (size_t)pargo::kSetWords;
+    p.sub_cap = (ntiles + pargo::kSub - 1) / pargo::kSub;
+    const size_t words = counters + 2 * (size_t)ntiles + 2 * (size_t)pargo::kSub * p.sub_cap;
+    const size_t edge_off = (sizeof(unsigned) * words + 255) / 256 * 256;
     rc = pargo::ensure_scratch(ctx, edge_off + sizeof(double) * 2 * pargo::kTH * (size_t)ntiles);
     if (rc) return rc;
     rc = pargo::ensure_report(ctx);
     if (rc) return rc;
     unsigned *scr = static_cast<unsigned *>(ctx->scratch);
     p.range = scr;
-    p.count = scr + 2;
+    p.total = scr + 2;
+    p.count = scr + 64;
     p.flags = scr + counters;
     p.list = reinterpret_cast<int *>(p.flags + 2 * (size_t)ntiles);
     p.edge = reinterpret_cast<double *>(static_cast<char *>(ctx->scratch) + edge_off);
 
-    hipLaunchKernelGGL(pargo::fill_reset_kernel, dim3((2 * ntiles + 255) / 256), dim3(256), 0, ctx->stream, p, 2 * ntiles);
+    hipLaunchKernelGGL(pargo::fill_reset_kernel, dim3((std::max(2 * ntiles, 3 * pargo::kSetWords) + 255) / 256), dim3(256), 0,
+                       ctx->stream, p, 2 * ntiles);
     hipLaunchKernelGGL(pargo::fill_init_kernel, dim3((p.tiles_x + 3) / 4, p.tiles_y), dim3(256), 0, ctx->stream, p);
     // a fixed grid walks each pass's worklist: as many workgroups as are
     // resident at once
@@ -608,8 +683,8 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     for (;;) {
         for (int k = 0; k < kBatch; k++)
             hipLaunchKernelGGL(pargo::fill_pass_kernel, dim3(pass_blocks), dim3(256), 0, ctx->stream, p, pass + k);
-        const unsigned *h = static_cast<const unsigned *>(ctx->report);  // range, then the list counts
-        PARGO_HIP(ctx, hipMemcpyAsync(ctx->report, scr, 5 * sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
+        const unsigned *h = static_cast<const unsigned *>(ctx->report);  // range, then the last pass's list length
+        PARGO_HIP(ctx, hipMemcpyAsync(ctx->report, scr, 3 * sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
         PARGO_HIP(ctx, hipStreamSynchronize(ctx->stream));
         rc = pargo::check_launch(ctx, "pargo_pit_remove");
         if (rc) return rc;
@@ -632,7 +707,7 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
                             g->nodata, lo);
         }
         pass += kBatch;
-        if (h[2 + pass % 3] == 0) break;  // nothing scheduled
+        if (h[2] == 0) break;  // the batch's last pass had nothing to do
         if (pass >= kMaxPasses)
             return fail(ctx, PARGO_E_NONTERM, "depression filling did not settle within %d passes", kMaxPasses);
     }

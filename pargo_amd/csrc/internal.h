@@ -74,7 +74,7 @@ int ensure_scratch(pargo_ctx *ctx, size_t bytes);
 
 // Allocates the context's page-locked report words: a device-to-host copy of
 // a few counters into pageable memory goes through the runtime's staging and
-// held the stream about 45 us per check of pitremove, into these CHECK_US.
+// held the stream about 50 us per check of pitremove, into these 25-30.
 int ensure_report(pargo_ctx *ctx);
 
 // Float interval [lo, hi] of the float32 values v for which the reference's
