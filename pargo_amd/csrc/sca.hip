@@ -29,7 +29,7 @@
 //
 // Device formulation: the dependencies that matter (non-source inflows the
 // cell waits for) form a forest, each cell feeding at most its one target.
-// A 16-bit static word per cell holds what a walk needs:
+// A 16-bit static word per cell holds what following it needs:
 //   bits  0-3   npend: inflows the cell waits for
 //   bits  4-7   nsrc: inflows from sources (each adds 1)
 //   bit   8     an inflow can never be available (border, or behind in
@@ -37,27 +37,39 @@
 //   bit   9     feeds: the cell is one of its target's pending inflows
 //   bits 10-13  the cell's code (window index of its target)
 //   bit  14     the cell has an area (interior, not NoData)
-// The static words sit in the context scratch in 8 x 8 blocks of 128 bytes,
-// one cache line each, so that the hops of a walk, which move to a
-// neighbour, mostly stay in a line that is already cached.
-// The output holds each cell's area as a double from the start when the
-// cell waits for nothing (1 + nsrc; NoData; 1 for a cell without a class).
-// A cell that waits (npend >= 1) holds an arrival accumulator instead until
-// it completes:
-//   bits  0-39  sum of the areas of done arrivals
-//   bits 40-43  arrivals that were not done
-//   bits 44-47  arrivals
-//   bit  63     the cell has not completed (a finished area is >= 1)
-// Every cell with npend == 0 that feeds starts a walk.  A hop reads the
-// target's static word: a target that waits for this walk alone completes
-// at once; a confluence (npend >= 2) takes an atomicAdd on its accumulator
-// and completes on the last arrival (the returned word holds the others).
-// The completing walk writes the target's area and carries on from there.
-// Each cell completes once, so the work is linear in the cells; the walk is
-// as long as the longest chain of completions.  Waiting cells and
-// completions are counted; cells that never complete (a cycle of codes,
-// which the converging mode admits for arbitrary codes) leave the counts
-// apart, and only then a last pass turns their accumulators into areas.
+// The forest is solved tile by tile (64 x 32 cells) in LDS, where a hop to
+// the next cell is one LDS atomic, and only what crosses tile edges goes
+// through memory.  Inside a tile every cell has an accumulator (the sum of
+// its done inflows' areas, the inflows still awaited, how many were not
+// done); a walk starts at each cell that waits for nothing and feeds, adds
+// its cell to the target's accumulator and goes on from there if nothing
+// else is awaited.
+//   1. sca_local_kernel forms the static words and runs the tile's walks
+//      with every inflow from outside taken as an arrival of area 0 that is
+//      done.  A cell through which the tile is left (an exit, a perimeter
+//      cell) then holds what its tile contributes, the number of inflows
+//      from outside upstream of it, and whether anything inside the tile
+//      keeps it from being done.  Its area when they have arrived is that
+//      sum plus theirs, and it is done when they all are, so an exit is one
+//      node of a graph whose links are "the exit that a walk entering here
+//      leaves through", found by following each entry to the tile's edge.
+//   2. sca_link_kernel resolves each exit's successor, the exit of the tile
+//      it enters.
+//   3. sca_cross_kernel walks that graph: a hop is one 64-bit atomic on the
+//      successor's word (sum, awaited, not done), with the successor's own
+//      link read beside it.
+//   4. sca_final_kernel runs the tile's walks once more, now with the areas
+//      that arrive from outside, and writes the areas.
+// Cells that never complete (a cycle of codes, which the converging mode
+// admits for arbitrary codes) keep the sum of the done inflows they
+// received, which is their area.
+//
+// Measured on the headline DEM's codes: 16384^2 in the reference mode 2.85 ms
+// (local 1.70, link 0.07, cross 0.12, final 1.00), 5003 x 7001 in the
+// converging mode 0.46 ms, and 0.11 ms for the codes of a filled 1501 x 2003
+// DEM, whose paths are long.  One walk over the whole raster with a global
+// atomic or a static word read per hop (33 bytes of HBM traffic, up to 1336
+// hops in a row) took 4.24, 1.21 and 1.15 ms.
 #include <cmath>
 
 #include "internal.h"
@@ -69,12 +81,39 @@ namespace {
 
 constexpr unsigned kNone = 15;
 constexpr int kTileC = 64, kTileR = 32;  // cells per workgroup: 64 x 32
-constexpr uint64_t kAccMask = (1ull << 40) - 1;
-constexpr uint64_t kOpen = 1ull << 63;   // accumulator tag: not completed
-// The waiting cells are counted by one atomic per init workgroup, spread
-// over 64 counters 256 bytes apart: one counter took 131,072 device-scope
-// atomics per pass at 16384^2, serialised at one address (about 0.3 ms).
-constexpr int kWaitSlots = 64, kWaitStride = 32;  // stride in 8-byte words
+constexpr int kTileN = kTileC * kTileR;
+
+// Perimeter slots of a tile: top row 0-63, bottom row 64-127, then the left
+// and the right column without the corners.
+constexpr int kSlots = 2 * kTileC + 2 * (kTileR - 2), kSlotStride = 192;
+static_assert(kSlots <= kSlotStride && kSlots <= 256, "one thread per slot");
+__device__ __forceinline__ int slot_of(int r, int c)
+{
+    return r == 0 ? c : r == kTileR - 1 ? kTileC + c : (c == 0 ? 2 * kTileC : 2 * kTileC + kTileR - 2) + r - 1;
+}
+__device__ __forceinline__ int cell_of_slot(int s)
+{
+    if (s < kTileC) return s;
+    if (s < 2 * kTileC) return (kTileR - 1) * kTileC + s - kTileC;
+    s -= 2 * kTileC;
+    return s < kTileR - 2 ? (s + 1) * kTileC : (s - (kTileR - 2) + 1) * kTileC + kTileC - 1;
+}
+
+// A tile's accumulators in sca_local_kernel, 32 bits: sum of areas (at most
+// the tile's cells and the 196 sources that can drain into it), inflows from
+// outside upstream (at most 196), not-done arrivals, arrivals awaited.
+constexpr int kLocExt = 12, kLocBad = 20, kLocPend = 24;
+constexpr unsigned kLocSum = (1u << kLocExt) - 1;
+static_assert(kTileN + 2 * (kTileC + kTileR) + 4 <= (int)kLocSum, "areas inside a tile fit their field");
+// In sca_final_kernel, 64 bits: sum of areas, not-done arrivals, awaited.
+constexpr int kFinBad = 40, kFinPend = 44;
+constexpr unsigned long long kFinSum = (1ull << kFinBad) - 1, kFinArea = 1ull << 63;  // kFinArea: the cell has one
+// An exit's word: sum of areas, arrivals awaited (255: not an exit, or never
+// complete), not-done arrivals, and a flag for the exits that await nothing
+// from the start.
+constexpr int kExitPend = 40, kExitBad = 48;
+constexpr unsigned long long kExitStart = 1ull << 63, kExitNever = 255ull << kExitPend;
+constexpr unsigned kNoExit = 0xffffffffu;
 
 __device__ __forceinline__ unsigned flow_of(unsigned b) { return (b <= 8u && b != 4u) ? b : kNone; }
 __device__ __forceinline__ unsigned excl_of(unsigned b)
@@ -88,14 +127,16 @@ __device__ __forceinline__ bool is_valid(unsigned b) { return b != PARGO_FLOW_NO
 struct ScaParams {
     const uint8_t *__restrict__ flow;
     const uint32_t *__restrict__ mask;  // may be null
-    unsigned long long *__restrict__ w; // the output buffer: areas (doubles) and accumulators
-    uint16_t *__restrict__ st;          // static words, 8 x 8 blocks
-    unsigned long long *__restrict__ counters;  // [0] walk cursor, [1] waiting cells, [2] completions
+    double *__restrict__ area;
+    uint16_t *__restrict__ st;          // static words, tile by tile
+    unsigned long long *__restrict__ exits;  // [tiles][kSlotStride] exit words
+    unsigned *__restrict__ next;        // [tiles][kSlotStride]: the perimeter cell an exit enters, then its successor
+    uint8_t *__restrict__ link;         // [tiles][kSlotStride]: slot of the exit reached from a perimeter cell (255: none)
+    uint8_t *__restrict__ ext;          // [tiles][kSlotStride]: pending inflows of a perimeter cell from outside
     unsigned *__restrict__ last_done;   // done flags of the 3 x 3 cells ending at (rows-1, cols-1)
-    unsigned long long *__restrict__ wait_slots;  // waiting cells, kWaitSlots partial counts kWaitStride apart
     long long pitch;
     int rows, cols, mask_words;
-    int bx, by;  // 8 x 8 blocks per block row, block rows
+    int tiles_x, ntiles;
     int converge;
     double nodata;
 };
@@ -107,13 +148,6 @@ __device__ __forceinline__ bool feeds_of(unsigned s) { return (s >> 9) & 1u; }
 __device__ __forceinline__ int code_of(unsigned s) { return (int)(s >> 10) & 15; }
 __device__ __forceinline__ bool area_of(unsigned s) { return (s >> 14) & 1u; }
 
-__device__ __forceinline__ long long st_index(const ScaParams &p, int r, int c)
-{
-    return ((long long)(r >> 3) * p.bx + (c >> 3)) * 64 + ((r & 7) << 3) + (c & 7);
-}
-
-__device__ __forceinline__ unsigned long long bits_of(double v) { return (unsigned long long)__double_as_longlong(v); }
-
 __device__ __forceinline__ unsigned load_class(const ScaParams &p, int r, int c)
 {
     if (r < 0 || r >= p.rows || c < 0 || c >= p.cols) return PARGO_FLOW_NODATA;
@@ -121,37 +155,21 @@ __device__ __forceinline__ unsigned load_class(const ScaParams &p, int r, int c)
     return p.flow[(long long)r * p.pitch + c];
 }
 
-__device__ __forceinline__ unsigned wave_sum(unsigned v)
-{
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-
-// Counters and last-cell flags to zero, before the init kernel counts.
-__global__ void sca_reset_kernel(ScaParams p)
-{
-    const int i = threadIdx.x;
-    if (i < 3) p.counters[i] = 0;
-    if (i < 9) p.last_done[i] = 0;
-    if (i < kWaitSlots) p.wait_slots[i * kWaitStride] = 0;
-}
-
-__device__ __forceinline__ void add_waiting(const ScaParams &p, unsigned n)
-{
-    if (n) atomicAdd(&p.wait_slots[(blockIdx.x & (kWaitSlots - 1)) * kWaitStride], (unsigned long long)n);
-}
-
-// Static words and starting values of a 64 x 32 tile.  Classes of the tile
-// plus a 2-cell halo go to LDS, then the inflow mask of the tile plus a
-// 1-cell halo (bit j set when the neighbour at window position j < 4 ? j :
-// j + 1 drains into the cell and is not excluded; a cell needs to know which
-// of its inflows are sources, and whether its target counts it).  Tiles are
-// dealt to the 8 XCDs in contiguous runs (workgroup g runs on XCD g % 8), so
-// neighbouring tiles share their halo lines in one L2.
+// Static words of a 64 x 32 tile.  Classes of the tile plus a 2-cell halo go
+// to LDS, then the inflow mask of the tile plus a 1-cell halo (bit j set when
+// the neighbour at window position j < 4 ? j : j + 1 drains into the cell and
+// is not excluded; a cell needs to know which of its inflows are sources, and
+// whether its target counts it).  Tiles are dealt to the 8 XCDs in contiguous
+// runs (workgroup g runs on XCD g % 8), so neighbouring tiles share their
+// halo lines in one L2.
 __device__ __forceinline__ int win_of_bit(int j) { return j < 4 ? j : j + 1; }
 __device__ __forceinline__ int bit_of_win(int k) { return k < 4 ? k : k - 1; }
 
-typedef unsigned long long u64x2_a8 __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ int xcd_tile(const ScaParams &p)
+{
+    const int per = (p.ntiles + 7) / 8, g = blockIdx.x;  // tiles per XCD
+    return (g & 7) * per + (g >> 3);
+}
 
 // A tile at least 2 cells from every border whose class rows can be read
 // as words, four cells per word (sca_swar.h): the halo columns c0 - 8 ..
@@ -162,12 +180,12 @@ __device__ __forceinline__ bool sca_swar_tile(const ScaParams &p, int r0, int c0
     return r0 >= 2 && r0 + kSwarTileR + 2 <= p.rows && c0 >= 11 && c0 + 76 <= p.cols;
 }
 
-// The init pass of such a tile, four cells per lane: the same static words
-// and starting values as the per-cell code of sca_init_kernel, with half its
-// VALU instructions and a sixth of its LDS accesses.
-__device__ __forceinline__ void sca_init_words(const ScaParams &p, SwarTile &T, unsigned *waiting, int r0, int c0)
+// The static words of such a tile, four cells per lane: the same words as the
+// per-cell code of general_words, with half its VALU instructions and a sixth
+// of its LDS accesses.
+__device__ __forceinline__ void swar_words(const ScaParams &p, SwarTile &T, uint16_t *stw, int r0, int c0)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x;
     {
         constexpr int N = kSwarClsRows * kSwarClsWords, PER = (N + 255) / 256;
         uint32_t lo[PER], hi[PER], mw[PER];
@@ -206,58 +224,28 @@ __device__ __forceinline__ void sca_init_words(const ScaParams &p, SwarTile &T, 
         T.inm[lr][q] = swar_inflow(T, lr, q);
     }
     __syncthreads();
-    unsigned nwait = 0;
-    // 16 lanes per 8 x 8 block of static words (128 contiguous bytes)
 #pragma unroll
     for (int k = 0; k < 2; k++) {
-        const int v = tid + 256 * k, blk = v >> 4, within = v & 15;
-        const int tr = (blk >> 3) * 8 + (within >> 1), g = (blk & 7) * 2 + (within & 1);
+        const int v = tid + 256 * k, tr = v >> 4, g = v & 15;
         const SwarCells o = swar_cells(T, tr, g, p.converge != 0);
-        const int r = r0 + tr, c = c0 + 4 * g;
-        *reinterpret_cast<uint2 *>(p.st + st_index(p, r, c)) = make_uint2(o.s01, o.s23);
-        unsigned long long val[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const unsigned npend = (o.npend >> (8 * j)) & 0xFFu, nsrc = (o.nsrc >> (8 * j)) & 0xFFu;
-            val[j] = ((o.nodata >> (8 * j + 7)) & 1u)  ? bits_of(p.nodata)
-                     : ((o.inert >> (8 * j + 7)) & 1u) ? bits_of(1.0)
-                     : npend                           ? kOpen
-                                                       : bits_of((double)(1u + nsrc));
-        }
-        // streamed past the caches: the walk reads these words later
-        u64x2_a8 *dst = reinterpret_cast<u64x2_a8 *>(p.w + (long long)r * p.pitch + c);
-        const u64x2_a8 v01 = {val[0], val[1]}, v23 = {val[2], val[3]};
-        __builtin_nontemporal_store(v01, dst);
-        __builtin_nontemporal_store(v23, dst + 1);
-        nwait += (unsigned)__builtin_popcount(o.waiting);
+        *reinterpret_cast<uint2 *>(stw + tr * kTileC + 4 * g) = make_uint2(o.s01, o.s23);
     }
-    nwait = wave_sum(nwait);
-    if (lane == 0) waiting[wave] = nwait;
-    __syncthreads();
-    if (tid == 0) add_waiting(p, waiting[0] + waiting[1] + waiting[2] + waiting[3]);
 }
 
-__global__ __launch_bounds__(256) void sca_init_kernel(ScaParams p, int tiles_x, int ntiles)
+// Per-cell form, for tiles near the raster's edge.
+struct GeneralTile {
+    uint8_t cls[kTileR + 4][kTileC + 4];  // classes, halo 2
+    uint8_t tgt[kTileR + 4][kTileC + 4];  // flow_of(class): window index of the target, kNone if none
+    uint8_t inm[kTileR + 2][kTileC + 2];  // inflow masks, halo 1
+};
+
+__device__ __forceinline__ void general_words(const ScaParams &p, GeneralTile &T, uint16_t *stw, int r0, int c0)
 {
-    constexpr int CW = kTileC + 4, CH = kTileR + 4;  // classes, halo 2
-    constexpr int NW = kTileC + 2, NH = kTileR + 2;  // inflow masks, halo 1
-    __shared__ uint8_t cls[CH][CW];
-    __shared__ uint8_t tgt[CH][CW];  // flow_of(class): window index of the target, kNone if none
-    __shared__ uint8_t inm[NH][NW];
-    __shared__ uint16_t stw[kTileR][kTileC];
-    __shared__ unsigned waiting[4];
+    constexpr int CW = kTileC + 4, CH = kTileR + 4, NW = kTileC + 2, NH = kTileR + 2;
     const int tid = threadIdx.x;
-    const int g = blockIdx.x;
-    const int per = (ntiles + 7) / 8;  // tiles per XCD
-    const int tile = (g & 7) * per + (g >> 3);
-    if (tile >= ntiles) return;  // the whole workgroup
-    const int r0 = (tile / tiles_x) * kTileR, c0 = (tile % tiles_x) * kTileC;
-    static_assert(kSwarTileR == kTileR && kSwarTileC == kTileC, "one tile shape");
-    if (sca_swar_tile(p, r0, c0)) {
-        __shared__ SwarTile T;
-        sca_init_words(p, T, waiting, r0, c0);
-        return;
-    }
+    auto &cls = T.cls;
+    auto &tgt = T.tgt;
+    auto &inm = T.inm;
     {
         // every load of the thread is issued before the first store to LDS,
         // so that their latencies overlap
@@ -303,7 +291,6 @@ __global__ __launch_bounds__(256) void sca_init_kernel(ScaParams p, int tiles_x,
         inm[lr - 1][lc - 1] = (uint8_t)m;
     }
     __syncthreads();
-    unsigned nwait = 0;
     for (int i = tid; i < kTileR * kTileC; i += 256) {
         const int tr = i / kTileC, tc = i % kTileC;
         const int r = r0 + tr, c = c0 + tc;
@@ -311,10 +298,8 @@ __global__ __launch_bounds__(256) void sca_init_kernel(ScaParams p, int tiles_x,
         if (r < p.rows && c < p.cols) {
             const bool interior = r >= 1 && r <= p.rows - 2 && c >= 1 && c <= p.cols - 2;
             const unsigned b = cls[tr + 2][tc + 2];
-            unsigned long long value = bits_of(p.nodata);
             if (interior && b == PARGO_FLOW_INERT) {
                 s = 1u << 14;
-                value = bits_of(1.0);
             } else if (interior && b != PARGO_FLOW_NODATA) {
                 const unsigned mine = inm[tr + 1][tc + 1];
                 // per inflow bit j: the neighbour is interior (intn), is a
@@ -353,159 +338,323 @@ __global__ __launch_bounds__(256) void sca_init_kernel(ScaParams p, int tiles_x,
                     feeds = (t_interior && ((tm >> bit_of_win(8 - (int)f)) & 1u)) ? 1u : 0u;
                 }
                 s = npend | (nsrc << 4) | (poison << 8) | (feeds << 9) | ((f == kNone ? 0u : f) << 10) | (1u << 14);
-                value = npend ? kOpen : bits_of((double)(1u + nsrc));
-                nwait += npend ? 1u : 0u;
             }
-            p.w[(long long)r * p.pitch + c] = value;
         }
-        stw[tr][tc] = (uint16_t)s;
+        stw[i] = (uint16_t)s;
     }
-    nwait = wave_sum(nwait);
-    if ((tid & 63) == 0) waiting[tid >> 6] = nwait;
+}
+
+// One step of a walk: the cell that `idx` (tile row * kTileC + column) with
+// code k drains to, -1 outside the tile.
+__device__ __forceinline__ int step_to(int idx, int k)
+{
+    const int r = (idx >> 6) + (int)((unsigned)k / 3u) - 1, c = (idx & 63) + (int)((unsigned)k % 3u) - 1;
+    static_assert(kTileC == 64, "a tile row is 64 cells");
+    return (unsigned)r < (unsigned)kTileR && (unsigned)c < (unsigned)kTileC ? r * kTileC + c : -1;
+}
+
+// Where a walk goes from a cell: the next cell's index in the tile, or
+// kLeaves + the cell's slot when it drains out of the tile, or kEnds.
+constexpr unsigned kLeaves = 0x8000u, kEnds = 0xffffu;
+__device__ __forceinline__ unsigned next_of(int idx, unsigned s)
+{
+    if (!feeds_of(s)) return kEnds;
+    const int t = step_to(idx, code_of(s));
+    return t >= 0 ? (unsigned)t : kLeaves + (unsigned)slot_of(idx >> 6, idx & 63);
+}
+
+// The cells where walks start, gathered into one list so that they fill as
+// few waves as they can (30 to 60 of a tile's cells start a walk, and a hop
+// costs a wave the same for one lane as for 64).  A start that is not on the
+// perimeter has a source inside the tile draining to it.
+constexpr int kStarts = kTileN / 2 + 512;
+static_assert(kStarts >= kTileN / 2 + kSlots, "every start has a place");
+struct StartList {
+    uint16_t cell[kStarts];
+    unsigned n;
+};
+// Adds this thread's cells 8 tid + k with bit k of `m` set (all lanes call).
+__device__ __forceinline__ void add_starts(StartList &L, unsigned m)
+{
+    unsigned total = 0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) total += (unsigned)__builtin_popcountll(__builtin_amdgcn_ballot_w64((m >> k) & 1u));
+    unsigned at = 0;
+    if (total != 0 && (threadIdx.x & 63) == 0) at = atomicAdd(&L.n, total);
+    at = (unsigned)__builtin_amdgcn_readfirstlane((int)at);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const unsigned long long b = __builtin_amdgcn_ballot_w64((m >> k) & 1u);
+        if ((m >> k) & 1u)
+            L.cell[at + __builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b, 0u))] =
+                (uint16_t)(8 * threadIdx.x + k);
+        at += (unsigned)__builtin_popcountll(b);
+    }
+}
+__device__ __forceinline__ unsigned half_word(const uint4 &w, int k)
+{
+    const unsigned h = k < 2 ? w.x : k < 4 ? w.y : k < 6 ? w.z : w.w;
+    return (h >> (16 * (k & 1))) & 0xffffu;
+}
+// The thread's eight next_of values into `nxt`.
+__device__ __forceinline__ void store_next(uint16_t *nxt, const uint4 &words)
+{
+    unsigned n[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) n[k] = next_of(8 * (int)threadIdx.x + k, half_word(words, k));
+    *reinterpret_cast<uint4 *>(nxt + 8 * threadIdx.x) =
+        make_uint4(n[0] | n[1] << 16, n[2] | n[3] << 16, n[4] | n[5] << 16, n[6] | n[7] << 16);
+}
+
+union LocalShared {
+    SwarTile swar;
+    GeneralTile general;
+    unsigned acc[kTileN];  // once the static words are formed
+};
+
+__global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
+{
+    __shared__ LocalShared S;
+    __shared__ __align__(16) uint16_t stw[kTileN], nxt[kTileN];
+    __shared__ StartList starts;
+    __shared__ uint8_t entry[kSlotStride];
+    __shared__ unsigned entries;
+    const int tid = threadIdx.x;
+    const int tile = xcd_tile(p);
+    if (tile >= p.ntiles) return;  // the whole workgroup
+    if (tid == 0) starts.n = entries = 0;
+    const int ty = tile / p.tiles_x, tx = tile - ty * p.tiles_x;
+    const int r0 = ty * kTileR, c0 = tx * kTileC;
+    static_assert(kSwarTileR == kTileR && kSwarTileC == kTileC, "one tile shape");
+    const bool inner = sca_swar_tile(p, r0, c0);
+    if (inner) swar_words(p, S.swar, stw, r0, c0);
+    else general_words(p, S.general, stw, r0, c0);
     __syncthreads();
-    if (tid == 0) {
-        const unsigned n = waiting[0] + waiting[1] + waiting[2] + waiting[3];
-        add_waiting(p, n);
+    const unsigned long long slot0 = (unsigned long long)tile * kSlotStride;
+    // the pending inflows of this thread's perimeter cell from outside the tile
+    const int pcell = tid < kSlots ? cell_of_slot(tid) : 0;
+    unsigned ext = 0;
+    if (tid < kSlots) {
+        const int lr = pcell >> 6, lc = pcell & 63;
+        auto inm_at = [&](int r, int c) -> unsigned {
+            return inner ? reinterpret_cast<const uint8_t *>(S.swar.inm[r + 1])[c + 4] : S.general.inm[r + 1][c + 1];
+        };
+        const unsigned mine = (stw[pcell] & 15u) ? inm_at(lr, lc) : 0u;  // only a cell that waits at all
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int k = win_of_bit(j), ur = lr + k / 3 - 1, uc = lc + k % 3 - 1;
+            if ((unsigned)ur < (unsigned)kTileR && (unsigned)uc < (unsigned)kTileC) continue;
+            const int gr = r0 + ur, gc = c0 + uc;
+            const bool interior = gr >= 1 && gr <= p.rows - 2 && gc >= 1 && gc <= p.cols - 2;
+            if (interior && ((mine >> j) & 1u) && (p.converge || j < 4) && inm_at(ur, uc) != 0) ext |= 1u << j;
+        }
     }
-    // the tile's 4 x 8 blocks, one wave-wide 128-byte line per block
-    for (int i = tid; i < kTileR * kTileC; i += 256) {
-        const int blk = i >> 6, within = i & 63;
-        const int tr = (blk >> 3) * 8 + (within >> 3), tc = (blk & 7) * 8 + (within & 7);
-        const int r = r0 + tr, c = c0 + tc;
-        if ((r >> 3) < p.by && (c >> 3) < p.bx) p.st[st_index(p, r, c)] = stw[tr][tc];
+    const unsigned next_ = (unsigned)__builtin_popcount(ext);
+    // the static words go out as they are; the tile keeps them with the
+    // awaited inflows from inside only
+    const uint4 words = *reinterpret_cast<const uint4 *>(stw + 8 * tid);
+    *reinterpret_cast<uint4 *>(p.st + (long long)tile * kTileN + 8 * tid) = words;
+    store_next(nxt, words);
+    if (ext) entry[atomicAdd(&entries, 1u)] = (uint8_t)tid;
+    __syncthreads();  // the classes and masks are read
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const unsigned s = half_word(words, k);
+        S.acc[8 * tid + k] = (1u + nsrc_of(s)) | ((unsigned)poisoned_of(s) << kLocBad) | (npend_of(s) << kLocPend);
+    }
+    __syncthreads();
+    if (ext) S.acc[pcell] += (next_ << kLocExt) - (next_ << kLocPend);
+    __syncthreads();
+    {
+        unsigned m = 0;  // cells that wait for nothing and feed
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            m |= (unsigned)(feeds_of(half_word(words, k)) && (S.acc[8 * tid + k] >> kLocPend) == 0) << k;
+        add_starts(starts, m);
+    }
+    __syncthreads();
+    for (unsigned i = tid; i < starts.n; i += 256) {
+        unsigned t = starts.cell[i], v = S.acc[t];
+        t = nxt[t];
+        while (t < kLeaves) {
+            // areas, and inflows from outside, go on only with a done cell
+            const unsigned add = ((v >> kLocBad) & 15u ? 1u << kLocBad : v & ((1u << kLocBad) - 1)) - (1u << kLocPend);
+            const unsigned after = nxt[t];
+            v = atomicAdd(&S.acc[t], add) + add;
+            if ((v >> kLocPend) != 0) break;  // others are on their way
+            t = after;
+        }
+    }
+    // the exit that each entry leads to (by the waves that walk least); a
+    // cycle of codes leads to none
+    for (unsigned i = (unsigned)tid ^ 192u; i < entries; i += 256) {
+        const unsigned slot = entry[i];
+        unsigned t = (unsigned)cell_of_slot((int)slot);
+        for (int n = 0; n < kTileN && t < kLeaves; n++) t = nxt[t];
+        p.link[slot0 + slot] = (uint8_t)(t >= kLeaves && t != kEnds ? t - kLeaves : 255u);
+    }
+    __syncthreads();
+    if (tid < kSlotStride) {
+        unsigned long long x = kExitNever;
+        unsigned to = kNoExit;
+        if (tid < kSlots) {
+            const unsigned s = stw[pcell], v = S.acc[pcell], t = nxt[pcell];
+            const int k = code_of(s);
+            if (t >= kLeaves && t != kEnds) {
+                const int gr = r0 + (pcell >> 6) + k / 3 - 1, gc = c0 + (pcell & 63) + k % 3 - 1;
+                const int beside = (gr / kTileR) * p.tiles_x + gc / kTileC;
+                to = (unsigned)beside * kSlotStride + (unsigned)slot_of(gr % kTileR, gc % kTileC);
+                if ((v >> kLocPend) == 0) {
+                    const unsigned n = (v >> kLocExt) & 255u;
+                    if ((v >> kLocBad) & 15u) x = kExitStart | (1ull << kExitBad);  // not done, whatever arrives
+                    else x = (v & kLocSum) | ((unsigned long long)n << kExitPend) | (n == 0 ? kExitStart : 0ull);
+                }
+            }
+        }
+        p.exits[slot0 + tid] = x;
+        p.next[slot0 + tid] = to;
+        p.ext[slot0 + tid] = (uint8_t)ext;
     }
 }
 
-// Walks, persistent: every lane runs one hop per iteration; a lane without
-// a walk takes the next cell of its wave's chunk (chunks of kChunk cells in
-// block order come from a global cursor) and starts a walk there if the cell
-// waits for nothing and feeds its target.  Lanes stay busy until the cursor
-// passes the last cell and every walk of the wave has ended.  Checking one
-// cell per idle lane and iteration keeps the number of hops in flight, and
-// so the queueing delay on the longest chain, moderate: starting every walk
-// at once was slower.
-//
-// The static words do not change during the walk, so their loads may hit
-// any cache.  Accumulators are only touched by atomics until their cell
-// completes; after that only the completing lane writes the area there.
-constexpr long long kChunk = 4096;
-
-__device__ __forceinline__ long long first_lane(long long v)
+// Each exit's successor: the exit that the perimeter cell it enters leads
+// to, none if that one awaits nothing (it is not done whatever arrives) or
+// never completes.
+__global__ __launch_bounds__(256) void sca_link_kernel(ScaParams p, unsigned n)
 {
-    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v & 0xffffffffll));
-    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)((unsigned long long)v >> 32));
-    return (long long)(((unsigned long long)hi << 32) | lo);
+    const unsigned i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    const unsigned to = p.next[i];
+    if (to == kNoExit) return;
+    const unsigned slot = p.link[to];
+    unsigned x = kNoExit;
+    if (slot != 255u) {
+        x = to / kSlotStride * kSlotStride + slot;
+        const unsigned pend = (unsigned)(p.exits[x] >> kExitPend) & 255u;
+        if (pend == 0 || pend == 255u) x = kNoExit;
+    }
+    p.next[i] = x;
 }
 
-__global__ __launch_bounds__(256) void sca_walk_kernel(ScaParams p)
+// Walks over the exits: kCrossPer slots per lane, each lane going on to its
+// next slot when its walk has ended.
+constexpr int kCrossPer = 8;
+
+__global__ __launch_bounds__(256) void sca_cross_kernel(ScaParams p, unsigned n)
 {
-    const long long nwords = (long long)p.by * p.bx * 64;
-    long long chunk_next = 0, chunk_end = 0;  // the same in every lane of a wave
-    bool more = true;                         // the same in every lane of a wave
-    int cr = -1, cc = 0;                      // cell this lane's walk stands on (cr < 0: none)
-    int code = 0;
-    unsigned long long val = 0;
-    bool done = false;
-    unsigned completions = 0;
+    const unsigned base = blockIdx.x * (256u * kCrossPer) + threadIdx.x;
+    unsigned starts = 0;
+    unsigned long long w[kCrossPer];
+#pragma unroll
+    for (int k = 0; k < kCrossPer; k++) {
+        const unsigned i = base + 256u * k;
+        // an exit that awaits something changes while others arrive, but its
+        // start flag does not
+        w[k] = i < n ? __atomic_load_n(&p.exits[i], __ATOMIC_RELAXED) : 0ull;
+    }
+#pragma unroll
+    for (int k = 0; k < kCrossPer; k++) starts |= (unsigned)((w[k] & kExitStart) != 0) << k;
+    unsigned at = kNoExit;
+    unsigned long long v = 0;
     for (;;) {
-        // the target's static word is requested first, so that its latency
-        // overlaps the refill below
-        int tr = 0, tc = 0;
-        unsigned ts = 0;
-        if (cr >= 0) {
-            tr = cr + code / 3 - 1;
-            tc = cc + code % 3 - 1;
-            ts = p.st[st_index(p, tr, tc)];
+        if (at == kNoExit) {
+            if (starts == 0) break;
+            const int k = __builtin_ffs((int)starts) - 1;
+            starts &= starts - 1;
+            const unsigned i = base + 256u * (unsigned)k;
+            at = p.next[i];
+            v = 0;
+#pragma unroll
+            for (int q = 0; q < kCrossPer; q++)
+                if (q == k) v = w[q];
         }
-        const unsigned long long need = __ballot(cr < 0);
-        int fr = -1, fc = 0;
-        unsigned fs = 0;
-        if (need != 0 && more) {
-            if (chunk_next >= chunk_end) {
-                long long b = 0;
-                if (__lane_id() == 0) b = (long long)atomicAdd(&p.counters[0], (unsigned long long)kChunk);
-                b = first_lane(b);
-                if (b >= nwords) {
-                    more = false;
-                } else {
-                    chunk_next = b;
-                    chunk_end = b + kChunk < nwords ? b + kChunk : nwords;
-                }
-            }
-            if (more) {
-                const unsigned rank =
-                    __builtin_amdgcn_mbcnt_hi((unsigned)(need >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)need, 0u));
-                const long long npop = __popcll(need);
-                const long long take = npop < chunk_end - chunk_next ? npop : chunk_end - chunk_next;
-                if (cr < 0 && (long long)rank < take) {
-                    const long long idx = chunk_next + rank;
-                    fs = p.st[idx];
-                    const long long blk = idx >> 6;
-                    const int within = (int)(idx & 63);
-                    const int br = (int)(blk / p.bx);
-                    fr = br * 8 + (within >> 3);
-                    fc = (int)(blk - (long long)br * p.bx) * 8 + (within & 7);
-                }
-                chunk_next += take;
-            }
+        if (at != kNoExit) {
+            const unsigned after = p.next[at];
+            const unsigned long long add =
+                ((v >> kExitBad) & 255ull ? 1ull << kExitBad : v & ((1ull << kExitPend) - 1)) - (1ull << kExitPend);
+            v = atomicAdd(&p.exits[at], add) + add;
+            at = ((v >> kExitPend) & 255ull) == 0 ? after : kNoExit;
         }
-        if (cr >= 0) {
-            const long long t = (long long)tr * p.pitch + tc;
-            bool complete = true;
-            unsigned long long old = 0;  // other arrivals: none when the walk is the only one awaited
-            if (npend_of(ts) != 1) {
-                const unsigned long long add =
-                    (done ? val : 0ull) | ((unsigned long long)(!done) << 40) | (1ull << 44);
-                old = atomicAdd(&p.w[t], add);
-                complete = ((unsigned)(old >> 44) & 15u) + 1u == npend_of(ts);
-            }
-            if (!complete) {
-                cr = -1;  // an inflow is still on its way
-            } else {
-                const unsigned long long acc = (old & kAccMask) + (done ? val : 0ull);
-                const unsigned not_done = ((unsigned)(old >> 40) & 15u) + (done ? 0u : 1u);
-                done = !poisoned_of(ts) && not_done == 0;
-                val = 1ull + nsrc_of(ts) + acc;
-                p.w[t] = bits_of((double)val);
-                completions++;
-                if (tr >= p.rows - 3 && tc >= p.cols - 3)
-                    p.last_done[(tr - (p.rows - 3)) * 3 + (tc - (p.cols - 3))] = done ? 1u : 0u;
-                if (feeds_of(ts)) {
-                    cr = tr;
-                    cc = tc;
-                    code = code_of(ts);
-                } else {
-                    cr = -1;
-                }
-            }
-        } else if (fr >= 0 && area_of(fs) && npend_of(fs) == 0 && feeds_of(fs)) {
-            cr = fr;
-            cc = fc;
-            code = code_of(fs);
-            val = 1ull + nsrc_of(fs);
-            done = !poisoned_of(fs);
-        }
-        if (!more && __ballot(cr >= 0) == 0) break;
     }
-    completions = wave_sum(completions);
-    if (__lane_id() == 0 && completions) atomicAdd(&p.counters[2], (unsigned long long)completions);
 }
 
-// Cells that never completed (their counts disagree only then): the area of
-// the done arrivals they received, as the converging semantics defines it.
-__global__ __launch_bounds__(256) void sca_open_kernel(ScaParams p)
+__global__ __launch_bounds__(256) void sca_final_kernel(ScaParams p)
 {
-    unsigned long long waiting = 0;
-    for (int i = 0; i < kWaitSlots; i++) waiting += p.wait_slots[i * kWaitStride];
-    if (waiting == p.counters[2]) return;
-    const long long n = (long long)p.rows * p.cols;
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
-        const int r = (int)(i / p.cols), c = (int)(i - (long long)r * p.cols);
-        const unsigned s = p.st[st_index(p, r, c)];
-        if (!area_of(s) || npend_of(s) == 0) continue;
-        const long long o = (long long)r * p.pitch + c;
-        const unsigned long long w = p.w[o];
-        if (w & kOpen) p.w[o] = bits_of((double)(1ull + nsrc_of(s) + (w & kAccMask)));
+    __shared__ unsigned long long acc[kTileN];
+    __shared__ __align__(16) uint16_t nxt[kTileN];
+    __shared__ StartList starts;
+    const int tid = threadIdx.x;
+    const int tile = xcd_tile(p);
+    if (tile >= p.ntiles) return;  // the whole workgroup
+    if (tid == 0) starts.n = 0;
+    const int ty = tile / p.tiles_x, tx = tile - ty * p.tiles_x;
+    const int r0 = ty * kTileR, c0 = tx * kTileC;
+    const uint4 words = *reinterpret_cast<const uint4 *>(p.st + (long long)tile * kTileN + 8 * tid);
+    const int pcell = tid < kSlots ? cell_of_slot(tid) : 0;
+    // what arrives at this thread's perimeter cell from outside: every load
+    // is issued before the first word is looked at (the slots that are not
+    // inflows read the tile's own first word)
+    const unsigned long long slot0 = (unsigned long long)tile * kSlotStride;
+    const unsigned ext = tid < kSlots ? p.ext[slot0 + tid] : 0u;
+    unsigned long long arrived = 0;
+    if (ext) {
+        unsigned long long x[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int k = win_of_bit(j), gr = r0 + (pcell >> 6) + k / 3 - 1, gc = c0 + (pcell & 63) + k % 3 - 1;
+            const unsigned long long u = (unsigned long long)((gr / kTileR) * p.tiles_x + gc / kTileC) * kSlotStride +
+                                         (unsigned)slot_of(gr % kTileR, gc % kTileC);
+            x[j] = p.exits[(ext >> j) & 1u ? u : slot0];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            if (!((ext >> j) & 1u) || ((x[j] >> kExitPend) & 255ull) != 0) continue;  // no inflow, or never complete
+            arrived += ((x[j] >> kExitBad) & 255ull ? 1ull << kFinBad : x[j] & kFinSum) - (1ull << kFinPend);
+        }
+    }
+    store_next(nxt, words);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const unsigned s = half_word(words, k);
+        acc[8 * tid + k] = area_of(s) ? kFinArea | (1ull + nsrc_of(s)) | ((unsigned long long)poisoned_of(s) << kFinBad) |
+                                            ((unsigned long long)npend_of(s) << kFinPend)
+                                      : 0ull;
+    }
+    __syncthreads();
+    if (ext) acc[pcell] += arrived;
+    __syncthreads();
+    {
+        unsigned m = 0;  // cells that wait for nothing and feed
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            m |= (unsigned)(feeds_of(half_word(words, k)) && ((acc[8 * tid + k] >> kFinPend) & 15ull) == 0) << k;
+        add_starts(starts, m);
+    }
+    __syncthreads();
+    for (unsigned i = tid; i < starts.n; i += 256) {
+        unsigned t = starts.cell[i];
+        unsigned long long v = acc[t];
+        t = nxt[t];
+        while (t < kLeaves) {
+            const unsigned long long add = ((v >> kFinBad) & 15ull ? 1ull << kFinBad : v & kFinSum) - (1ull << kFinPend);
+            const unsigned after = nxt[t];
+            v = atomicAdd(&acc[t], add) + add;
+            if (((v >> kFinPend) & 15ull) != 0) break;  // others are on their way
+            t = after;
+        }
+    }
+    __syncthreads();
+    const int lane = tid & 63, wave = tid >> 6, c = c0 + lane;
+    if (c >= p.cols) return;
+#pragma unroll
+    for (int k = 0; k < kTileR / 4; k++) {
+        const int tr = wave + 4 * k, r = r0 + tr;
+        if (r >= p.rows) break;
+        const unsigned long long v = acc[tr * kTileC + lane];
+        const double a = v & kFinArea ? (double)(v & kFinSum) : p.nodata;
+        __builtin_nontemporal_store(a, &p.area[(long long)r * p.pitch + c]);
+        if (r >= p.rows - 3 && c >= p.cols - 3)
+            p.last_done[(r - (p.rows - 3)) * 3 + (c - (p.cols - 3))] = (v >> kFinBad) == kFinArea >> kFinBad ? 1u : 0u;
     }
 }
 
@@ -524,12 +673,9 @@ __global__ void sca_last_cell_kernel(ScaParams p)
         const int ur = r + k / 3 - 1, uc = c + k % 3 - 1;
         if (ur < 1 || ur > p.rows - 2 || uc < 1 || uc > p.cols - 2) continue;
         if (flow_of(load_class(p, ur, uc)) != (unsigned)(8 - k)) continue;
-        const unsigned s = p.st[st_index(p, ur, uc)];
-        const bool done = npend_of(s) == 0 ? !poisoned_of(s)
-                                           : p.last_done[(ur - (p.rows - 3)) * 3 + (uc - (p.cols - 3))] != 0;
-        if (done) v += __longlong_as_double((long long)p.w[(long long)ur * p.pitch + uc]);
+        if (p.last_done[(ur - (p.rows - 3)) * 3 + (uc - (p.cols - 3))]) v += p.area[(long long)ur * p.pitch + uc];
     }
-    p.w[(long long)r * p.pitch + c] = bits_of(v);
+    p.area[(long long)r * p.pitch + c] = v;
 }
 
 // Reference D8 layer (double) to flow classes: NoData when
@@ -625,40 +771,39 @@ extern "C" int pargo_sca_d8(pargo_ctx *ctx, const pargo_grid *g, const uint8_t *
     if (ntiles > (1ll << 24))
         return fail(ctx, PARGO_E_INVALID, "grid of %d x %d cells needs %lld tiles, more than 2^24", g->rows, g->cols,
                     ntiles);
-    // scratch: counters and last-cell flags, the waiting-cell partial
-    // counts, then the static words in 8 x 8 blocks (2 bytes per cell, rows
-    // and columns rounded up to 8)
-    const int bx = (g->cols + 7) / 8, by = (g->rows + 7) / 8;
-    const size_t head = 256 + (size_t)pargo::kWaitSlots * pargo::kWaitStride * sizeof(unsigned long long);
-    rc = pargo::ensure_scratch(ctx, head + (size_t)bx * by * 64 * sizeof(uint16_t));
+    // scratch: the last-cell flags, then per tile the static words (2 bytes
+    // per cell) and, per perimeter slot, the exit word, its successor, the
+    // entry's exit and its inflows from outside
+    constexpr size_t head = 256;
+    const size_t slots = (size_t)ntiles * pargo::kSlotStride;
+    rc = pargo::ensure_scratch(ctx, head + (size_t)ntiles * pargo::kTileN * sizeof(uint16_t) + slots * (8 + 4 + 1 + 1));
     if (rc) return rc;
     char *scr = static_cast<char *>(ctx->scratch);
     pargo::ScaParams p{};
     p.flow = flow;
     p.mask = nodata_mask;
-    p.w = reinterpret_cast<unsigned long long *>(sca_out);
-    p.st = reinterpret_cast<uint16_t *>(scr + head);
-    p.counters = reinterpret_cast<unsigned long long *>(scr);
-    p.last_done = reinterpret_cast<unsigned *>(scr + 64);
-    p.wait_slots = reinterpret_cast<unsigned long long *>(scr + 256);
+    p.area = sca_out;
+    p.last_done = reinterpret_cast<unsigned *>(scr);
+    p.exits = reinterpret_cast<unsigned long long *>(scr + head);
+    p.st = reinterpret_cast<uint16_t *>(p.exits + slots);
+    p.next = reinterpret_cast<unsigned *>(p.st + (size_t)ntiles * pargo::kTileN);
+    p.link = reinterpret_cast<uint8_t *>(p.next + slots);
+    p.ext = p.link + slots;
     p.pitch = pitch;
     p.rows = g->rows;
     p.cols = g->cols;
     p.mask_words = (g->cols + 31) / 32;
-    p.bx = bx;
-    p.by = by;
+    p.tiles_x = tiles_x;
+    p.ntiles = (int)ntiles;
     p.converge = mode == PARGO_SCA_CONVERGE;
     p.nodata = g->nodata;
-    hipLaunchKernelGGL(pargo::sca_reset_kernel, dim3(1), dim3(64), 0, ctx->stream, p);
-    const int per_xcd = (int)((ntiles + 7) / 8);
-    hipLaunchKernelGGL(pargo::sca_init_kernel, dim3(8 * per_xcd), dim3(256), 0, ctx->stream, p, tiles_x, (int)ntiles);
-    // persistent walk: 4 workgroups of 4 waves per CU.  Fewer walks in flight
-    // queue less on the longest chains; measured at 16384^2 (reference /
-    // converging mode): 1 per CU 8.0 / 11.6 ms, 2 5.4 / 8.3, 4 4.4 / 7.6,
-    // 8 4.6 / 8.3, 16 4.6 / 8.3
-    const int cus = ctx->num_cu > 0 ? ctx->num_cu : 256;
-    hipLaunchKernelGGL(pargo::sca_walk_kernel, dim3(cus * 4), dim3(256), 0, ctx->stream, p);
-    hipLaunchKernelGGL(pargo::sca_open_kernel, dim3(cus * 4), dim3(256), 0, ctx->stream, p);
+    const dim3 tiles(8 * (unsigned)((ntiles + 7) / 8)), threads(256);
+    const unsigned n = (unsigned)slots;
+    hipLaunchKernelGGL(pargo::sca_local_kernel, tiles, threads, 0, ctx->stream, p);
+    hipLaunchKernelGGL(pargo::sca_link_kernel, dim3((n + 255u) / 256u), threads, 0, ctx->stream, p, n);
+    constexpr unsigned per = 256u * pargo::kCrossPer;
+    hipLaunchKernelGGL(pargo::sca_cross_kernel, dim3((n + per - 1) / per), threads, 0, ctx->stream, p, n);
+    hipLaunchKernelGGL(pargo::sca_final_kernel, tiles, threads, 0, ctx->stream, p);
     if (last_rule) hipLaunchKernelGGL(pargo::sca_last_cell_kernel, dim3(1), dim3(1), 0, ctx->stream, p);
     return pargo::check_launch(ctx, "pargo_sca_d8");
 }
