@@ -171,10 +171,11 @@ __device__ __forceinline__ int xcd_tile(const ScaParams &p)
     return (g & 7) * per + (g >> 3);
 }
 
+typedef uint32_t u32_b1 __attribute__((aligned(1)));  // one dword load at any byte address on gfx950
+
 // A tile at least 2 cells from every border whose class rows can be read
-// as words, four cells per word (sca_swar.h): the halo columns c0 - 8 ..
-// c0 + 71, each word from the aligned pair around it, so bytes c0 - 11 ..
-// c0 + 75 of each row are read.
+// as words, four cells per word (sca_swar.h): columns c0 - 8 .. c0 + 71 of
+// each row (the bound leaves a word more on either side).
 __device__ __forceinline__ bool sca_swar_tile(const ScaParams &p, int r0, int c0)
 {
     return r0 >= 2 && r0 + kSwarTileR + 2 <= p.rows && c0 >= 11 && c0 + 76 <= p.cols;
@@ -188,21 +189,16 @@ __device__ __forceinline__ void swar_words(const ScaParams &p, SwarTile &T, uint
     const int tid = threadIdx.x;
     {
         constexpr int N = kSwarClsRows * kSwarClsWords, PER = (N + 255) / 256;
-        uint32_t lo[PER], hi[PER], mw[PER];
-        unsigned sh[PER];
+        uint32_t v[PER], mw[PER];
         // every load of the thread is issued before the first is used
 #pragma unroll
         for (int k = 0; k < PER; k++) {
             const int i = tid + 256 * k;
-            lo[k] = hi[k] = mw[k] = sh[k] = 0;
+            v[k] = mw[k] = 0;
             if (i < N) {
                 const int rr = i / kSwarClsWords, w = i - rr * kSwarClsWords;
                 const int r = r0 - 2 + rr, col = c0 - 8 + 4 * w;
-                const uintptr_t a = (uintptr_t)(p.flow + (long long)r * p.pitch + col);
-                const uint32_t *al = reinterpret_cast<const uint32_t *>(a & ~(uintptr_t)3);
-                sh[k] = (unsigned)(a & 3);
-                lo[k] = al[0];
-                hi[k] = al[1];
+                v[k] = *reinterpret_cast<const u32_b1 *>(p.flow + (long long)r * p.pitch + col);
                 if (p.mask) mw[k] = p.mask[(long long)r * p.mask_words + (col >> 5)] >> (col & 31);
             }
         }
@@ -211,24 +207,41 @@ __device__ __forceinline__ void swar_words(const ScaParams &p, SwarTile &T, uint
             const int i = tid + 256 * k;
             if (i < N) {
                 const int rr = i / kSwarClsWords, w = i - rr * kSwarClsWords;
-                const uint32_t v = swar_select(swar_bits_to_mask(mw[k]), swar_splat(PARGO_FLOW_NODATA),
-                                               __builtin_amdgcn_alignbyte(hi[k], lo[k], sh[k]));
-                T.cls[rr][w] = v;
-                T.tgt[rr][w] = swar_flow_of(v);
+                const uint32_t b = p.mask ? swar_select(swar_bits_to_mask(mw[k]), swar_splat(PARGO_FLOW_NODATA), v[k]) : v[k];
+                T.cls[rr][w] = b;
+                T.tgt[rr][w] = swar_flow_of(b);
             }
         }
     }
     __syncthreads();
-    for (int i = tid; i < kSwarInmRows * kSwarInmWords; i += 256) {
-        const int lr = i / kSwarInmWords, q = i - lr * kSwarInmWords;
-        T.inm[lr][q] = swar_inflow(T, lr, q);
+    // Two words, eight cells, at a time: the four words of a row they need
+    // are two aligned 64-bit reads (the compiler joined the three words of a
+    // single one into unaligned 96-bit reads, and the LDS spent 7,000 cycles
+    // a tile on those, 60 % of them stalled on the alignment).
+    struct Four {
+        uint32_t w[4];
+    };
+    auto four = [](const uint32_t *row, int w) -> Four {
+        const uint2 a = *reinterpret_cast<const uint2 *>(row + w), b = *reinterpret_cast<const uint2 *>(row + w + 2);
+        return Four{{a.x, a.y, b.x, b.y}};
+    };
+    static_assert(kSwarClsWords % 2 == 0 && kSwarInmWords % 2 == 0, "rows keep the 8-byte alignment");
+    for (int i = tid; i < kSwarInmRows * (kSwarInmWords / 2); i += 256) {
+        const int lr = i / (kSwarInmWords / 2), q = 2 * (i - lr * (kSwarInmWords / 2));
+        const Four b = four(T.cls[lr + 1], q);
+        const Four t0 = four(T.tgt[lr], q), t1 = four(T.tgt[lr + 1], q), t2 = four(T.tgt[lr + 2], q);
+        *reinterpret_cast<uint2 *>(&T.inm[lr][q]) =
+            make_uint2(swar_inflow_rows(b.w[1], t0.w, t1.w, t2.w, 0), swar_inflow_rows(b.w[2], t0.w, t1.w, t2.w, 1));
     }
     __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int v = tid + 256 * k, tr = v >> 4, g = v & 15;
-        const SwarCells o = swar_cells(T, tr, g, p.converge != 0);
-        *reinterpret_cast<uint2 *>(stw + tr * kTileC + 4 * g) = make_uint2(o.s01, o.s23);
+    {
+        const int tr = tid >> 3, g = 2 * (tid & 7);
+        const uint2 b = *reinterpret_cast<const uint2 *>(&T.cls[tr + 2][g + 2]);
+        const uint2 f = *reinterpret_cast<const uint2 *>(&T.tgt[tr + 2][g + 2]);
+        const Four m0 = four(T.inm[tr], g), m1 = four(T.inm[tr + 1], g), m2 = four(T.inm[tr + 2], g);
+        const SwarCells u = swar_cells_rows(b.x, f.x, m0.w, m1.w, m2.w, 0, p.converge != 0);
+        const SwarCells v = swar_cells_rows(b.y, f.y, m0.w, m1.w, m2.w, 1, p.converge != 0);
+        *reinterpret_cast<uint4 *>(stw + 8 * tid) = make_uint4(u.s01, u.s23, v.s01, v.s23);
     }
 }
 
@@ -373,7 +386,9 @@ struct StartList {
     uint16_t cell[kStarts];
     unsigned n;
 };
-// Adds this thread's cells 8 tid + k with bit k of `m` set (all lanes call).
+// A thread's cells from here on: column `lane` of tile rows wave + 4k.
+__device__ __forceinline__ int my_cell(int k) { return ((int)(threadIdx.x >> 6) + 4 * k) * kTileC + (int)(threadIdx.x & 63); }
+// Adds the thread's cells k with bit k of `m` set (all lanes call).
 __device__ __forceinline__ void add_starts(StartList &L, unsigned m)
 {
     unsigned total = 0;
@@ -387,23 +402,18 @@ __device__ __forceinline__ void add_starts(StartList &L, unsigned m)
         const unsigned long long b = __builtin_amdgcn_ballot_w64((m >> k) & 1u);
         if ((m >> k) & 1u)
             L.cell[at + __builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b, 0u))] =
-                (uint16_t)(8 * threadIdx.x + k);
+                (uint16_t)my_cell(k);
         at += (unsigned)__builtin_popcountll(b);
     }
 }
-__device__ __forceinline__ unsigned half_word(const uint4 &w, int k)
+// next_of for a cell whose next cell lies in the tile (perimeter cells are
+// set by next_of afterwards): the index plus the code's offset, by a byte
+// lookup for codes 0..7 (the centre, code 4, never feeds).
+__device__ __forceinline__ unsigned next_inside(int idx, unsigned s)
 {
-    const unsigned h = k < 2 ? w.x : k < 4 ? w.y : k < 6 ? w.z : w.w;
-    return (h >> (16 * (k & 1))) & 0xffffu;
-}
-// The thread's eight next_of values into `nxt`.
-__device__ __forceinline__ void store_next(uint16_t *nxt, const uint4 &words)
-{
-    unsigned n[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) n[k] = next_of(8 * (int)threadIdx.x + k, half_word(words, k));
-    *reinterpret_cast<uint4 *>(nxt + 8 * threadIdx.x) =
-        make_uint4(n[0] | n[1] << 16, n[2] | n[3] << 16, n[4] | n[5] << 16, n[6] | n[7] << 16);
+    const unsigned code = (s >> 10) & 15u;
+    const int off = code == 8u ? 65 : (int)(int8_t)__builtin_amdgcn_perm(0x403F0100u, 0xFFC1C0BFu, code);
+    return feeds_of(s) ? (unsigned)(idx + off) & 0xFFFFu : kEnds;
 }
 
 union LocalShared {
@@ -454,22 +464,26 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
     // awaited inflows from inside only
     const uint4 words = *reinterpret_cast<const uint4 *>(stw + 8 * tid);
     *reinterpret_cast<uint4 *>(p.st + (long long)tile * kTileN + 8 * tid) = words;
-    store_next(nxt, words);
+    unsigned s[kTileN / 256];
+#pragma unroll
+    for (int k = 0; k < kTileN / 256; k++) {
+        s[k] = stw[my_cell(k)];
+        nxt[my_cell(k)] = (uint16_t)next_inside(my_cell(k), s[k]);
+    }
     if (ext) entry[atomicAdd(&entries, 1u)] = (uint8_t)tid;
     __syncthreads();  // the classes and masks are read
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const unsigned s = half_word(words, k);
-        S.acc[8 * tid + k] = (1u + nsrc_of(s)) | ((unsigned)poisoned_of(s) << kLocBad) | (npend_of(s) << kLocPend);
-    }
+    for (int k = 0; k < kTileN / 256; k++)
+        S.acc[my_cell(k)] = (1u + nsrc_of(s[k])) | ((unsigned)poisoned_of(s[k]) << kLocBad) | (npend_of(s[k]) << kLocPend);
     __syncthreads();
+    if (tid < kSlots) nxt[pcell] = (uint16_t)next_of(pcell, stw[pcell]);
     if (ext) S.acc[pcell] += (next_ << kLocExt) - (next_ << kLocPend);
     __syncthreads();
     {
         unsigned m = 0;  // cells that wait for nothing and feed
 #pragma unroll
-        for (int k = 0; k < 8; k++)
-            m |= (unsigned)(feeds_of(half_word(words, k)) && (S.acc[8 * tid + k] >> kLocPend) == 0) << k;
+        for (int k = 0; k < kTileN / 256; k++)
+            m |= (unsigned)(feeds_of(s[k]) && (S.acc[my_cell(k)] >> kLocPend) == 0) << k;
         add_starts(starts, m);
     }
     __syncthreads();
@@ -596,6 +610,7 @@ __global__ __launch_bounds__(256) void sca_final_kernel(ScaParams p)
     // inflows read the tile's own first word)
     const unsigned long long slot0 = (unsigned long long)tile * kSlotStride;
     const unsigned ext = tid < kSlots ? p.ext[slot0 + tid] : 0u;
+    const unsigned pword = tid < kSlots ? p.st[(long long)tile * kTileN + pcell] : 0u;
     unsigned long long arrived = 0;
     if (ext) {
         unsigned long long x[8];
@@ -612,22 +627,27 @@ __global__ __launch_bounds__(256) void sca_final_kernel(ScaParams p)
             arrived += ((x[j] >> kExitBad) & 255ull ? 1ull << kFinBad : x[j] & kFinSum) - (1ull << kFinPend);
         }
     }
-    store_next(nxt, words);
+    *reinterpret_cast<uint4 *>(nxt + 8 * tid) = words;
+    __syncthreads();
+    unsigned s[kTileN / 256];
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const unsigned s = half_word(words, k);
-        acc[8 * tid + k] = area_of(s) ? kFinArea | (1ull + nsrc_of(s)) | ((unsigned long long)poisoned_of(s) << kFinBad) |
-                                            ((unsigned long long)npend_of(s) << kFinPend)
-                                      : 0ull;
+    for (int k = 0; k < kTileN / 256; k++) {
+        s[k] = nxt[my_cell(k)];  // each cell's word is read and written by one thread
+        nxt[my_cell(k)] = (uint16_t)next_inside(my_cell(k), s[k]);
+        acc[my_cell(k)] = area_of(s[k]) ? kFinArea | (1ull + nsrc_of(s[k])) |
+                                              ((unsigned long long)poisoned_of(s[k]) << kFinBad) |
+                                              ((unsigned long long)npend_of(s[k]) << kFinPend)
+                                        : 0ull;
     }
     __syncthreads();
+    if (tid < kSlots) nxt[pcell] = (uint16_t)next_of(pcell, pword);
     if (ext) acc[pcell] += arrived;
     __syncthreads();
     {
         unsigned m = 0;  // cells that wait for nothing and feed
 #pragma unroll
-        for (int k = 0; k < 8; k++)
-            m |= (unsigned)(feeds_of(half_word(words, k)) && ((acc[8 * tid + k] >> kFinPend) & 15ull) == 0) << k;
+        for (int k = 0; k < kTileN / 256; k++)
+            m |= (unsigned)(feeds_of(s[k]) && ((acc[my_cell(k)] >> kFinPend) & 15ull) == 0) << k;
         add_starts(starts, m);
     }
     __syncthreads();

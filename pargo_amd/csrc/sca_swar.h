@@ -18,7 +18,7 @@ constexpr int kSwarClsRows = kSwarTileR + 4, kSwarClsWords = 20;
 constexpr int kSwarInmRows = kSwarTileR + 2, kSwarInmWords = 18;
 constexpr uint32_t kSwarNoData = 254u, kSwarInert = 253u, kSwarExcl = 0x10u;
 
-struct SwarTile {
+struct alignas(16) SwarTile {
     uint32_t cls[kSwarClsRows][kSwarClsWords];
     uint32_t tgt[kSwarClsRows][kSwarClsWords];  // target window index of each class, 15 if none
     uint32_t inm[kSwarInmRows][kSwarInmWords];  // inflow masks
@@ -46,6 +46,11 @@ PARGO_SWAR_FN uint32_t swar_perm(uint32_t hi, uint32_t lo, uint32_t sel)
 #endif
 }
 
+// 0x80 in each byte of x that is 0, for bytes of at most 0x80; the other
+// bits of the byte are whatever is left (mask them off).  One subtraction
+// where the general test takes four operations.
+PARGO_SWAR_FN uint32_t swar_small_zero(uint32_t x) { return kSwarHi - x; }
+
 // targets: the class itself for 0..8 except 4, else 15
 PARGO_SWAR_FN uint32_t swar_flow_of(uint32_t b)
 {
@@ -60,19 +65,18 @@ PARGO_SWAR_FN uint32_t swar_row_window(const uint32_t *row, int w, int dc)
     return dc < 0 ? swar_window(row[w], row[w + 1], 3) : (dc == 0 ? row[w + 1] : swar_window(row[w + 1], row[w + 2], 1));
 }
 
-// Inflow masks of the four cells of inflow word (lr, q) (class row lr + 1,
-// class word q + 1): bit j set when the neighbour at window position
-// swar_win_of_bit(j) drains into the cell and the cell does not exclude
-// it; zero for NoData and inert cells.
-PARGO_SWAR_FN uint32_t swar_inflow(const SwarTile &T, int lr, int q)
+// Inflow masks of the four cells with classes b: bit j set when the
+// neighbour at window position swar_win_of_bit(j) drains into the cell and
+// the cell does not exclude it; zero for NoData and inert cells.  t0, t1, t2:
+// the targets of the rows above, at and below the cells, their word at w + 1.
+PARGO_SWAR_FN uint32_t swar_inflow_rows(uint32_t b, const uint32_t *t0, const uint32_t *t1, const uint32_t *t2, int w)
 {
-    const uint32_t b = T.cls[lr + 1][q + 1];
     uint32_t m = 0;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
         const int k = swar_win_of_bit(j), dr = k / 3 - 1, dc = k % 3 - 1;
-        const uint32_t win = swar_row_window(T.tgt[lr + 1 + dr], q, dc);
-        m |= swar_zero(win ^ swar_splat((uint32_t)(8 - k))) >> (7 - j);
+        const uint32_t win = swar_row_window(dr < 0 ? t0 : dr == 0 ? t1 : t2, w, dc);
+        m |= (swar_small_zero(win ^ swar_splat((uint32_t)(8 - k))) >> (7 - j)) & swar_splat(1u << j);
     }
     // the excluded window position: the class for 0..8, its low nibble for
     // PARGO_FLOW_EXCL | k (k <= 8); bit swar_bit_of_win(k) is cleared
@@ -86,9 +90,16 @@ PARGO_SWAR_FN uint32_t swar_inflow(const SwarTile &T, int lr, int q)
     return m & keep & ~swar_mask(invalid);
 }
 
-// The four cells of tile row tr, columns c0 + 4g ..: static words (s01:
-// cells 0 and 1, s23: cells 2 and 3, 16 bits each), and per byte the
-// pending and source counts and the NoData / inert flags.
+// The same for inflow word (lr, q) of a tile (class row lr + 1, class word
+// q + 1).
+PARGO_SWAR_FN uint32_t swar_inflow(const SwarTile &T, int lr, int q)
+{
+    return swar_inflow_rows(T.cls[lr + 1][q + 1], T.tgt[lr], T.tgt[lr + 1], T.tgt[lr + 2], q);
+}
+
+// Four cells: static words (s01: cells 0 and 1, s23: cells 2 and 3, 16 bits
+// each), and per byte the pending and source counts and the NoData / inert
+// flags.
 struct SwarCells {
     uint32_t s01, s23;
     uint32_t npend, nsrc;     // counts per byte
@@ -96,26 +107,27 @@ struct SwarCells {
     uint32_t waiting;         // 0x80 flags: valid cells with npend > 0
 };
 
-PARGO_SWAR_FN SwarCells swar_cells(const SwarTile &T, int tr, int g, bool converge)
+// Of cells with classes b and targets f; m0, m1, m2: the inflow masks of the
+// rows above, at and below the cells, their word at w + 1.
+PARGO_SWAR_FN SwarCells swar_cells_rows(uint32_t b, uint32_t f, const uint32_t *m0, const uint32_t *m1,
+                                        const uint32_t *m2, int w, bool converge)
 {
-    const uint32_t b = T.cls[tr + 2][g + 2];
-    const uint32_t f = T.tgt[tr + 2][g + 2];
-    const uint32_t mine = T.inm[tr + 1][g + 1];
+    const uint32_t mine = m1[w + 1];
     uint32_t srcn = 0, feeds = 0;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
         const int k = swar_win_of_bit(j), dr = k / 3 - 1, dc = k % 3 - 1;
-        const uint32_t win = swar_row_window(T.inm[tr + 1 + dr], g, dc);
+        const uint32_t win = swar_row_window(dr < 0 ? m0 : dr == 0 ? m1 : m2, w, dc);
         srcn |= swar_zero(win) >> (7 - j);
         // a cell draining to window k feeds when its target's inflow mask
         // has it (bit swar_bit_of_win(8 - k) of that mask), and then only in
         // the converging mode or when the target comes later in the sweep
         if (converge || k > 4) {
             const int tb = swar_bit_of_win(8 - k);
-            feeds |= swar_zero(f ^ swar_splat((uint32_t)k)) & (win << (7 - tb));
+            feeds |= swar_small_zero(f ^ swar_splat((uint32_t)k)) & (win << (7 - tb));
         }
     }
-    feeds &= ~swar_zero(mine);  // sources never walk
+    feeds &= ~swar_zero(mine) & kSwarHi;  // sources never walk
     const uint32_t waitable = converge ? 0xFFFFFFFFu : 0x0F0F0F0Fu;  // window bits 0-3: NW, N, NE, W
     SwarCells o;
     o.nsrc = swar_popc(mine & srcn);
@@ -132,6 +144,12 @@ PARGO_SWAR_FN SwarCells swar_cells(const SwarTile &T, int tr, int g, bool conver
     o.s23 = swar_perm(hb, lb, 0x07030602u);
     o.waiting = ~swar_zero(o.npend) & kSwarHi & vm;
     return o;
+}
+
+// The same for the cells of tile row tr, columns c0 + 4g ..
+PARGO_SWAR_FN SwarCells swar_cells(const SwarTile &T, int tr, int g, bool converge)
+{
+    return swar_cells_rows(T.cls[tr + 2][g + 2], T.tgt[tr + 2][g + 2], T.inm[tr], T.inm[tr + 1], T.inm[tr + 2], g, converge);
 }
 
 }  // namespace pargo
