@@ -64,9 +64,9 @@
 // admits for arbitrary codes) keep the sum of the done inflows they
 // received, which is their area.
 //
-// Measured on the headline DEM's codes: 16384^2 in the reference mode 2.85 ms
-// (local 1.70, link 0.07, cross 0.12, final 1.00), 5003 x 7001 in the
-// converging mode 0.46 ms, and 0.11 ms for the codes of a filled 1501 x 2003
+// Measured on the headline DEM's codes: 16384^2 in the reference mode 2.06 ms
+// (local 0.99, link 0.07, cross 0.12, final 0.94), 5003 x 7001 in the
+// converging mode 0.35 ms, and 0.11 ms for the codes of a filled 1501 x 2003
 // DEM, whose paths are long.  One walk over the whole raster with a global
 // atomic or a static word read per hop (33 bytes of HBM traffic, up to 1336
 // hops in a row) took 4.24, 1.21 and 1.15 ms.
@@ -219,11 +219,11 @@ __device__ __forceinline__ void swar_words(const ScaParams &p, SwarTile &T, uint
     // single one into unaligned 96-bit reads, and the LDS spent 7,000 cycles
     // a tile on those, 60 % of them stalled on the alignment).
     struct Four {
-        uint32_t w[4];
+        SwarRow lo, hi;  // around the first and the second word of the pair
     };
     auto four = [](const uint32_t *row, int w) -> Four {
         const uint2 a = *reinterpret_cast<const uint2 *>(row + w), b = *reinterpret_cast<const uint2 *>(row + w + 2);
-        return Four{{a.x, a.y, b.x, b.y}};
+        return Four{{a.x, a.y, b.x}, {a.y, b.x, b.y}};
     };
     static_assert(kSwarClsWords % 2 == 0 && kSwarInmWords % 2 == 0, "rows keep the 8-byte alignment");
     for (int i = tid; i < kSwarInmRows * (kSwarInmWords / 2); i += 256) {
@@ -231,7 +231,7 @@ __device__ __forceinline__ void swar_words(const ScaParams &p, SwarTile &T, uint
         const Four b = four(T.cls[lr + 1], q);
         const Four t0 = four(T.tgt[lr], q), t1 = four(T.tgt[lr + 1], q), t2 = four(T.tgt[lr + 2], q);
         *reinterpret_cast<uint2 *>(&T.inm[lr][q]) =
-            make_uint2(swar_inflow_rows(b.w[1], t0.w, t1.w, t2.w, 0), swar_inflow_rows(b.w[2], t0.w, t1.w, t2.w, 1));
+            make_uint2(swar_inflow_rows(b.lo.b, t0.lo, t1.lo, t2.lo), swar_inflow_rows(b.hi.b, t0.hi, t1.hi, t2.hi));
     }
     __syncthreads();
     {
@@ -239,8 +239,8 @@ __device__ __forceinline__ void swar_words(const ScaParams &p, SwarTile &T, uint
         const uint2 b = *reinterpret_cast<const uint2 *>(&T.cls[tr + 2][g + 2]);
         const uint2 f = *reinterpret_cast<const uint2 *>(&T.tgt[tr + 2][g + 2]);
         const Four m0 = four(T.inm[tr], g), m1 = four(T.inm[tr + 1], g), m2 = four(T.inm[tr + 2], g);
-        const SwarCells u = swar_cells_rows(b.x, f.x, m0.w, m1.w, m2.w, 0, p.converge != 0);
-        const SwarCells v = swar_cells_rows(b.y, f.y, m0.w, m1.w, m2.w, 1, p.converge != 0);
+        const SwarCells u = swar_cells_rows(b.x, f.x, m0.lo, m1.lo, m2.lo, p.converge != 0);
+        const SwarCells v = swar_cells_rows(b.y, f.y, m0.hi, m1.hi, m2.hi, p.converge != 0);
         *reinterpret_cast<uint4 *>(stw + 8 * tid) = make_uint4(u.s01, u.s23, v.s01, v.s23);
     }
 }

@@ -58,24 +58,32 @@ PARGO_SWAR_FN uint32_t swar_flow_of(uint32_t b)
     return swar_select(swar_mask(ok), b, swar_splat(15));
 }
 
-// four consecutive bytes of a row of words, starting dc bytes (-1, 0, 1)
-// from word w + 1 (the word of the cells)
-PARGO_SWAR_FN uint32_t swar_row_window(const uint32_t *row, int w, int dc)
+// Three consecutive words of a row, the cells' own in the middle (values
+// rather than a pointer: the byte windows of an array would be read from
+// private memory).
+struct SwarRow {
+    uint32_t a, b, c;
+};
+PARGO_SWAR_FN SwarRow swar_row(const uint32_t *row) { return SwarRow{row[0], row[1], row[2]}; }
+
+// four consecutive bytes of a row, starting dc bytes (-1, 0, 1) from the
+// cells' word
+PARGO_SWAR_FN uint32_t swar_row_window(const SwarRow &r, int dc)
 {
-    return dc < 0 ? swar_window(row[w], row[w + 1], 3) : (dc == 0 ? row[w + 1] : swar_window(row[w + 1], row[w + 2], 1));
+    return dc < 0 ? swar_window(r.a, r.b, 3) : (dc == 0 ? r.b : swar_window(r.b, r.c, 1));
 }
 
 // Inflow masks of the four cells with classes b: bit j set when the
 // neighbour at window position swar_win_of_bit(j) drains into the cell and
 // the cell does not exclude it; zero for NoData and inert cells.  t0, t1, t2:
-// the targets of the rows above, at and below the cells, their word at w + 1.
-PARGO_SWAR_FN uint32_t swar_inflow_rows(uint32_t b, const uint32_t *t0, const uint32_t *t1, const uint32_t *t2, int w)
+// the targets of the rows above, at and below the cells.
+PARGO_SWAR_FN uint32_t swar_inflow_rows(uint32_t b, const SwarRow &t0, const SwarRow &t1, const SwarRow &t2)
 {
     uint32_t m = 0;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
         const int k = swar_win_of_bit(j), dr = k / 3 - 1, dc = k % 3 - 1;
-        const uint32_t win = swar_row_window(dr < 0 ? t0 : dr == 0 ? t1 : t2, w, dc);
+        const uint32_t win = swar_row_window(dr < 0 ? t0 : dr == 0 ? t1 : t2, dc);
         m |= (swar_small_zero(win ^ swar_splat((uint32_t)(8 - k))) >> (7 - j)) & swar_splat(1u << j);
     }
     // the excluded window position: the class for 0..8, its low nibble for
@@ -94,7 +102,7 @@ PARGO_SWAR_FN uint32_t swar_inflow_rows(uint32_t b, const uint32_t *t0, const ui
 // q + 1).
 PARGO_SWAR_FN uint32_t swar_inflow(const SwarTile &T, int lr, int q)
 {
-    return swar_inflow_rows(T.cls[lr + 1][q + 1], T.tgt[lr], T.tgt[lr + 1], T.tgt[lr + 2], q);
+    return swar_inflow_rows(T.cls[lr + 1][q + 1], swar_row(T.tgt[lr] + q), swar_row(T.tgt[lr + 1] + q), swar_row(T.tgt[lr + 2] + q));
 }
 
 // Four cells: static words (s01: cells 0 and 1, s23: cells 2 and 3, 16 bits
@@ -108,16 +116,16 @@ struct SwarCells {
 };
 
 // Of cells with classes b and targets f; m0, m1, m2: the inflow masks of the
-// rows above, at and below the cells, their word at w + 1.
-PARGO_SWAR_FN SwarCells swar_cells_rows(uint32_t b, uint32_t f, const uint32_t *m0, const uint32_t *m1,
-                                        const uint32_t *m2, int w, bool converge)
+// rows above, at and below the cells.
+PARGO_SWAR_FN SwarCells swar_cells_rows(uint32_t b, uint32_t f, const SwarRow &m0, const SwarRow &m1, const SwarRow &m2,
+                                        bool converge)
 {
-    const uint32_t mine = m1[w + 1];
+    const uint32_t mine = m1.b;
     uint32_t srcn = 0, feeds = 0;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
         const int k = swar_win_of_bit(j), dr = k / 3 - 1, dc = k % 3 - 1;
-        const uint32_t win = swar_row_window(dr < 0 ? m0 : dr == 0 ? m1 : m2, w, dc);
+        const uint32_t win = swar_row_window(dr < 0 ? m0 : dr == 0 ? m1 : m2, dc);
         srcn |= swar_zero(win) >> (7 - j);
         // a cell draining to window k feeds when its target's inflow mask
         // has it (bit swar_bit_of_win(8 - k) of that mask), and then only in
@@ -149,7 +157,8 @@ PARGO_SWAR_FN SwarCells swar_cells_rows(uint32_t b, uint32_t f, const uint32_t *
 // The same for the cells of tile row tr, columns c0 + 4g ..
 PARGO_SWAR_FN SwarCells swar_cells(const SwarTile &T, int tr, int g, bool converge)
 {
-    return swar_cells_rows(T.cls[tr + 2][g + 2], T.tgt[tr + 2][g + 2], T.inm[tr], T.inm[tr + 1], T.inm[tr + 2], g, converge);
+    return swar_cells_rows(T.cls[tr + 2][g + 2], T.tgt[tr + 2][g + 2], swar_row(T.inm[tr] + g), swar_row(T.inm[tr + 1] + g),
+                           swar_row(T.inm[tr + 2] + g), converge);
 }
 
 }  // namespace pargo

@@ -54,7 +54,13 @@ PARGO_SWAR_FN uint32_t swar_select(uint32_t mask, uint32_t a, uint32_t b) { retu
 // (lo, hi): what __builtin_amdgcn_alignbyte(hi, lo, s) returns
 PARGO_SWAR_FN uint32_t swar_window(uint32_t lo, uint32_t hi, unsigned s)
 {
+#if defined(__HIP_DEVICE_COMPILE__)
+    // the builtin, or the compiler takes the shift of two adjacent words for
+    // an unaligned read of the memory they came from and keeps them there
+    return __builtin_amdgcn_alignbyte(hi, lo, s);
+#else
     return s == 0 ? lo : (uint32_t)((((uint64_t)hi << 32) | lo) >> (8u * s));
+#endif
 }
 
 }  // namespace pargo
