@@ -605,27 +605,35 @@ __global__ __launch_bounds__(256) void sca_final_kernel(ScaParams p)
     const int r0 = ty * kTileR, c0 = tx * kTileC;
     const uint4 words = *reinterpret_cast<const uint4 *>(p.st + (long long)tile * kTileN + 8 * tid);
     const int pcell = tid < kSlots ? cell_of_slot(tid) : 0;
-    // what arrives at this thread's perimeter cell from outside: every load
-    // is issued before the first word is looked at (the slots that are not
-    // inflows read the tile's own first word)
+    // What arrives at this thread's perimeter cell from outside.  The words
+    // of its first three inflows are all requested before one is looked at;
+    // more than three drain only into a few corners.
     const unsigned long long slot0 = (unsigned long long)tile * kSlotStride;
     const unsigned ext = tid < kSlots ? p.ext[slot0 + tid] : 0u;
     const unsigned pword = tid < kSlots ? p.st[(long long)tile * kTileN + pcell] : 0u;
     unsigned long long arrived = 0;
     if (ext) {
-        unsigned long long x[8];
+        auto word = [&](unsigned e) -> unsigned long long {  // of the lowest inflow in e
+            const unsigned k = (unsigned)win_of_bit(__builtin_ctz(e));
+            const unsigned gr = (unsigned)(r0 + (pcell >> 6) - 1) + k / 3u, gc = (unsigned)(c0 + (pcell & 63) - 1) + k % 3u;
+            return p.exits[(unsigned long long)((gr / kTileR) * (unsigned)p.tiles_x + gc / kTileC) * kSlotStride +
+                           (unsigned)slot_of((int)(gr % kTileR), (int)(gc % kTileC))];
+        };
+        auto arrival = [&](unsigned long long x) -> unsigned long long {
+            if (((x >> kExitPend) & 255ull) != 0) return 0;  // never complete
+            return ((x >> kExitBad) & 255ull ? 1ull << kFinBad : x & kFinSum) - (1ull << kFinPend);
+        };
+        unsigned e = ext;
+        unsigned long long x[3];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int k = win_of_bit(j), gr = r0 + (pcell >> 6) + k / 3 - 1, gc = c0 + (pcell & 63) + k % 3 - 1;
-            const unsigned long long u = (unsigned long long)((gr / kTileR) * p.tiles_x + gc / kTileC) * kSlotStride +
-                                         (unsigned)slot_of(gr % kTileR, gc % kTileC);
-            x[j] = p.exits[(ext >> j) & 1u ? u : slot0];
+        for (int q = 0; q < 3; q++) {
+            x[q] = kExitNever;
+            if (e) x[q] = word(e);
+            e &= e - 1;
         }
+        for (; e; e &= e - 1) arrived += arrival(word(e));
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            if (!((ext >> j) & 1u) || ((x[j] >> kExitPend) & 255ull) != 0) continue;  // no inflow, or never complete
-            arrived += ((x[j] >> kExitBad) & 255ull ? 1ull << kFinBad : x[j] & kFinSum) - (1ull << kFinPend);
-        }
+        for (int q = 0; q < 3; q++) arrived += arrival(x[q]);
     }
     *reinterpret_cast<uint4 *>(nxt + 8 * tid) = words;
     __syncthreads();
