@@ -15,6 +15,7 @@
 // Work split as in focal.hip: a lane owns 4 adjacent columns and walks a
 // strip of rows; it computes p for its columns plus one halo column on each
 // side (so it needs z two columns out), which keeps every wave independent.
+#include <algorithm>
 #include <cmath>
 
 #include "focal_common.h"
@@ -266,6 +267,21 @@ __global__ __launch_bounds__(256) void slope_adjoint_kernel(AdjParams p)
     }
 }
 
+// Rows per strip.  A wave's rows are a serial chain (about 1.1 us each) and a
+// strip evaluates the per-cell terms of two halo rows again, twice the halo
+// of the forward kernels: up to 32,768 wave-rows (2048 x 4096 cells) the
+// strip that gives 2048 waves, above it one of 16 to 32 rows that gives 8192.
+// Measured with 32 rows before: 256^2 38.2 -> 6.2 us (1 row), 1024^2 34.4 ->
+// 8.6 (2), 1501 x 2003 42.5 -> 16.3 (6), 2048^2 36.2 -> 17.4 (8), 4096^2
+// 55.2 -> 49.0 (16), 7001 x 5003 126.7 -> 113.5 (17); 8192^2 keeps 32 (172,
+// 185 at 16 rows).
+int adjoint_strip_rows(int rows, int cols)
+{
+    const long long work = (long long)rows * ((cols + 64 * ACPT - 1) / (64 * ACPT));
+    if (work <= 32768) return (int)std::max(1ll, (work + 2047) / 2048);
+    return (int)std::min(32ll, std::max(16ll, (work + 4096) / 8192));
+}
+
 }  // namespace
 
 }  // namespace pargo
@@ -293,7 +309,7 @@ extern "C" int pargo_slope_adjoint(pargo_ctx *ctx, const pargo_grid *g, const fl
     p.pitch = pitch;
     p.rows = g->rows;
     p.cols = g->cols;
-    p.rows_per_strip = 32;
+    p.rows_per_strip = pargo::adjoint_strip_rows(g->rows, g->cols);
     pargo::nodata_interval(g->nodata, 0.0000001, &p.nd_lo, &p.nd_hi);
     if (p.nd_lo > p.nd_hi) {
         p.nd_lo = INFINITY;

@@ -766,6 +766,7 @@ __device__ __forceinline__ void focal_raster(const FocalParams &p)
     unsigned cb = blockIdx.x, strip = blockIdx.y;
     if (MASK) xcd_strip_order(cb, strip);
     const int wave_c0 = (int)(cb * 4 + wave) * 64 * CPT;
+    if (wave_c0 >= p.cols) return;  // a wave past the right edge
     const int rbeg = (int)strip * p.rows_per_strip;
     const int rend = min(rbeg + p.rows_per_strip, p.rows);
     focal_strip<CPT, VEC, DO_SLOPE, DO_D8, SM, MASK>(p, wave_c0, lane, rbeg, rend);
@@ -998,21 +999,21 @@ static void launch_focal(const FocalParams &p, const LaunchCfg &cfg, bool vec, b
     launch_focal_h(p, cfg, vec, do_slope, do_d8, slope_mode(p), s);
 }
 
-static LaunchCfg default_cfg(int rows)
+static LaunchCfg default_cfg(int rows, int cols)
 {
     LaunchCfg c;
-    // 4 columns per lane and 16-row strips measured best for the fused
-    // kernel on 16384^2 (MI355X, 4 waves per SIMD): 0.495 ms against 0.500
-    // at 32 rows, 0.504 at 12, 0.52-0.58 at 48-128 rows (fewer, longer work
-    // items leave a ragged tail); the extra halo rows cost less than that.
+    // 4 columns per lane, and at most 16-row strips, which measured best for
+    // the fused kernel on 16384^2 (MI355X, 4 waves per SIMD): 0.495 ms
+    // against 0.500 at 32 rows, 0.504 at 12, 0.52-0.58 at 48-128 rows (fewer,
+    // longer work items leave a ragged tail); the extra halo rows cost less
+    // than that.
     c.cpt = 4;
-    c.rows_per_strip = 16;
+    c.rows_per_strip = strip_rows(rows, cols, 64 * c.cpt, 16);
     if (const char *e = getenv("PARGO_FOCAL_CPT")) c.cpt = atoi(e) == 2 ? 2 : 4;
     if (const char *e = getenv("PARGO_FOCAL_ROWS")) {
         int v = atoi(e);
         if (v >= 1 && v <= 4096) c.rows_per_strip = v;
     }
-    (void)rows;
     return c;
 }
 
@@ -1148,7 +1149,7 @@ static int run_focal(pargo_ctx *ctx, const pargo_grid *g, const float *dem, int 
     if (!slope_out && !code_out && !mask_out) return PARGO_OK;
     rc = bind(ctx);
     if (rc) return rc;
-    LaunchCfg cfg = default_cfg(g->rows);
+    LaunchCfg cfg = default_cfg(g->rows, g->cols);
     p.rows_per_strip = cfg.rows_per_strip;
     const bool do_slope = slope_out != nullptr;
     const bool do_d8 = code_out != nullptr;

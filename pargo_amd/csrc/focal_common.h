@@ -63,4 +63,26 @@ __device__ __forceinline__ void xcd_strip_order(unsigned &cb, unsigned &strip)
     strip = w / gx;
 }
 
+// Rows per strip of a kernel whose waves walk strips of `width` columns, for
+// a raster of rows x cols: a wave's rows are a serial chain (about 1 us each),
+// so a small raster takes the strip that still gives every SIMD four waves
+// (4096 waves on 256 CUs), down to single rows, and a larger one the strip
+// that gives about five rounds of them, up to `most`; the two halo rows a
+// strip reads again come from the caches.  Measured with strips of 16 rows
+// before, us for slope / slope + D8 / slope + D8 with the mask:
+//   256 x 256     16.4 / 22.7 / 27.6   now  3.6 /  4.7 /  4.5  (1 row)
+//   1024 x 1024   16.5 / 23.3 / 28.6        5.7 /  7.4 /  8.0  (1 row)
+//   1501 x 2003   17.5 / 25.4 / 30.4        9.5 / 13.2 / 15.5  (3 rows)
+//   4096 x 4096   30.4 / 41.9 / 58.8       28.5 / 40.2 / 52.1  (4 rows)
+//   7001 x 5003   58.0 / 76.4 / 102.9      52.6 / 71.6 / 97.1  (7 rows)
+// At 16384^2 the longest strips stay the fastest (1 row doubles the time).
+inline int strip_rows(int rows, int cols, int width, int most)
+{
+    constexpr long long kWaves = 4096;
+    const long long work = (long long)rows * ((cols + width - 1) / width);
+    const long long n = work <= 4 * kWaves ? (work + kWaves - 1) / kWaves : (work + 5 * kWaves / 2) / (5 * kWaves);
+    const long long least = work <= 4 * kWaves ? 1 : 4;
+    return (int)(n < least ? least : n > most ? most : n);
+}
+
 }  // namespace pargo
