@@ -34,6 +34,7 @@
 #include <cmath>
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "focal_common.h"
@@ -69,6 +70,25 @@ constexpr Lut8Init make_lut8()
 }  // namespace
 
 __constant__ Lut8Init c_lut8 = make_lut8();
+
+// ESRI bit of a window index (not the centre).
+__device__ __forceinline__ unsigned bit_of_win8(unsigned w)
+{
+    // E=5 SE=8 S=7 SW=6 W=3 NW=0 N=1 NE=2: exponents 5 6 7 4 - 0 3 2 1, four bits each
+    return 1u << ((0x123004765ull >> (4u * w)) & 15u);
+}
+// dirType 8 from codes of one ESRI bit or none: the bit's number (all ones
+// for no bit), then the window indices of four of them by one byte lookup
+// (255 for a selector above 12, so for no bit).  A table in memory, one
+// gather per cell and row, made every row wait for all its prefetched rows:
+// at 16384^2 D8 with the mask 517 -> 412 us, slope + D8 631 -> 520.
+__device__ __forceinline__ unsigned first_bit(unsigned c)
+{
+    unsigned n;
+    asm("v_ffbl_b32 %0, %1" : "=v"(n) : "v"(c));
+    return n;
+}
+__device__ __forceinline__ unsigned wins_of_bits(unsigned n) { return __builtin_amdgcn_perm(0x02010003u, 0x06070805u, n); }
 
 struct FocalParams {
     const float *__restrict__ dem;
@@ -456,7 +476,7 @@ __device__ __forceinline__ float slope_unit(float s, int unit)
 // `special` is set when a window of this lane holds a value the fast path
 // does not handle.  MASK false compiles the NoData mask output out (p.mask
 // is then ignored); MASK true writes it when p.mask is set.
-template <int CPT, bool VECLOAD, bool DO_SLOPE, bool DO_D8, int SM, bool MASK>
+template <int CPT, bool VECLOAD, bool DO_SLOPE, int DO_D8, int SM, bool MASK>
 __device__ __forceinline__ void focal_step(const FocalParams &p, int r, int rlast, int c0, int lane, unsigned colb,
                                            Slot<CPT> &up, Slot<CPT> &mid, Slot<CPT> &dn, RawRow<CPT> &raw,
                                            bool &special)
@@ -596,6 +616,8 @@ __device__ __forceinline__ void focal_step(const FocalParams &p, int r, int rlas
                 const unsigned c64 = d8_window_fp64(up.zf[i - 1], up.zf[i], up.zf[i + 1], mid.zf[i - 1], mid.zf[i],
                                                     mid.zf[i + 1], dn.zf[i - 1], dn.zf[i], dn.zf[i + 1]);
                 if (amb) cd[j] = c64;
+                // dirType 8: a tie becomes the bit of its median direction
+                if (DO_D8 == 8 && (cd[j] & (cd[j] - 1u))) cd[j] = bit_of_win8(c_lut8.v[cd[j]]);
             }
         }
     }
@@ -614,9 +636,10 @@ __device__ __forceinline__ void focal_step(const FocalParams &p, int r, int rlas
             ndbits |= (unsigned)(m && (c0 + j) < p.cols) << j;
         }
     }
-    if (DO_D8 && p.dirtype == 8) {
+    if (DO_D8 == 8) {
+        // every code is one bit or none by now; the lookup is in the stores
 #pragma unroll
-        for (int j = 0; j < CPT; j++) cd[j] = cd[j] ? (unsigned)c_lut8.v[cd[j]] : 255u;
+        for (int j = 0; j < CPT; j++) cd[j] = first_bit(cd[j]);
     }
 
     // ---- stores --------------------------------------------------------------
@@ -648,21 +671,23 @@ __device__ __forceinline__ void focal_step(const FocalParams &p, int r, int rlas
         uint8_t *crow = p.code + rbase;
         if constexpr (VECLOAD) {
             if constexpr (CPT == 4) {
-                const unsigned packed = __builtin_amdgcn_perm(
+                unsigned packed = __builtin_amdgcn_perm(
                     __builtin_amdgcn_perm(cd[3], cd[2], 0x0c0c0400u), __builtin_amdgcn_perm(cd[1], cd[0], 0x0c0c0400u),
                     0x05040100u);  // byte 0 of each code, three byte permutes
+                if (DO_D8 == 8) packed = wins_of_bits(packed);
                 __builtin_nontemporal_store(packed, reinterpret_cast<u32_b1 *>(crow + uc0));
             } else if constexpr (CPT == 2) {
-                __builtin_nontemporal_store((unsigned short)(cd[0] | (cd[1] << 8)),
-                                            reinterpret_cast<u16_b1 *>(crow + uc0));
+                unsigned packed = __builtin_amdgcn_perm(cd[1], cd[0], 0x0c0c0400u);
+                if (DO_D8 == 8) packed = wins_of_bits(packed);
+                __builtin_nontemporal_store((unsigned short)packed, reinterpret_cast<u16_b1 *>(crow + uc0));
             } else {
 #pragma unroll
-                for (int j = 0; j < CPT; j++) crow[uc0 + j] = (uint8_t)cd[j];
+                for (int j = 0; j < CPT; j++) crow[uc0 + j] = (uint8_t)(DO_D8 == 8 ? wins_of_bits(cd[j]) : cd[j]);
             }
         } else {
 #pragma unroll
             for (int j = 0; j < CPT; j++)
-                if (c0 + j < p.cols) crow[uc0 + j] = (uint8_t)cd[j];
+                if (c0 + j < p.cols) crow[uc0 + j] = (uint8_t)(DO_D8 == 8 ? wins_of_bits(cd[j]) : cd[j]);
         }
     }
     if (MASK && p.mask) {
@@ -685,7 +710,7 @@ __device__ __forceinline__ void focal_step(const FocalParams &p, int r, int rlas
 }
 
 // Pairs from a row to the row below (the prologue of a strip).
-template <int CPT, bool DO_SLOPE, bool DO_D8, int SM>
+template <int CPT, bool DO_SLOPE, int DO_D8, int SM>
 __device__ __forceinline__ void pair_rows(Slot<CPT> &up, const Slot<CPT> &below)
 {
     if (DO_D8) {
@@ -700,7 +725,7 @@ __device__ __forceinline__ void pair_rows(Slot<CPT> &up, const Slot<CPT> &below)
 
 // One wave computes output rows [rbeg, rend) of the 64*CPT columns that
 // start at wave_c0 (wave-uniform).
-template <int CPT, bool VECLOAD, bool DO_SLOPE, bool DO_D8, int SM, bool MASK>
+template <int CPT, bool VECLOAD, bool DO_SLOPE, int DO_D8, int SM, bool MASK>
 __device__ __forceinline__ void focal_strip_impl(const FocalParams &p, int wave_c0, int lane, int rbeg, int rend)
 {
     const int c0 = wave_c0 + lane * CPT;
@@ -739,7 +764,7 @@ __device__ __forceinline__ void focal_strip_impl(const FocalParams &p, int wave_
 
 // VEC: the raster's pitch and base allow vector access; a wave uses it when
 // all its columns are inside the raster.
-template <int CPT, bool VEC, bool DO_SLOPE, bool DO_D8, int SM, bool MASK = true>
+template <int CPT, bool VEC, bool DO_SLOPE, int DO_D8, int SM, bool MASK = true>
 __device__ __forceinline__ void focal_strip(const FocalParams &p, int wave_c0, int lane, int rbeg, int rend)
 {
     if constexpr (VEC) {
@@ -752,7 +777,7 @@ __device__ __forceinline__ void focal_strip(const FocalParams &p, int wave_c0, i
 }
 
 // One raster: block = 4 waves side by side, one row strip per block.
-template <int CPT, bool VEC, bool DO_SLOPE, bool DO_D8, int SM, bool MASK = true>
+template <int CPT, bool VEC, bool DO_SLOPE, int DO_D8, int SM, bool MASK = true>
 __device__ __forceinline__ void focal_raster(const FocalParams &p)
 {
     const int lane = threadIdx.x & 63;
@@ -772,30 +797,31 @@ __device__ __forceinline__ void focal_raster(const FocalParams &p)
     focal_strip<CPT, VEC, DO_SLOPE, DO_D8, SM, MASK>(p, wave_c0, lane, rbeg, rend);
 }
 
-template <int CPT, bool VEC, bool DO_SLOPE, bool DO_D8, int SM>
+template <int CPT, bool VEC, bool DO_SLOPE, int DO_D8, int SM>
 __global__ __launch_bounds__(256) void focal_kernel(FocalParams p)
 {
     focal_raster<CPT, VEC, DO_SLOPE, DO_D8, SM>(p);
 }
 
-// The fused Horn slope + D8 pass without a NoData mask, at four waves per
-// SIMD (at most 128 VGPRs, a few spilled to scratch): it ran faster than at
+// The fused slope + D8 passes without a NoData mask, at four waves per SIMD
+// (at most 128 VGPRs, a few spilled to scratch): they ran faster than at
 // three waves without spills, since the pass issues VALU work most of the
-// time and a fourth wave fills the dependency stalls.  That balance is
-// fragile: any extra state in the loop (the mask's, for one) brings spill
-// reloads into it, and each reload waits for every load in flight.  The
-// variant that writes the mask therefore runs at three waves, like the
-// other kernels.
-template <int CPT, bool VEC>
+// time and a fourth wave fills the dependency stalls (16384^2: Horn 509
+// against 575 us, TFDW 618 against 709).  That balance is fragile: any extra
+// state in the loop (the mask's, for one, or a dirType known only at run
+// time) brings spill reloads into it, and each reload waits for every load
+// in flight.  The variants that write the mask therefore run at three waves
+// (Horn 578 against 606 us, TFDW 737 against 760).
+template <int CPT, bool VEC, int D8, int SM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void focal_kernel_fused(FocalParams p)
 {
-    focal_raster<CPT, VEC, true, true, 1, false>(p);
+    focal_raster<CPT, VEC, true, D8, SM, false>(p);
 }
 
-template <int CPT, bool VEC>
+template <int CPT, bool VEC, int D8, int SM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void focal_kernel_fused_mask(FocalParams p)
 {
-    focal_raster<CPT, VEC, true, true, 1, true>(p);
+    focal_raster<CPT, VEC, true, D8, SM, true>(p);
 }
 
 // Many rasters in one persistent launch: every wave takes (tile, column
@@ -803,7 +829,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // numbered tile by tile (first[t] = first item of tile t; tiles are in
 // decreasing size so that the tail of the queue holds the small items).
 // Batch tiles carry no NoData mask, so the mask code is compiled out.
-template <int CPT, bool DO_SLOPE, bool DO_D8, int SM>
+template <int CPT, bool DO_SLOPE, int DO_D8, int SM>
 __device__ __forceinline__ void focal_batch_body(const FocalParams *__restrict__ tiles,
                                                  const unsigned *__restrict__ first, int ntiles,
                                                  unsigned *__restrict__ queue, unsigned total)
@@ -838,7 +864,7 @@ __device__ __forceinline__ void focal_batch_body(const FocalParams *__restrict__
     }
 }
 
-template <int CPT, bool DO_SLOPE, bool DO_D8, int SM>
+template <int CPT, bool DO_SLOPE, int DO_D8, int SM>
 __global__ __launch_bounds__(256) void focal_batch_kernel(const FocalParams *__restrict__ tiles,
                                                           const unsigned *__restrict__ first, int ntiles,
                                                           unsigned *__restrict__ queue, unsigned total)
@@ -848,11 +874,12 @@ __global__ __launch_bounds__(256) void focal_batch_kernel(const FocalParams *__r
 
 // The fused Horn slope + D8 batch at 4 columns per lane runs at four waves
 // per SIMD, like the single-raster fused kernel.
+template <int D8>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void focal_batch_kernel_fused(
     const FocalParams *__restrict__ tiles, const unsigned *__restrict__ first, int ntiles,
     unsigned *__restrict__ queue, unsigned total)
 {
-    focal_batch_body<4, true, true, true>(tiles, first, ntiles, queue, total);
+    focal_batch_body<4, true, D8, 1>(tiles, first, ntiles, queue, total);
 }
 
 // Zeroes the batch queue head (a kernel rather than a memset, so that the
@@ -930,7 +957,7 @@ struct LaunchCfg {
     int rows_per_strip;
 };
 
-template <bool DO_SLOPE, bool DO_D8, int SM>
+template <bool DO_SLOPE, int DO_D8, int SM>
 static void launch_t(const FocalParams &p, const LaunchCfg &cfg, bool vec, hipStream_t s)
 {
     const int threads = 256;
@@ -938,13 +965,13 @@ static void launch_t(const FocalParams &p, const LaunchCfg &cfg, bool vec, hipSt
     const int cols_per_block = threads * cfg.cpt;
     dim3 grid((p.cols + cols_per_block - 1) / cols_per_block, (p.rows + cfg.rows_per_strip - 1) / cfg.rows_per_strip);
     if (cfg.cpt == 4) {
-        if constexpr (DO_SLOPE && DO_D8 && SM == 1) {
+        if constexpr (DO_SLOPE && DO_D8 && SM != 0) {
             if (p.mask) {
-                if (vec) hipLaunchKernelGGL((focal_kernel_fused_mask<4, true>), grid, block, 0, s, p);
-                else hipLaunchKernelGGL((focal_kernel_fused_mask<4, false>), grid, block, 0, s, p);
+                if (vec) hipLaunchKernelGGL((focal_kernel_fused_mask<4, true, DO_D8, SM>), grid, block, 0, s, p);
+                else hipLaunchKernelGGL((focal_kernel_fused_mask<4, false, DO_D8, SM>), grid, block, 0, s, p);
             } else {
-                if (vec) hipLaunchKernelGGL((focal_kernel_fused<4, true>), grid, block, 0, s, p);
-                else hipLaunchKernelGGL((focal_kernel_fused<4, false>), grid, block, 0, s, p);
+                if (vec) hipLaunchKernelGGL((focal_kernel_fused<4, true, DO_D8, SM>), grid, block, 0, s, p);
+                else hipLaunchKernelGGL((focal_kernel_fused<4, false, DO_D8, SM>), grid, block, 0, s, p);
             }
         } else {
             if (vec) hipLaunchKernelGGL((focal_kernel<4, true, DO_SLOPE, DO_D8, SM>), grid, block, 0, s, p);
@@ -977,20 +1004,24 @@ static int slope_mode(const FocalParams &p)
     return p.method == PARGO_SLOPE_FD ? 1 : 2;
 }
 
+template <int DO_D8>
+static void launch_focal_d(const FocalParams &p, const LaunchCfg &cfg, bool vec, bool do_slope, int sm, hipStream_t s)
+{
+    if (do_slope) {
+        if (sm == 1) launch_t<true, DO_D8, 1>(p, cfg, vec, s);
+        else if (sm == 2) launch_t<true, DO_D8, 2>(p, cfg, vec, s);
+        else launch_t<true, DO_D8, 0>(p, cfg, vec, s);
+    } else if constexpr (DO_D8 != 0) {
+        launch_t<false, DO_D8, 1>(p, cfg, vec, s);
+    }
+}
+
 static void launch_focal_h(const FocalParams &p, const LaunchCfg &cfg, bool vec, bool do_slope, bool do_d8,
                            int sm, hipStream_t s)
 {
-    if (do_slope && do_d8) {
-        if (sm == 1) launch_t<true, true, 1>(p, cfg, vec, s);
-        else if (sm == 2) launch_t<true, true, 2>(p, cfg, vec, s);
-        else launch_t<true, true, 0>(p, cfg, vec, s);
-    } else if (do_slope) {
-        if (sm == 1) launch_t<true, false, 1>(p, cfg, vec, s);
-        else if (sm == 2) launch_t<true, false, 2>(p, cfg, vec, s);
-        else launch_t<true, false, 0>(p, cfg, vec, s);
-    } else {
-        launch_t<false, true, 1>(p, cfg, vec, s);
-    }
+    if (do_d8 && p.dirtype == 8) launch_focal_d<8>(p, cfg, vec, do_slope, sm, s);
+    else if (do_d8) launch_focal_d<256>(p, cfg, vec, do_slope, sm, s);
+    else launch_focal_d<0>(p, cfg, vec, true, sm, s);
 }
 
 static void launch_focal(const FocalParams &p, const LaunchCfg &cfg, bool vec, bool do_slope, bool do_d8,
@@ -1203,13 +1234,13 @@ void free_batch_plan(pargo_ctx *ctx)
     ctx->batch = nullptr;
 }
 
-template <int CPT, bool DO_SLOPE, bool DO_D8, int SM>
+template <int CPT, bool DO_SLOPE, int DO_D8, int SM>
 static int batch_blocks(pargo_ctx *ctx)
 {
     int per_cu = 0;
     hipError_t e;
-    if constexpr (CPT == 4 && DO_SLOPE && DO_D8 && SM == 1)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, focal_batch_kernel_fused, 256, 0);
+    if constexpr (CPT == 4 && DO_SLOPE && DO_D8 != 0 && SM == 1)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, focal_batch_kernel_fused<DO_D8>, 256, 0);
     else
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, focal_batch_kernel<CPT, DO_SLOPE, DO_D8, SM>, 256, 0);
     if (e != hipSuccess || per_cu < 1) per_cu = 2;
@@ -1217,45 +1248,48 @@ static int batch_blocks(pargo_ctx *ctx)
     return per_cu * cus;
 }
 
-template <int CPT, bool DO_SLOPE, bool DO_D8, int SM>
+template <int CPT, bool DO_SLOPE, int DO_D8, int SM>
 static void launch_batch_t(const BatchPlan &b, hipStream_t s)
 {
-    if constexpr (CPT == 4 && DO_SLOPE && DO_D8 && SM == 1)
-        hipLaunchKernelGGL(focal_batch_kernel_fused, dim3(b.blocks), dim3(256), 0, s, (const FocalParams *)b.d_tiles,
+    if constexpr (CPT == 4 && DO_SLOPE && DO_D8 != 0 && SM == 1)
+        hipLaunchKernelGGL((focal_batch_kernel_fused<DO_D8>), dim3(b.blocks), dim3(256), 0, s, (const FocalParams *)b.d_tiles,
                            (const unsigned *)b.d_first, b.ntiles, b.d_queue, b.total);
     else
         hipLaunchKernelGGL((focal_batch_kernel<CPT, DO_SLOPE, DO_D8, SM>), dim3(b.blocks), dim3(256), 0, s,
                            (const FocalParams *)b.d_tiles, (const unsigned *)b.d_first, b.ntiles, b.d_queue, b.total);
 }
 
+// Calls f with the batch's kernel shape: D8 output (0, 8 or 256) and slope mode.
+template <int CPT, typename F>
+static auto with_batch_shape(const BatchPlan &b, F f)
+{
+    const int d8 = b.do_d8 ? b.h_tiles[0].dirtype : 0;
+    auto mode = [&](auto d) {
+        constexpr int D = decltype(d)::value;
+        if (!b.do_slope) return f(std::false_type{}, std::integral_constant<int, D ? D : 256>{}, std::integral_constant<int, 1>{});
+        if (b.sm == 1) return f(std::true_type{}, d, std::integral_constant<int, 1>{});
+        if (b.sm == 2) return f(std::true_type{}, d, std::integral_constant<int, 2>{});
+        return f(std::true_type{}, d, std::integral_constant<int, 0>{});
+    };
+    if (d8 == 8) return mode(std::integral_constant<int, 8>{});
+    if (d8) return mode(std::integral_constant<int, 256>{});
+    return mode(std::integral_constant<int, 0>{});
+}
+
 template <int CPT>
 static void launch_batch_c(const BatchPlan &b, hipStream_t s)
 {
-    if (b.do_slope && b.do_d8) {
-        if (b.sm == 1) launch_batch_t<CPT, true, true, 1>(b, s);
-        else if (b.sm == 2) launch_batch_t<CPT, true, true, 2>(b, s);
-        else launch_batch_t<CPT, true, true, 0>(b, s);
-    } else if (b.do_slope) {
-        if (b.sm == 1) launch_batch_t<CPT, true, false, 1>(b, s);
-        else if (b.sm == 2) launch_batch_t<CPT, true, false, 2>(b, s);
-        else launch_batch_t<CPT, true, false, 0>(b, s);
-    } else {
-        launch_batch_t<CPT, false, true, 1>(b, s);
-    }
+    with_batch_shape<CPT>(b, [&](auto slope, auto d8, auto sm) {
+        launch_batch_t<CPT, decltype(slope)::value, decltype(d8)::value, decltype(sm)::value>(b, s);
+    });
 }
 
 template <int CPT>
 static int blocks_c(pargo_ctx *ctx, const BatchPlan &b)
 {
-    if (b.do_slope && b.do_d8)
-        return b.sm == 1   ? batch_blocks<CPT, true, true, 1>(ctx)
-               : b.sm == 2 ? batch_blocks<CPT, true, true, 2>(ctx)
-                           : batch_blocks<CPT, true, true, 0>(ctx);
-    if (b.do_slope)
-        return b.sm == 1   ? batch_blocks<CPT, true, false, 1>(ctx)
-               : b.sm == 2 ? batch_blocks<CPT, true, false, 2>(ctx)
-                           : batch_blocks<CPT, true, false, 0>(ctx);
-    return batch_blocks<CPT, false, true, 1>(ctx);
+    return with_batch_shape<CPT>(b, [&](auto slope, auto d8, auto sm) {
+        return batch_blocks<CPT, decltype(slope)::value, decltype(d8)::value, decltype(sm)::value>(ctx);
+    });
 }
 
 // The persistent sequence: queue reset, batch kernel, fixup.
