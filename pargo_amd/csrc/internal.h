@@ -38,7 +38,7 @@ struct pargo_ctx {
     // launch shape chosen by pargo_batch_autotune
     pargo::BatchPlan *batch = nullptr;
     int batch_cpt = 4;
-    int batch_rows = 32;
+    int batch_rows = 32;  // once batch_tuned; by the batch's size before
     int batch_tuned = 0;
     // queue order of batch tiles: PARGO_ORDER_ESTIMATE (cells), _ROWS (as
     // given) or _MEASURED (batch_load, per-tile kernel times of one pass)
