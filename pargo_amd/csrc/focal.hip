@@ -895,18 +895,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     focal_batch_body<4, true, D8, 1>(tiles, first, ntiles, queue, total);
 }
 
-// Zeroes the batch queue head (a kernel rather than a memset, so that the
-// sequence can be captured in a HIP graph and replayed).
-__global__ void focal_queue_reset(unsigned *queue) { queue[0] = 0; }
-
 // Recomputes, with the reference-order FP64 code, every window holding Inf
 // or |z| >= 2^40 in the queued strips (width: columns per strip).  If the
 // queue overflowed it scans every raster instead.  The last block to finish
-// resets the queue for the next call on the stream.  `tiles` is NULL for a
-// single raster (then `one` describes it).
+// resets the queue for the next call on the stream, and the batch's item
+// queue if there is one (a launch less than a kernel of its own for it; no
+// memset, so that the sequence can be captured in a HIP graph and replayed).
+// `tiles` is NULL for a single raster (then `one` describes it).
 template <bool DO_SLOPE, bool DO_D8>
 __global__ __launch_bounds__(256) void focal_fixup_kernel(FocalParams one, const FocalParams *__restrict__ tiles,
-                                                          int ntiles, int width)
+                                                          int ntiles, int width, unsigned *items)
 {
     const unsigned *cnt = one.fix_count;
     const unsigned n = __atomic_load_n(&cnt[0], __ATOMIC_RELAXED);
@@ -954,6 +952,7 @@ __global__ __launch_bounds__(256) void focal_fixup_kernel(FocalParams one, const
         if (done == gridDim.x - 1) {
             c[0] = 0;
             c[1] = 0;
+            if (items) items[0] = 0;
             __threadfence();
         }
     }
@@ -997,13 +996,13 @@ static void launch_t(const FocalParams &p, const LaunchCfg &cfg, bool vec, hipSt
 }
 
 static void launch_fixup(const FocalParams &p, const FocalParams *tiles, int ntiles, bool do_slope, bool do_d8,
-                         int cpt, hipStream_t s)
+                         int cpt, hipStream_t s, unsigned *items = nullptr)
 {
     dim3 block(256), grid(kFixupBlocks);
     const int width = 64 * cpt;
-    if (do_slope && do_d8) hipLaunchKernelGGL((focal_fixup_kernel<true, true>), grid, block, 0, s, p, tiles, ntiles, width);
-    else if (do_slope) hipLaunchKernelGGL((focal_fixup_kernel<true, false>), grid, block, 0, s, p, tiles, ntiles, width);
-    else hipLaunchKernelGGL((focal_fixup_kernel<false, true>), grid, block, 0, s, p, tiles, ntiles, width);
+    if (do_slope && do_d8) hipLaunchKernelGGL((focal_fixup_kernel<true, true>), grid, block, 0, s, p, tiles, ntiles, width, items);
+    else if (do_slope) hipLaunchKernelGGL((focal_fixup_kernel<true, false>), grid, block, 0, s, p, tiles, ntiles, width, items);
+    else hipLaunchKernelGGL((focal_fixup_kernel<false, true>), grid, block, 0, s, p, tiles, ntiles, width, items);
 }
 
 // Slope mode of the kernels: 1 the Horn fast path (FD), 2 the other
@@ -1116,7 +1115,8 @@ __global__ void fixup_counters_reset(unsigned *c)
 
 // Validates the request and fills the kernel parameters.
 static int prepare(pargo_ctx *ctx, const pargo_grid *g, const float *dem, int method, int unit, int dirtype,
-                   float *slope_out, uint8_t *code_out, uint32_t *mask_out, FocalParams &p, bool &vec)
+                   float *slope_out, uint8_t *code_out, uint32_t *mask_out, FocalParams &p, bool &vec,
+                   const pargo_grid *last = nullptr, const FocalParams *like = nullptr)
 {
     if (!ctx) return PARGO_E_INVALID;
     if (!g || !dem) return fail(ctx, PARGO_E_INVALID, "null grid or DEM pointer");
@@ -1143,8 +1143,16 @@ static int prepare(pargo_ctx *ctx, const pargo_grid *g, const float *dem, int me
     p.rows = g->rows;
     p.cols = g->cols;
     p.mask_words = (g->cols + 31) / 32;
-    nodata_interval(g->nodata, 0.0000001, &p.nd_lo, &p.nd_hi);
-    nodata_interval(g->nodata, 0.000001, &p.nd8_lo, &p.nd8_hi);
+    if (last && last->nodata == g->nodata) {
+        // the NoData intervals of the batch's previous raster
+        p.nd_lo = like->nd_lo;
+        p.nd_hi = like->nd_hi;
+        p.nd8_lo = like->nd8_lo;
+        p.nd8_hi = like->nd8_hi;
+    } else {
+        nodata_interval(g->nodata, 0.0000001, &p.nd_lo, &p.nd_hi);
+        nodata_interval(g->nodata, 0.000001, &p.nd8_lo, &p.nd8_hi);
+    }
     {
         const bool e1 = p.nd_lo > p.nd_hi, e2 = p.nd8_lo > p.nd8_hi;
         if (e1 && e2) {
@@ -1220,7 +1228,6 @@ static int run_focal(pargo_ctx *ctx, const pargo_grid *g, const float *dem, int 
 
 struct BatchPlan {
     std::vector<unsigned char> key;  // tiles + parameters the plan was built for
-    void *d_mem = nullptr;
     FocalParams *d_tiles = nullptr;
     unsigned *d_first = nullptr;
     unsigned *d_queue = nullptr;
@@ -1231,6 +1238,7 @@ struct BatchPlan {
     int blocks = 0;
     bool do_slope = false, do_d8 = false;
     int sm = 0;  // slope mode shared by every tile (slope_mode)
+    unsigned long long runs = 0;  // graph runs so far
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
 };
@@ -1239,12 +1247,25 @@ void free_batch_plan(pargo_ctx *ctx)
 {
     BatchPlan *b = ctx->batch;
     if (!b) return;
-    hipStreamSynchronize(ctx->stream);
-    if (b->exec) hipGraphExecDestroy(b->exec);
+    if (b->exec) {
+        hipStreamSynchronize(ctx->stream);  // it may be running
+        hipGraphExecDestroy(b->exec);
+    }
     if (b->graph) hipGraphDestroy(b->graph);
-    if (b->d_mem) hipFree(b->d_mem);
     delete b;
     ctx->batch = nullptr;
+}
+
+void free_batch_mem(pargo_ctx *ctx)
+{
+    if (ctx->batch_mem) hipFree(ctx->batch_mem);
+    if (ctx->batch_host) hipHostFree(ctx->batch_host);
+    for (hipEvent_t &e : ctx->batch_copied) {
+        if (e) hipEventDestroy(e);
+        e = nullptr;
+    }
+    ctx->batch_mem = ctx->batch_host = nullptr;
+    ctx->batch_mem_bytes = 0;
 }
 
 template <int CPT, bool DO_SLOPE, int DO_D8, int SM>
@@ -1305,13 +1326,46 @@ static int blocks_c(pargo_ctx *ctx, const BatchPlan &b)
     });
 }
 
-// The persistent sequence: queue reset, batch kernel, fixup.
+// The persistent sequence: batch kernel, fixup (which leaves the item queue
+// at zero again, as the plan's upload does at first).
 static void enqueue_batch(const BatchPlan &b, hipStream_t s)
 {
-    hipLaunchKernelGGL(focal_queue_reset, dim3(1), dim3(1), 0, s, b.d_queue);
     if (b.cpt == 2) launch_batch_c<2>(b, s);
     else launch_batch_c<4>(b, s);
-    launch_fixup(b.h_tiles[0], b.d_tiles, b.ntiles, b.do_slope, b.do_d8, b.cpt, s);
+    launch_fixup(b.h_tiles[0], b.d_tiles, b.ntiles, b.do_slope, b.do_d8, b.cpt, s, b.d_queue);
+}
+
+// The device copy of the batch plan and two page-locked host copies, kept by
+// the context: a new plan is uploaded in stream order behind the runs of the
+// one before, with no allocation and no wait (each host copy is written again
+// only when its last upload has been made).
+static int ensure_batch_mem(pargo_ctx *ctx, size_t bytes, unsigned char **host)
+{
+    // a captured upload would read the host copy at every replay
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    PARGO_HIP(ctx, hipStreamIsCapturing(ctx->stream, &capturing));
+    if (capturing != hipStreamCaptureStatusNone)
+        return fail(ctx, PARGO_E_DEVICE, "a batch's first run cannot be captured: run it once before");
+    if (ctx->batch_mem_bytes < bytes) {
+        hipError_t e = hipStreamSynchronize(ctx->stream);  // the old copies may be in use
+        if (e != hipSuccess) return fail(ctx, PARGO_E_DEVICE, "hipStreamSynchronize: %s", hipGetErrorString(e));
+        free_batch_mem(ctx);
+        const size_t want = 2 * bytes;
+        e = dev_malloc(&ctx->batch_mem, want, "batch plan");
+        if (e == hipSuccess) e = hipHostMalloc(&ctx->batch_host, 2 * want, hipHostMallocDefault);
+        for (int k = 0; k < 2 && e == hipSuccess; k++)
+            e = hipEventCreateWithFlags(&ctx->batch_copied[k], hipEventDisableTiming);
+        if (e != hipSuccess) {
+            free_batch_mem(ctx);
+            return fail(ctx, PARGO_E_NOMEM, "hipMalloc for the batch plan: %s%s", hipGetErrorString(e), injected_note());
+        }
+        ctx->batch_mem_bytes = want;
+    }
+    ctx->batch_slot ^= 1;
+    const hipError_t e = hipEventSynchronize(ctx->batch_copied[ctx->batch_slot]);
+    if (e != hipSuccess) return fail(ctx, PARGO_E_DEVICE, "hipEventSynchronize: %s", hipGetErrorString(e));
+    *host = static_cast<unsigned char *>(ctx->batch_host) + ctx->batch_slot * ctx->batch_mem_bytes;
+    return PARGO_OK;
 }
 
 static int build_batch(pargo_ctx *ctx, const pargo_tile *tiles, int ntiles, int method, int unit, int dirtype, int cpt,
@@ -1349,7 +1403,7 @@ static int build_batch(pargo_ctx *ctx, const pargo_tile *tiles, int ntiles, int 
         }
         bool vec = false;
         rc = prepare(ctx, &tiles[t].grid, tiles[t].dem, method, unit, dirtype, tiles[t].slope_out, tiles[t].code_out,
-                     nullptr, b->h_tiles[t], vec);
+                     nullptr, b->h_tiles[t], vec, t > 0 ? &tiles[t - 1].grid : nullptr, t > 0 ? &b->h_tiles[t - 1] : nullptr);
         if (rc) {
             delete b;
             return rc;
@@ -1396,24 +1450,28 @@ static int build_batch(pargo_ctx *ctx, const pargo_tile *tiles, int ntiles, int 
         return fail(ctx, PARGO_E_INVALID, "batch has too many work items");
     }
     b->total = (unsigned)total;
+    // one upload: the rasters, the first items, the queue at zero
     const size_t bt = sizeof(FocalParams) * ntiles, bf = sizeof(unsigned) * ntiles;
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    hipError_t e = dev_malloc(&b->d_mem, al(bt) + al(bf) + 256, "batch plan");
-    if (e != hipSuccess) {
+    const size_t bytes = al(bt) + al(bf) + 256;
+    unsigned char *host = nullptr;
+    rc = ensure_batch_mem(ctx, bytes, &host);
+    if (rc) {
         delete b;
-        return fail(ctx, PARGO_E_NOMEM, "hipMalloc for the batch plan: %s%s", hipGetErrorString(e), injected_note());
+        return rc;
     }
-    b->d_tiles = (FocalParams *)b->d_mem;
-    b->d_first = (unsigned *)((char *)b->d_mem + al(bt));
-    b->d_queue = (unsigned *)((char *)b->d_mem + al(bt) + al(bf));
-    e = hipMemcpyAsync(b->d_tiles, dev.data(), bt, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(b->d_first, first.data(), bf, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    std::memcpy(host, dev.data(), bt);
+    std::memcpy(host + al(bt), first.data(), bf);
+    std::memset(host + al(bt) + al(bf), 0, 256);
+    hipError_t e = hipMemcpyAsync(ctx->batch_mem, host, bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) e = hipEventRecord(ctx->batch_copied[ctx->batch_slot], ctx->stream);
     if (e != hipSuccess) {
-        hipFree(b->d_mem);
         delete b;
         return fail(ctx, PARGO_E_DEVICE, "uploading the batch plan: %s", hipGetErrorString(e));
     }
+    b->d_tiles = (FocalParams *)ctx->batch_mem;
+    b->d_first = (unsigned *)((char *)ctx->batch_mem + al(bt));
+    b->d_queue = (unsigned *)((char *)ctx->batch_mem + al(bt) + al(bf));
     b->blocks = cpt == 2 ? blocks_c<2>(ctx, *b) : blocks_c<4>(ctx, *b);
     b->blocks = (int)std::min((long long)b->blocks, ((long long)b->total + 3) / 4);  // four waves each
     ctx->batch = b;
@@ -1447,6 +1505,16 @@ static int run_batch(pargo_ctx *ctx, BatchPlan *b, int mode, int rows_per_strip)
     if (mode == PARGO_BATCH_PERSISTENT) {
         enqueue_batch(*b, s);
         return check_launch(ctx, "pargo_batch_slope_d8 (persistent)");
+    }
+    // The first run of a plan is launched as it is; a batch that is run again
+    // is worth the capture (about 60 us).  So is a run on a stream that the
+    // caller is capturing: its launches go into the caller's graph (a graph
+    // launched there would not).
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    PARGO_HIP(ctx, hipStreamIsCapturing(s, &capturing));
+    if (b->runs++ == 0 || capturing != hipStreamCaptureStatusNone) {
+        enqueue_batch(*b, s);
+        return check_launch(ctx, "pargo_batch_slope_d8 (graph)");
     }
     if (!b->exec) {
         // capture on a private stream so that a caller's legacy default

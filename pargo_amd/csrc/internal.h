@@ -37,6 +37,11 @@ struct pargo_ctx {
     // batched slope/D8: the last plan (with its captured graph) and the
     // launch shape chosen by pargo_batch_autotune
     pargo::BatchPlan *batch = nullptr;
+    void *batch_mem = nullptr;   // the plan's device copy (ensure_batch_mem)
+    void *batch_host = nullptr;  // two page-locked host copies
+    size_t batch_mem_bytes = 0;
+    hipEvent_t batch_copied[2] = {nullptr, nullptr};  // each host copy's last upload
+    int batch_slot = 0;
     int batch_cpt = 4;
     int batch_rows = 32;  // once batch_tuned; by the batch's size before
     int batch_tuned = 0;
@@ -48,6 +53,7 @@ struct pargo_ctx {
 
 namespace pargo {
 void free_batch_plan(pargo_ctx *ctx);
+void free_batch_mem(pargo_ctx *ctx);
 // Resolves ctx->noalloc_scratch with ctx->device current.
 int resolve_noalloc_scratch(pargo_ctx *ctx);
 }
