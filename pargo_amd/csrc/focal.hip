@@ -113,7 +113,7 @@ struct FocalParams {
     // Strips (one wave's columns over a row strip) with a window that holds
     // Inf or |z| >= 2^40 are queued here; focal_fixup_kernel recomputes those
     // windows with the reference-order FP64 code.
-    unsigned *fix_count;  // [0] queued strips, [1] finished fixup blocks
+    unsigned *fix_count;  // [0] queued strips, [1] finished fixup blocks; null: the waves do it themselves
     uint4 *fix_list;      // (tile index, first row, end row, first column)
     unsigned fix_cap;
     unsigned tile_id;     // index of this raster in a batch (0 otherwise)
@@ -709,6 +709,31 @@ __device__ __forceinline__ void focal_step(const FocalParams &p, int r, int rlas
     }
 }
 
+// The window of cell (r, c) with the reference-order FP64 code, if it holds
+// Inf or |z| >= 2^40; nothing otherwise.
+template <bool DO_SLOPE, bool DO_D8>
+__device__ __forceinline__ void exact_window(const FocalParams &p, int r, int c)
+{
+    if (r < 1 || r > p.rows - 2 || c < 1 || c > p.cols - 2) return;
+    double d[9];
+    bool nd = false, nd8 = false, sp = false;
+    for (int k = 0; k < 9; k++) {
+        const float f = p.dem[(long long)(r + k / 3 - 1) * p.pitch + (c + k % 3 - 1)];
+        nd |= in_interval(f, p.nd_lo, p.nd_hi);
+        nd8 |= in_interval(f, p.nd8_lo, p.nd8_hi);
+        sp |= !(__builtin_fabsf(f) < 0x1p40f);
+        d[k] = (double)f;
+    }
+    if (!sp) return;
+    const long long o = (long long)r * p.pitch + c;
+    if (DO_D8 && !nd8) {
+        unsigned v = d8_exact(d);
+        if (p.dirtype == 8) v = v ? (unsigned)c_lut8.v[v] : 255u;
+        p.code[o] = (uint8_t)v;
+    }
+    if (DO_SLOPE && !nd) p.slope[o] = slope_unit((float)slope_generic(d, p.method, p.cs), p.unit);
+}
+
 // Pairs from a row to the row below (the prologue of a strip).
 template <int CPT, bool DO_SLOPE, int DO_D8, int SM>
 __device__ __forceinline__ void pair_rows(Slot<CPT> &up, const Slot<CPT> &below)
@@ -725,7 +750,7 @@ __device__ __forceinline__ void pair_rows(Slot<CPT> &up, const Slot<CPT> &below)
 
 // One wave computes output rows [rbeg, rend) of the 64*CPT columns that
 // start at wave_c0 (wave-uniform).
-template <int CPT, bool VECLOAD, bool DO_SLOPE, int DO_D8, int SM, bool MASK>
+template <int CPT, bool VECLOAD, bool DO_SLOPE, int DO_D8, int SM, bool MASK, bool IN_WAVE>
 __device__ __forceinline__ void focal_strip_impl(const FocalParams &p, int wave_c0, int lane, int rbeg, int rend)
 {
     const int c0 = wave_c0 + lane * CPT;
@@ -755,25 +780,32 @@ __device__ __forceinline__ void focal_strip_impl(const FocalParams &p, int wave_
         if (r + 2 >= rend) break;
         focal_step<CPT, VECLOAD, DO_SLOPE, DO_D8, SM, MASK>(p, r + 2, rend, c0, lane, colb, C, A, B, R2, special);
     }
-    // queue the strip for the exact pass (rare: Inf or |z| >= 2^40 nearby)
-    if (__builtin_amdgcn_ballot_w64(special) != 0 && lane == 0) {
+    // the exact pass (rare: Inf or |z| >= 2^40 nearby): by the wave itself in
+    // a small raster, else queued
+    if (__builtin_amdgcn_ballot_w64(special) == 0) return;
+    if (IN_WAVE && p.fix_count == nullptr) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the strip's own stores are made
+        for (int r = rbeg; r < rend; r++)
+            for (int j = 0; j < CPT; j++) exact_window<DO_SLOPE, DO_D8 != 0>(p, r, c0 + j);
+    } else if (lane == 0) {
         const unsigned k = atomicAdd(p.fix_count, 1u);
         if (k < p.fix_cap) p.fix_list[k] = make_uint4(p.tile_id, (unsigned)rbeg, (unsigned)rend, (unsigned)wave_c0);
     }
 }
 
 // VEC: the raster's pitch and base allow vector access; a wave uses it when
-// all its columns are inside the raster.
-template <int CPT, bool VEC, bool DO_SLOPE, int DO_D8, int SM, bool MASK = true>
+// all its columns are inside the raster.  IN_WAVE false (batches) compiles
+// the exact pass by the wave itself out.
+template <int CPT, bool VEC, bool DO_SLOPE, int DO_D8, int SM, bool MASK = true, bool IN_WAVE = true>
 __device__ __forceinline__ void focal_strip(const FocalParams &p, int wave_c0, int lane, int rbeg, int rend)
 {
     if constexpr (VEC) {
         if (wave_c0 + 64 * CPT <= p.cols) {
-            focal_strip_impl<CPT, true, DO_SLOPE, DO_D8, SM, MASK>(p, wave_c0, lane, rbeg, rend);
+            focal_strip_impl<CPT, true, DO_SLOPE, DO_D8, SM, MASK, IN_WAVE>(p, wave_c0, lane, rbeg, rend);
             return;
         }
     }
-    focal_strip_impl<CPT, false, DO_SLOPE, DO_D8, SM, MASK>(p, wave_c0, lane, rbeg, rend);
+    focal_strip_impl<CPT, false, DO_SLOPE, DO_D8, SM, MASK, IN_WAVE>(p, wave_c0, lane, rbeg, rend);
 }
 
 // One raster: block = 4 waves side by side, one row strip per block.
@@ -797,8 +829,9 @@ __device__ __forceinline__ void focal_raster(const FocalParams &p)
     focal_strip<CPT, VEC, DO_SLOPE, DO_D8, SM, MASK>(p, wave_c0, lane, rbeg, rend);
 }
 
+// (D8 alone: at most 128 VGPRs, for four waves per SIMD.)
 template <int CPT, bool VEC, bool DO_SLOPE, int DO_D8, int SM>
-__global__ __launch_bounds__(256) void focal_kernel(FocalParams p)
+__global__ __launch_bounds__(256, DO_SLOPE ? 1 : 4) void focal_kernel(FocalParams p)
 {
     focal_raster<CPT, VEC, DO_SLOPE, DO_D8, SM>(p);
 }
@@ -872,8 +905,8 @@ __device__ __forceinline__ void focal_batch_body(const FocalParams *__restrict__
         const int wx = (int)(local % (unsigned)p.waves_x), strip = (int)(local / (unsigned)p.waves_x);
         const int rbeg = strip * p.rows_per_strip;
         const int rend = min(rbeg + p.rows_per_strip, p.rows);
-        if (p.vec) focal_strip<CPT, true, DO_SLOPE, DO_D8, SM, false>(p, wx * 64 * CPT, lane, rbeg, rend);
-        else focal_strip<CPT, false, DO_SLOPE, DO_D8, SM, false>(p, wx * 64 * CPT, lane, rbeg, rend);
+        if (p.vec) focal_strip<CPT, true, DO_SLOPE, DO_D8, SM, false, false>(p, wx * 64 * CPT, lane, rbeg, rend);
+        else focal_strip<CPT, false, DO_SLOPE, DO_D8, SM, false, false>(p, wx * 64 * CPT, lane, rbeg, rend);
     }
 }
 
@@ -908,26 +941,7 @@ __global__ __launch_bounds__(256) void focal_fixup_kernel(FocalParams one, const
 {
     const unsigned *cnt = one.fix_count;
     const unsigned n = __atomic_load_n(&cnt[0], __ATOMIC_RELAXED);
-    auto fix = [&](const FocalParams &p, int r, int c) {
-        if (r < 1 || r > p.rows - 2 || c < 1 || c > p.cols - 2) return;
-        double d[9];
-        bool nd = false, nd8 = false, sp = false;
-        for (int k = 0; k < 9; k++) {
-            const float f = p.dem[(long long)(r + k / 3 - 1) * p.pitch + (c + k % 3 - 1)];
-            nd |= in_interval(f, p.nd_lo, p.nd_hi);
-            nd8 |= in_interval(f, p.nd8_lo, p.nd8_hi);
-            sp |= !(__builtin_fabsf(f) < 0x1p40f);
-            d[k] = (double)f;
-        }
-        if (!sp) return;
-        const long long o = (long long)r * p.pitch + c;
-        if (DO_D8 && !nd8) {
-            unsigned v = d8_exact(d);
-            if (p.dirtype == 8) v = v ? (unsigned)c_lut8.v[v] : 255u;
-            p.code[o] = (uint8_t)v;
-        }
-        if (DO_SLOPE && !nd) p.slope[o] = slope_unit((float)slope_generic(d, p.method, p.cs), p.unit);
-    };
+    auto fix = [&](const FocalParams &p, int r, int c) { exact_window<DO_SLOPE, DO_D8>(p, r, c); };
     if (n <= one.fix_cap) {
         for (unsigned k = blockIdx.x; k < n; k += gridDim.x) {
             const uint4 e = one.fix_list[k];
@@ -1206,20 +1220,27 @@ static int run_focal(pargo_ctx *ctx, const pargo_grid *g, const float *dem, int 
     const bool do_slope = slope_out != nullptr;
     const bool do_d8 = code_out != nullptr;
     if (!do_slope && !do_d8) return fail(ctx, PARGO_E_INVALID, "%s: a NoData mask needs a slope or code output", name);
+    // A raster of few rows a wave (strip_rows' first range, up to 2048 x 2048
+    // cells) redoes its special windows in the waves that met them: the
+    // second launch, nearly always for an empty queue, costs 4 us and the gap
+    // before it.  In a large raster the queue spreads them over workgroups of
+    // their own.
+    const bool in_wave = strip_work(g->rows, g->cols, 64 * cfg.cpt) <= 4 * kStripWaves;
     if (noalloc) {
         // the static queue: no allocation; its counters may hold what an
         // interrupted earlier call left, so they are cleared first
         if (!ctx->noalloc_scratch) return fail(ctx, PARGO_E_DEVICE, "%s: the static fixup queue is unresolved", name);
         attach_fixup_at(ctx->noalloc_scratch, p);
-        hipLaunchKernelGGL(fixup_counters_reset, dim3(1), dim3(1), 0, ctx->stream, p.fix_count);
+        if (!in_wave) hipLaunchKernelGGL(fixup_counters_reset, dim3(1), dim3(1), 0, ctx->stream, p.fix_count);
     } else {
         rc = ensure_fixup(ctx);
         if (rc) return rc;
         attach_fixup(ctx, p);
     }
+    if (in_wave) p.fix_count = nullptr;
     launch_focal(p, cfg, vec, do_slope, do_d8, ctx->stream);
     rc = check_launch(ctx, name);
-    if (rc) return rc;
+    if (rc || in_wave) return rc;
     launch_fixup(p, nullptr, 1, do_slope, do_d8, cfg.cpt, ctx->stream);
     return check_launch(ctx, name);
 }

@@ -76,16 +76,18 @@ __device__ __forceinline__ void xcd_strip_order(unsigned &cb, unsigned &strip)
 //   4096 x 4096   30.4 / 41.9 / 58.8       28.5 / 40.2 / 52.1  (4 rows)
 //   7001 x 5003   58.0 / 76.4 / 102.9      52.6 / 71.6 / 97.1  (7 rows)
 // At 16384^2 the longest strips stay the fastest (1 row doubles the time).
+constexpr long long kStripWaves = 4096;
 inline int strip_rows_of(long long work, int most)  // work: rows times strips side by side
 {
-    constexpr long long kWaves = 4096;
-    const long long n = work <= 4 * kWaves ? (work + kWaves - 1) / kWaves : (work + 5 * kWaves / 2) / (5 * kWaves);
-    const long long least = work <= 4 * kWaves ? 1 : 4;
+    const long long n =
+        work <= 4 * kStripWaves ? (work + kStripWaves - 1) / kStripWaves : (work + 5 * kStripWaves / 2) / (5 * kStripWaves);
+    const long long least = work <= 4 * kStripWaves ? 1 : 4;
     return (int)(n < least ? least : n > most ? most : n);
 }
+inline long long strip_work(int rows, int cols, int width) { return (long long)rows * ((cols + width - 1) / width); }
 inline int strip_rows(int rows, int cols, int width, int most)
 {
-    return strip_rows_of((long long)rows * ((cols + width - 1) / width), most);
+    return strip_rows_of(strip_work(rows, cols, width), most);
 }
 
 }  // namespace pargo
