@@ -87,6 +87,8 @@ int ensure_scratch(pargo_ctx *ctx, size_t bytes)
 int ensure_report(pargo_ctx *ctx)
 {
     if (ctx->report) return PARGO_OK;
+    for (hipEvent_t &e : ctx->report_event)
+        if (!e) PARGO_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     hipError_t e = alloc_should_fail("report words") ? hipErrorOutOfMemory
                                                      : hipHostMalloc(&ctx->report, 64, hipHostMallocDefault);
     if (e != hipSuccess) {
@@ -203,6 +205,8 @@ int pargo_destroy(pargo_ctx *ctx)
     if (ctx->stream && ctx->stream != ctx->own_stream) hipStreamSynchronize(ctx->stream);
     if (ctx->scratch) hipFree(ctx->scratch);
     if (ctx->report) hipHostFree(ctx->report);
+    for (hipEvent_t e : ctx->report_event)
+        if (e) hipEventDestroy(e);
     pargo::free_batch_plan(ctx);
     pargo::free_batch_mem(ctx);
     if (ctx->fix_mem) hipFree(ctx->fix_mem);

@@ -30,6 +30,7 @@ struct pargo_ctx {
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
     void *report = nullptr;  // page-locked host words that progress counters are copied to (64 bytes)
+    hipEvent_t report_event[2] = {nullptr, nullptr};  // recorded behind such a copy
     void *fix_mem = nullptr;  // focal fixup queue (counters + cell list)
     // device address of the static fixup queue of pargo_slope_d8_noalloc on
     // this context's device (resolved once by pargo_create)
@@ -78,7 +79,7 @@ const char *injected_note();
 // Grows the context scratch to at least `bytes`.
 int ensure_scratch(pargo_ctx *ctx, size_t bytes);
 
-// Allocates the context's page-locked report words: a device-to-host copy of
+// Allocates the context's page-locked report words and their events: a device-to-host copy of
 // a few counters into pageable memory goes through the runtime's staging and
 // held the stream about 50 us per check of pitremove, into these 25-30.
 int ensure_report(pargo_ctx *ctx);
