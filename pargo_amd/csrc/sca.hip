@@ -391,20 +391,20 @@ __device__ __forceinline__ int my_cell(int k) { return ((int)(threadIdx.x >> 6) 
 // Adds the thread's cells k with bit k of `m` set (all lanes call).
 __device__ __forceinline__ void add_starts(StartList &L, unsigned m)
 {
-    unsigned total = 0;
+    if (__builtin_amdgcn_ballot_w64(m != 0) == 0) return;
+    // the lanes' counts, up to 8 each, summed bit by bit over the lanes below
+    unsigned before = 0, total = 0;
+    const unsigned n = (unsigned)__builtin_popcount(m);
 #pragma unroll
-    for (int k = 0; k < 8; k++) total += (unsigned)__builtin_popcountll(__builtin_amdgcn_ballot_w64((m >> k) & 1u));
-    unsigned at = 0;
-    if (total != 0 && (threadIdx.x & 63) == 0) at = atomicAdd(&L.n, total);
-    at = (unsigned)__builtin_amdgcn_readfirstlane((int)at);
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const unsigned long long b = __builtin_amdgcn_ballot_w64((m >> k) & 1u);
-        if ((m >> k) & 1u)
-            L.cell[at + __builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b, 0u))] =
-                (uint16_t)my_cell(k);
-        at += (unsigned)__builtin_popcountll(b);
+    for (int bit = 0; bit < 4; bit++) {
+        const unsigned long long b = __builtin_amdgcn_ballot_w64((n >> bit) & 1u);
+        before += __builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b, 0u)) << bit;
+        total += (unsigned)__builtin_popcountll(b) << bit;
     }
+    unsigned at = 0;
+    if ((threadIdx.x & 63) == 0) at = atomicAdd(&L.n, total);
+    at = (unsigned)__builtin_amdgcn_readfirstlane((int)at) + before;
+    for (; m; m &= m - 1) L.cell[at++] = (uint16_t)my_cell(__builtin_ctz(m));
 }
 // next_of for a cell whose next cell lies in the tile (perimeter cells are
 // set by next_of afterwards): the index plus the code's offset, by a byte
@@ -449,14 +449,18 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
         auto inm_at = [&](int r, int c) -> unsigned {
             return inner ? reinterpret_cast<const uint8_t *>(S.swar.inm[r + 1])[c + 4] : S.general.inm[r + 1][c + 1];
         };
-        const unsigned mine = (stw[pcell] & 15u) ? inm_at(lr, lc) : 0u;  // only a cell that waits at all
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int k = win_of_bit(j), ur = lr + k / 3 - 1, uc = lc + k % 3 - 1;
-            if ((unsigned)ur < (unsigned)kTileR && (unsigned)uc < (unsigned)kTileC) continue;
-            const int gr = r0 + ur, gc = c0 + uc;
-            const bool interior = gr >= 1 && gr <= p.rows - 2 && gc >= 1 && gc <= p.cols - 2;
-            if (interior && ((mine >> j) & 1u) && (p.converge || j < 4) && inm_at(ur, uc) != 0) ext |= 1u << j;
+        // inflows from outside that may be waited for, of a cell that waits
+        // at all: bits 0-2 come from the row above, 5-7 from the row below,
+        // 0, 3, 5 from the left and 2, 4, 7 from the right
+        unsigned m = (stw[pcell] & 15u) ? inm_at(lr, lc) : 0u;
+        m &= (lr == 0 ? 0x07u : 0u) | (lr == kTileR - 1 ? 0xE0u : 0u) | (lc == 0 ? 0x29u : 0u) | (lc == kTileC - 1 ? 0x94u : 0u);
+        if (!p.converge) m &= 0x0Fu;
+        for (; m; m &= m - 1) {
+            const int j = __builtin_ctz(m);
+            const unsigned k = (unsigned)win_of_bit(j);
+            const int ur = lr + (int)(k / 3u) - 1, uc = lc + (int)(k % 3u) - 1, gr = r0 + ur, gc = c0 + uc;
+            const bool interior = inner || (gr >= 1 && gr <= p.rows - 2 && gc >= 1 && gc <= p.cols - 2);
+            if (interior && inm_at(ur, uc) != 0) ext |= 1u << j;
         }
     }
     const unsigned next_ = (unsigned)__builtin_popcount(ext);
