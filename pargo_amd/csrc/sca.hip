@@ -64,9 +64,9 @@
 // admits for arbitrary codes) keep the sum of the done inflows they
 // received, which is their area.
 //
-// Measured on the headline DEM's codes: 16384^2 in the reference mode 2.06 ms
-// (local 0.99, link 0.07, cross 0.12, final 0.94), 5003 x 7001 in the
-// converging mode 0.35 ms, and 0.11 ms for the codes of a filled 1501 x 2003
+// Measured on the headline DEM's codes: 16384^2 in the reference mode 1.96 ms
+// (local 0.94, link 0.07, cross 0.12, final 0.88), 5003 x 7001 in the
+// converging mode 0.34 ms, and 0.11 ms for the codes of a filled 1501 x 2003
 // DEM, whose paths are long.  One walk over the whole raster with a global
 // atomic or a static word read per hop (33 bytes of HBM traffic, up to 1336
 // hops in a row) took 4.24, 1.21 and 1.15 ms.
@@ -715,29 +715,40 @@ __global__ void sca_last_cell_kernel(ScaParams p)
 // neither (NaN) marks a cell that takes no inflow.  A valid cell flows to
 // window index k when v == k; it rejects inflow from window cell k when
 // dir + v == 8 in double for dir = 8 - k (scaOperator.cpp:71,94).
+// A whole number 0..8 needs no search; the others that can satisfy either
+// equation lie strictly between -1 and 9.
+__device__ __forceinline__ unsigned classify(double v, double nodata)
+{
+    const double dv = fabs(v - nodata);
+    if (dv < 0.000001) return PARGO_FLOW_NODATA;
+    if (!(dv > 0.000001)) return PARGO_FLOW_INERT;
+    if (!(v > -1.0 && v < 9.0)) return PARGO_FLOW_NONE;
+    const int whole = (int)v;
+    if ((double)whole == v) return whole == 4 ? (unsigned)PARGO_FLOW_NONE : (unsigned)whole;
+    unsigned ex = kNone;
+    for (int dir = 0; dir <= 8; dir++)
+        if (dir != 4 && (double)dir + v == 8.0) ex = 8u - (unsigned)dir;
+    return ex != kNone ? PARGO_FLOW_EXCL | ex : (unsigned)PARGO_FLOW_NONE;
+}
+
+// Memory-bound (9 bytes a cell): four cells a lane, as two 16-byte loads and
+// one 4-byte store (5003 x 7001: 56 us, one cell a lane took 101).
+typedef double f64x2_a8 __attribute__((ext_vector_type(2), aligned(8)));
+
 __global__ __launch_bounds__(256) void d8_classify_kernel(const double *__restrict__ d8, uint8_t *__restrict__ out,
                                                           long long pitch, int rows, int cols, double nodata)
 {
-    const int c = blockIdx.x * 256 + threadIdx.x, r = blockIdx.y;
+    const int c = (blockIdx.x * 256 + threadIdx.x) * 4, r = blockIdx.y;
     if (c >= cols) return;
     const long long i = (long long)r * pitch + c;
-    const double v = d8[i];
-    const double dv = fabs(v - nodata);
-    unsigned b;
-    if (dv < 0.000001) {
-        b = PARGO_FLOW_NODATA;
-    } else if (dv > 0.000001) {
-        unsigned ex = kNone;
-        for (int dir = 0; dir <= 8; dir++)
-            if (dir != 4 && (double)dir + v == 8.0) ex = 8u - (unsigned)dir;
-        b = PARGO_FLOW_NONE;
-        for (int k = 0; k <= 8; k++)
-            if (k != 4 && v == (double)k) b = (unsigned)k;
-        if (b == PARGO_FLOW_NONE && ex != kNone) b = PARGO_FLOW_EXCL | ex;
+    if (c + 4 <= cols) {
+        const f64x2_a8 a = *reinterpret_cast<const f64x2_a8 *>(d8 + i), b = *reinterpret_cast<const f64x2_a8 *>(d8 + i + 2);
+        const unsigned w = classify(a.x, nodata) | classify(a.y, nodata) << 8 | classify(b.x, nodata) << 16 |
+                           classify(b.y, nodata) << 24;
+        *reinterpret_cast<u32_b1 *>(out + i) = w;
     } else {
-        b = PARGO_FLOW_INERT;
+        for (int k = 0; c + k < cols; k++) out[i + k] = (uint8_t)classify(d8[i + k], nodata);
     }
-    out[i] = (uint8_t)b;
 }
 
 // NoData values the flow classes cannot carry: the reference would treat
@@ -771,7 +782,7 @@ extern "C" int pargo_d8_classify(pargo_ctx *ctx, const pargo_grid *g, const doub
                     g->nodata);
     int rc = pargo::bind(ctx);
     if (rc) return rc;
-    dim3 grid((g->cols + 255) / 256, g->rows);
+    dim3 grid((g->cols + 1023) / 1024, g->rows);
     hipLaunchKernelGGL(pargo::d8_classify_kernel, grid, dim3(256), 0, ctx->stream, d8, flow_out, pitch, g->rows,
                        g->cols, g->nodata);
     return pargo::check_launch(ctx, "pargo_d8_classify");
