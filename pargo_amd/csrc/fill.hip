@@ -90,8 +90,9 @@ constexpr unsigned kAll = 1u << 15;  // never visited: every row is to be evalua
 
 // A worklist is kSub lists, a tile's by its number modulo kSub, each with a
 // counter in a cache line of its own: returning atomics on one address take
-// about 11 ns each here whatever else runs, and with one counter the passes
-// at 16384^2 took as long as their 300,000 appends did.
+// turns (577,000 of them, from a cursor over the list, added 6.4 ms at
+// 16384^2, 11 ns each).  With one counter per list the passes took 7.09 ms
+// with their init against 6.85, the init 0.89 against 0.62.
 constexpr int kSub = 64, kSubStride = 32;  // stride in 4-byte words
 constexpr int kSetWords = kSub * kSubStride;
 
