@@ -28,8 +28,9 @@
 // monotone, so min_n RN(W(n) + gap) = RN(min_n W(n) + gap)); taking the cell
 // itself into min_n changes nothing, since W + gap >= W.
 //
-// Device order: 64 x 32 tiles, one workgroup of four waves each, a wave
-// holding 8 rows in registers (one column per lane).  With h(r) the minimum
+// Device order: 64 x 32 tiles, one workgroup of four waves each (two for
+// large rasters), a wave holding 8 (16) rows in registers, one column per
+// lane.  With h(r) the minimum
 // of a row's W over each column and its two neighbours (two DPP moves), an
 // update of row r is two minima over h(r-1), h(r), h(r+1), one addition, a
 // maximum and a compare; h(r) is formed again only when the row changed.
@@ -40,7 +41,7 @@
 // of the tile's first and last columns, which the tiles beside it read as
 // their halo columns), and the tiles across each changed edge or corner are
 // scheduled for the next pass with flags that say which edge (and for side
-// edges which bands of 8 rows) changed; only the waves next to such a
+// edges which waves' rows) changed; only the waves next to such a
 // change start with rows to evaluate, and the others load nothing unless
 // the change reaches them.  Passes repeat until none is scheduled.  Tiles
 // read each other's edges while they change; that only feeds the monotone
@@ -53,14 +54,14 @@
 // the init kernel opened: with every valid W at 10000, nothing else can
 // change.
 //
-// Measured at 16384^2 on the synthetic DEM: 6.8 ms (19.3 ms with nine-cell
-// windows swept over whole tiles, two launches per pass): 0.6 ms init, 6 ms
-// in 32 passes, 525,000 visits of which half change something and 3.3 waves
-// on average load.  A visit that changes nothing reads 26 KB at 5.1 TB/s
-// (0.67 ms for all 131,072 tiles), which is 2.2 ms of the passes; the rest is
-// the evaluations (3.4 rounds a visit), the rows written (4.8 GB) and the
-// 15-20 us a pass of few tiles takes.  Occupancy (4 to 6 waves per SIMD),
-// a tiled layout of W and 16- or 64-row tiles changed nothing or lost
+// Measured at 16384^2 on the synthetic DEM: 6.1 ms (19.3 ms with nine-cell
+// windows swept over whole tiles, two launches per pass).  With four waves a
+// tile, 6.8 ms: 0.6 ms init, 6 ms in 32 passes, 525,000 visits of which half
+// change something and 3.3 waves on average load.  A visit that changes
+// nothing reads 26 KB at 5.1 TB/s (0.67 ms for all 131,072 tiles), which is
+// 2.2 ms of the passes; the rest is the evaluations (3.4 rounds a visit), the
+// rows written (4.8 GB) and the 15-20 us a pass of few tiles takes.  Also with four waves: occupancy (4 to
+// 6 waves per SIMD), a tiled layout of W and 16- or 64-row tiles changed nothing or lost
 // (16 rows 11.2 ms, 64 rows 8.9 ms against 7.2); putting a visit off when a
 // neighbour has changed during the pass saved no visits and took 56 passes
 // instead of 32.
@@ -75,15 +76,20 @@ namespace pargo {
 namespace {
 
 constexpr int kTW = 64, kTH = 32;  // tile: 64 columns x 32 rows
-constexpr int kRW = 8;             // rows per wave
-constexpr int kWaves = kTH / kRW;
 static_assert(kTW == 64, "a lane is a column of the tile");
-static_assert(kWaves == 4, "the flags hold one bit per band of kRW rows and side, four of each");
+// From this many tiles on, a tile is held by two waves of 16 rows instead of
+// four of 8: fewer waves wait for each other at the round's barrier (eight
+// waves of 4 rows took 12.4 ms at 16384^2, four 6.8, two 6.1), but a wave's
+// chain of rows is longer, which a raster that does not fill the GPU many
+// times over waits for.  us, four waves / two: 1000^2 (512 tiles) 438 / 484,
+// 2048^2 678 / 734, 3000 x 4000 (5,922) 1014 / 1057, 5003 x 7001 (17,270)
+// 1785 / 1735, 8192^2 2827 / 2610, 16384^2 6989 / 6173.
+constexpr int kTallTiles = 16384;
 constexpr double kGap = 0.0005;    // pitRemoveOperator.cpp:36
 constexpr double kStart = 10000.0; // pitRemoveOperator.cpp:41
 
 // What changed around a tile since it was last settled.
-constexpr unsigned kLeft = 1u, kRight = 1u << 4;  // halo column, one bit per band of kRW rows
+constexpr unsigned kLeft = 1u, kRight = 1u << 4;  // halo column, one bit per wave's band of rows (at most 4)
 constexpr unsigned kTop = 1u << 8, kBottom = 1u << 9;
 constexpr unsigned kTopLeft = 1u << 10, kTopRight = 1u << 11, kBottomLeft = 1u << 12, kBottomRight = 1u << 13;
 constexpr unsigned kAll = 1u << 15;  // never visited: every row is to be evaluated
@@ -304,7 +310,9 @@ __global__ void fill_reset_kernel(FillParams p, int n)
     }
 }
 
+template <int RW>
 struct FillShared {
+    static constexpr int kWaves = kTH / RW;
     double h[2][kWaves][2][kTW];  // per round parity and wave: h of its first and last row
     unsigned note[2][kWaves];     // per round parity and wave: kSentTop, kSentBottom, kGoing
     unsigned start[2];            // by parity of the visit: its flags (0: none)
@@ -328,9 +336,12 @@ struct Flagged {
 };
 
 // One visit of one tile (see the top of the file).
+template <int RW>
 __device__ __forceinline__ void fill_tile(const FillParams &p, int tile, unsigned start, int parity, int pass,
-                                          FillShared &S, Flagged &flagged)
+                                          FillShared<RW> &S, Flagged &flagged)
 {
+    constexpr int kRW = RW, kWaves = kTH / RW;
+    static_assert(kWaves <= 4, "the flags hold one bit per wave and side, four of each");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     auto flush = [&]() {
@@ -509,7 +520,7 @@ __device__ __forceinline__ void fill_tile(const FillParams &p, int tile, unsigne
             // that: the band's own and, from its first or last row, the next
             const unsigned bands = 1u << wave | (touched & 1u) << wave >> 1 | (touched >> (kRW - 1) & 1u) << wave << 1;
             const unsigned lb = cols & 1ull ? bands : 0u, rb = cols >> 63 ? bands : 0u;
-            unsigned o = (lb & 15u) * kLeft | (rb & 15u) * kRight;
+            unsigned o = (lb & ((1u << kWaves) - 1u)) * kLeft | (rb & ((1u << kWaves) - 1u)) * kRight;
             if (wave == 0 && first) o |= kTop | (first & 1ull ? kTopLeft : 0u) | (first >> 63 ? kTopRight : 0u);
             if (wave == kWaves - 1 && last)
                 o |= kBottom | (last & 1ull ? kBottomLeft : 0u) | (last >> 63 ? kBottomRight : 0u);
@@ -545,9 +556,10 @@ __device__ __forceinline__ void flag_around(const FillParams &p, int tile, unsig
     }
 }
 
-__global__ __launch_bounds__(256, 5) void fill_pass_kernel(FillParams p, int pass)
+template <int RW>
+__global__ __launch_bounds__(64 * (kTH / RW), RW == 8 ? 5 : 3) void fill_pass_kernel(FillParams p, int pass)
 {
-    __shared__ FillShared S;
+    __shared__ FillShared<RW> S;
     const int lane = threadIdx.x & 63;
     // the sublists' lengths, one per lane, and where each ends in the whole list
     const unsigned len = p.count[(pass % 3) * kSetWords + lane * kSubStride];
@@ -594,7 +606,7 @@ __global__ __launch_bounds__(256, 5) void fill_pass_kernel(FillParams p, int pas
         unsigned next_start = 0;
         if (more && threadIdx.x == 0) next_start = *visit_flags(p, next_tile, pass);
         if (e + 2 * stride < n) ahead = entry(e + 2 * stride);
-        fill_tile(p, tile, start, parity, pass, S, flagged);
+        fill_tile<RW>(p, tile, start, parity, pass, S, flagged);
         if (more && threadIdx.x == 0) {
             S.start[parity ^ 1] = next_start;
             S.out[parity ^ 1] = 0;
@@ -676,7 +688,11 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     // resident at once
     const int cus = ctx->num_cu > 0 ? ctx->num_cu : 256;
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pargo::fill_pass_kernel, 256, 0) != hipSuccess ||
+    const bool tall = ntiles >= pargo::kTallTiles;
+    const int pass_threads = tall ? 128 : 256;
+    if ((tall ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pargo::fill_pass_kernel<16>, pass_threads, 0)
+              : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pargo::fill_pass_kernel<8>, pass_threads, 0)) !=
+            hipSuccess ||
         per_cu < 1)
         per_cu = 4;
     const int pass_blocks = std::min(ntiles, cus * per_cu);
@@ -686,7 +702,12 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     // the end, take 2 us each.
     auto launch = [&](int first) -> int {
         for (int k = 0; k < kBatch; k++)
-            hipLaunchKernelGGL(pargo::fill_pass_kernel, dim3(pass_blocks), dim3(256), 0, ctx->stream, p, first + k);
+            if (tall)
+                hipLaunchKernelGGL(pargo::fill_pass_kernel<16>, dim3(pass_blocks), dim3(pass_threads), 0, ctx->stream, p,
+                                   first + k);
+            else
+                hipLaunchKernelGGL(pargo::fill_pass_kernel<8>, dim3(pass_blocks), dim3(pass_threads), 0, ctx->stream, p,
+                                   first + k);
         const int slot = first / kBatch & 1;
         PARGO_HIP(ctx, hipMemcpyAsync(static_cast<unsigned *>(ctx->report) + 4 * slot, scr, 3 * sizeof(unsigned),
                                       hipMemcpyDeviceToHost, ctx->stream));

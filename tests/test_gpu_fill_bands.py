@@ -61,3 +61,26 @@ def test_nodata_outside_the_usual_range(nodata):
     if np.isfinite(nodata):
         z[40:43, 60:70] = nodata
     check(z, nodata)
+
+
+@pytest.mark.parametrize("rows,cols", [(1050, 32001), (16401, 2011)])
+def test_two_waves_a_tile(rows, cols):
+    # rasters of 16,384 tiles and more; too large for the oracle's sweeps, so
+    # the settled equations, which have one solution, are checked at every cell
+    import torch
+    from pargo_amd import hydro, synth
+    z = torch.from_numpy(synth.workload_dem("slope_d8", rows, cols)).cuda()
+    w, _ = hydro.pit_remove(z, ND)
+    d = z.double()
+    out = (d - ND).abs() <= 1e-6
+    out[0], out[-1], out[:, 0], out[:, -1] = True, True, True, True
+    assert bool((w[out] == ND).all())
+    v = torch.where(out, torch.full_like(w, -np.inf), w)  # NoData opens its neighbours
+    n = torch.full_like(v[1:-1, 1:-1], np.inf)
+    for i in range(3):
+        for j in range(3):
+            if (i, j) != (1, 1):
+                n = torch.minimum(n, v[i:rows - 2 + i, j:cols - 2 + j])
+    want = torch.clamp(torch.maximum(d[1:-1, 1:-1], n + 0.0005), max=10000.0)
+    live = ~out[1:-1, 1:-1]
+    assert bool((w[1:-1, 1:-1][live] == want[live]).all())
