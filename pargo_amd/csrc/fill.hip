@@ -118,6 +118,24 @@ struct FillParams {
     double nodata;
 };
 
+// The least filled value there can be, min(smallest valid elevation, 10000),
+// from the range word; NaN when no cell is valid.
+__host__ __device__ inline double lowest_filled(unsigned key)
+{
+    const unsigned u = (key & 0x80000000u) ? (key & 0x7fffffffu) : ~key;
+    float mn;
+    __builtin_memcpy(&mn, &u, sizeof(mn));
+    return mn < kStart ? (double)mn : (mn != mn ? (double)mn : kStart);
+}
+
+// Whether the DEM is refused: NaN cells, or a NoData value that a filled one
+// can come within 1e-6 of (every valid W lies in [min(dem, 10000), 10000]).
+__host__ __device__ inline bool fill_refused(unsigned key, unsigned nans, double nodata)
+{
+    const double lo = lowest_filled(key);
+    return nans != 0 || (lo == lo && !(nodata < lo - 0.000001 || nodata > kStart + 0.000001));
+}
+
 __device__ __forceinline__ bool is_nd(const FillParams &p, float v) { return v >= p.nd_lo && v <= p.nd_hi; }
 
 // FP64 minimum and maximum without the quieting the compiler puts in front
@@ -569,7 +587,11 @@ __global__ __launch_bounds__(64 * (kTH / RW), RW == 8 ? 5 : 3) void fill_pass_ke
         const unsigned o = (unsigned)__shfl_up((int)end, off);
         if (lane >= off) end += o;
     }
-    const unsigned n = (unsigned)__builtin_amdgcn_readlane((int)end, kSub - 1);
+    // a DEM that is refused (the host learns it from the same words, passes
+    // later) is left as the init kernel made it: pass 0 does nothing, so the
+    // lists stay empty
+    const bool refused = pass == 0 && fill_refused(p.range[0], p.range[1], p.nodata);
+    const unsigned n = refused ? 0u : (unsigned)__builtin_amdgcn_readlane((int)end, kSub - 1);
     if (blockIdx.x == 0 && threadIdx.x < kSub) {
         // the counters that pass + 1 fills (pass - 1 read them)
         p.count[((pass + 2) % 3) * kSetWords + lane * kSubStride] = 0;
@@ -715,39 +737,41 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
         return PARGO_OK;
     };
     int pass = 0;
-    rc = launch(0);
-    if (rc) return rc;
-    for (;;) {
-        rc = launch(pass + kBatch);
+    auto settle = [&]() -> int {
+        int rc = launch(0);
         if (rc) return rc;
-        const int slot = pass / kBatch & 1;
-        PARGO_HIP(ctx, hipEventSynchronize(ctx->report_event[slot]));
-        const unsigned *h = static_cast<const unsigned *>(ctx->report) + 4 * slot;  // range, the last pass's list length
-        rc = pargo::check_launch(ctx, "pargo_pit_remove");
-        if (rc) return rc;
-        if (pass == 0) {
-            // monotonicity check: every valid W lies in [min(dem, 10000), 10000]
-            if (h[1])
-                return fail(ctx, PARGO_E_INVALID, "the DEM holds %u NaN cells: the reference never settles there", h[1]);
-            unsigned u = h[0];
-            u = (u & 0x80000000u) ? (u & 0x7fffffffu) : ~u;
-            float mn;
-            std::memcpy(&mn, &u, sizeof(mn));
-            // no valid cell leaves the smallest key's image at NaN
-            const bool any_valid = !std::isnan(mn);
-            const double lo = any_valid ? std::min((double)mn, 10000.0) : 0.0;
-            const bool ok = !any_valid || g->nodata < lo - 0.000001 || g->nodata > 10000.0 + 0.000001;
-            if (!ok)
+        for (;;) {
+            rc = launch(pass + kBatch);
+            if (rc) return rc;
+            const int slot = pass / kBatch & 1;
+            PARGO_HIP(ctx, hipEventSynchronize(ctx->report_event[slot]));
+            const unsigned *h = static_cast<const unsigned *>(ctx->report) + 4 * slot;  // range, the last pass's list length
+            rc = pargo::check_launch(ctx, "pargo_pit_remove");
+            if (rc) return rc;
+            if (pass == 0 && pargo::fill_refused(h[0], h[1], g->nodata)) {
+                if (h[1])
+                    return fail(ctx, PARGO_E_INVALID, "the DEM holds %u NaN cells: the reference never settles there", h[1]);
                 return fail(ctx, PARGO_E_UNSUPPORTED,
                             "NoData %.17g lies inside the range of filled values [%.17g, 10000]: the reference's "
                             "result would depend on its sweep order",
-                            g->nodata, lo);
+                            g->nodata, pargo::lowest_filled(h[0]));
+            }
+            pass += kBatch;
+            if (h[2] == 0) return PARGO_OK;  // the batch's last pass had nothing to do
+            if (pass >= kMaxPasses)
+                return fail(ctx, PARGO_E_NONTERM, "depression filling did not settle within %d passes", kMaxPasses);
         }
-        pass += kBatch;
-        if (h[2] == 0) break;  // the batch's last pass had nothing to do
-        if (pass >= kMaxPasses)
-            return fail(ctx, PARGO_E_NONTERM, "depression filling did not settle within %d passes", kMaxPasses);
+    };
+    rc = settle();
+    if (rc) {
+        // the passes of the batch ahead read the DEM and write the output:
+        // the caller gets both back only when they have ended
+        hipStreamSynchronize(ctx->stream);
+        return rc;
     }
+    // The batch ahead of the one that settled is not waited for: its lists are
+    // empty, so it touches the context's memory only (with the wait the
+    // 1501 x 2003 chain took 772 us instead of 731).
     if (passes_out) *passes_out = pass;
     return PARGO_OK;
 }
