@@ -267,7 +267,7 @@ int pargo_sca_d8(pargo_ctx *ctx, const pargo_grid *grid, const uint8_t *flow, co
  * or written any more, refusals and errors included (up to eight checks that
  * found nothing to do may still be queued on the stream; they touch the
  * context's own memory only).  *passes (host, may be NULL) receives the
- * number of device passes.
+ * number of device passes that had tiles to visit.
  * Working memory: the context's scratch grows to 528 bytes per
  * 64 x 32 tile (worklists, flags and a copy of each tile's edge columns)
  * plus 25 KB, kept until pargo_destroy.  A refused DEM leaves filled_out

@@ -107,7 +107,7 @@ struct FillParams {
     double *__restrict__ w;
     unsigned *__restrict__ flags;    // [2][tiles]: what the tile's next visit starts from (even, odd passes)
     unsigned *__restrict__ count;    // [3][kSub]: entries of the worklists (kSubStride apart), pass p's in set p % 3
-    unsigned *__restrict__ total;    // entries of the last pass that ran
+    unsigned *__restrict__ ran;      // passes that had tiles on their list
     int *__restrict__ list;          // [2][kSub][sub_cap]: tiles of the pass (even, odd)
     double *__restrict__ edge;       // [tiles][2][kTH]: W of each tile's first and last column, NoData as +infinity
     unsigned *__restrict__ range;    // [0] smallest valid elevation (ordered bits), [1] NaN cells
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(256) void fill_init_kernel(FillParams p)
     }
 }
 
-// Flags cleared, empty worklists and no range, before the init kernel.
+// Flags cleared, empty worklists, no range and no passes, before the init kernel.
 __global__ void fill_reset_kernel(FillParams p, int n)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
@@ -325,6 +325,7 @@ __global__ void fill_reset_kernel(FillParams p, int n)
     if (i == 0) {
         p.range[0] = 0xffffffffu;
         p.range[1] = 0;
+        *p.ran = 0;
     }
 }
 
@@ -595,7 +596,7 @@ __global__ __launch_bounds__(64 * (kTH / RW), RW == 8 ? 5 : 3) void fill_pass_ke
     if (blockIdx.x == 0 && threadIdx.x < kSub) {
         // the counters that pass + 1 fills (pass - 1 read them)
         p.count[((pass + 2) % 3) * kSetWords + lane * kSubStride] = 0;
-        if (lane == 0) *p.total = n;
+        if (lane == 0 && n != 0) *p.ran = (unsigned)pass + 1u;
     }
     // A fixed stride over the list, whose neighbours are tiles kSub apart.
     // The grid is what fits on the GPU at once, so no workgroup starts late
@@ -684,7 +685,7 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     const int ntiles = p.tiles_x * p.tiles_y;
     constexpr int kBatch = 8;      // passes between checks
     constexpr int kMaxPasses = 1 << 20;
-    // scratch: the range check's two words and the last list's length, the
+    // scratch: the range check's two words and the passes that had work, the
     // list counters, then the flags, the two worklists and the tiles' edge
     // columns
     const size_t counters = 64 + 3 * (size_t)pargo::kSetWords;
@@ -697,7 +698,7 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     if (rc) return rc;
     unsigned *scr = static_cast<unsigned *>(ctx->scratch);
     p.range = scr;
-    p.total = scr + 2;
+    p.ran = scr + 2;
     p.count = scr + 64;
     p.flags = scr + counters;
     p.list = reinterpret_cast<int *>(p.flags + 2 * (size_t)ntiles);
@@ -736,7 +737,7 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
         PARGO_HIP(ctx, hipEventRecord(ctx->report_event[slot], ctx->stream));
         return PARGO_OK;
     };
-    int pass = 0;
+    int pass = 0, ran = 0;
     auto settle = [&]() -> int {
         int rc = launch(0);
         if (rc) return rc;
@@ -745,7 +746,7 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
             if (rc) return rc;
             const int slot = pass / kBatch & 1;
             PARGO_HIP(ctx, hipEventSynchronize(ctx->report_event[slot]));
-            const unsigned *h = static_cast<const unsigned *>(ctx->report) + 4 * slot;  // range, the last pass's list length
+            const unsigned *h = static_cast<const unsigned *>(ctx->report) + 4 * slot;  // range, passes with work
             rc = pargo::check_launch(ctx, "pargo_pit_remove");
             if (rc) return rc;
             if (pass == 0 && pargo::fill_refused(h[0], h[1], g->nodata)) {
@@ -757,7 +758,8 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
                             g->nodata, pargo::lowest_filled(h[0]));
             }
             pass += kBatch;
-            if (h[2] == 0) return PARGO_OK;  // the batch's last pass had nothing to do
+            ran = (int)h[2];
+            if (ran < pass) return PARGO_OK;  // the batch's last pass had nothing to do
             if (pass >= kMaxPasses)
                 return fail(ctx, PARGO_E_NONTERM, "depression filling did not settle within %d passes", kMaxPasses);
         }
@@ -772,6 +774,6 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     // The batch ahead of the one that settled is not waited for: its lists are
     // empty, so it touches the context's memory only (with the wait the
     // 1501 x 2003 chain took 772 us instead of 731).
-    if (passes_out) *passes_out = pass;
+    if (passes_out) *passes_out = ran;
     return PARGO_OK;
 }

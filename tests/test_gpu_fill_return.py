@@ -66,3 +66,18 @@ def test_no_valid_cell_is_accepted_whatever_nodata():
     z = np.full((40, 70), 500.0, np.float32)
     got, _ = gpu_fill(z, 500.0)
     assert (got == 500.0).all()
+
+
+def test_the_passes_reported_are_those_that_had_tiles():
+    z = (100 + np.add.outer(np.arange(30), np.arange(60)) * 0.5).astype(np.float32)
+    _, passes = gpu_fill(z)
+    assert passes == 1  # one tile, and none beside it to schedule
+    # a basin over two tiles with its outlet in the left one: what the right
+    # tile settles to waits for the left one, so the first pass is not the last
+    z = np.full((32, 128), 10001.0, np.float32)
+    z[3:-3, 3:-3] = 50.0
+    z[10, 5] = ND
+    ref, _, ok = pyoracle.pit_remove(z, ND)
+    assert ok
+    got, passes = gpu_fill(z)
+    assert np.array_equal(got, ref) and 2 <= passes < 8, passes
