@@ -179,7 +179,13 @@ typedef struct {
  * pargo_slope_d8 calls bit for bit, except that a batch holding a tile whose
  * cell size is outside [2^-20, 2^40] takes the generic FP64 Horn path for
  * every tile: then the other tiles' slopes are within 1e-5 of pargo_slope_d8
- * (which takes the FP32-root path for them) and their D8 codes identical. */
+ * (which takes the FP32-root path for them) and their D8 codes identical.
+ * On a stream that the caller is capturing, a batch that was run once before
+ * goes into the caller's graph, in every mode (a first run is refused with
+ * PARGO_E_DEVICE and leaves the capture intact).  The device memory such a
+ * graph reads stays its own until pargo_destroy, whatever runs on the context
+ * meanwhile; a replay uses the context like a run, so it is ordered with the
+ * context's other work and ends before pargo_destroy. */
 int pargo_batch_slope_d8(pargo_ctx *ctx, const pargo_tile *tiles, int ntiles, int method, int unit, int dirtype,
                          int mode);
 

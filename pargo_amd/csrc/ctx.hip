@@ -209,6 +209,7 @@ int pargo_destroy(pargo_ctx *ctx)
         if (e) hipEventDestroy(e);
     pargo::free_batch_plan(ctx);
     pargo::free_batch_mem(ctx);
+    pargo::free_captured_batch_mem(ctx);
     if (ctx->fix_mem) hipFree(ctx->fix_mem);
     if (ctx->switch_event) hipEventDestroy(ctx->switch_event);
     if (ctx->own_stream) hipStreamDestroy(ctx->own_stream);

@@ -1258,6 +1258,7 @@ struct BatchPlan {
     int cpt = 4;
     int blocks = 0;
     bool do_slope = false, do_d8 = false;
+    bool captured = false;  // a caller's graph holds its launches
     int sm = 0;  // slope mode shared by every tile (slope_mode)
     unsigned long long runs = 0;  // graph runs so far
     hipGraphExec_t exec = nullptr;
@@ -1287,6 +1288,12 @@ void free_batch_mem(pargo_ctx *ctx)
     }
     ctx->batch_mem = ctx->batch_host = nullptr;
     ctx->batch_mem_bytes = 0;
+}
+
+void free_captured_batch_mem(pargo_ctx *ctx)
+{
+    for (void *m : ctx->batch_captured) hipFree(m);
+    ctx->batch_captured.clear();
 }
 
 template <int CPT, bool DO_SLOPE, int DO_D8, int SM>
@@ -1356,17 +1363,20 @@ static void enqueue_batch(const BatchPlan &b, hipStream_t s)
     launch_fixup(b.h_tiles[0], b.d_tiles, b.ntiles, b.do_slope, b.do_d8, b.cpt, s, b.d_queue);
 }
 
+static int is_capturing(pargo_ctx *ctx, bool *capturing)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    PARGO_HIP(ctx, hipStreamIsCapturing(ctx->stream, &status));
+    *capturing = status != hipStreamCaptureStatusNone;
+    return PARGO_OK;
+}
+
 // The device copy of the batch plan and two page-locked host copies, kept by
 // the context: a new plan is uploaded in stream order behind the runs of the
 // one before, with no allocation and no wait (each host copy is written again
 // only when its last upload has been made).
 static int ensure_batch_mem(pargo_ctx *ctx, size_t bytes, unsigned char **host)
 {
-    // a captured upload would read the host copy at every replay
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    PARGO_HIP(ctx, hipStreamIsCapturing(ctx->stream, &capturing));
-    if (capturing != hipStreamCaptureStatusNone)
-        return fail(ctx, PARGO_E_DEVICE, "a batch's first run cannot be captured: run it once before");
     if (ctx->batch_mem_bytes < bytes) {
         hipError_t e = hipStreamSynchronize(ctx->stream);  // the old copies may be in use
         if (e != hipSuccess) return fail(ctx, PARGO_E_DEVICE, "hipStreamSynchronize: %s", hipGetErrorString(e));
@@ -1402,8 +1412,15 @@ static int build_batch(pargo_ctx *ctx, const pargo_tile *tiles, int ntiles, int 
         *out = ctx->batch;
         return PARGO_OK;
     }
+    // A captured upload would read the host copy at every replay.  Asked
+    // before anything is waited for or dropped, so that the caller's capture
+    // and the context's plan outlive the refusal.
+    bool capturing = false;
+    int rc = is_capturing(ctx, &capturing);
+    if (rc) return rc;
+    if (capturing) return fail(ctx, PARGO_E_DEVICE, "a batch's first run cannot be captured: run it once before");
     free_batch_plan(ctx);
-    int rc = ensure_fixup(ctx);
+    rc = ensure_fixup(ctx);
     if (rc) return rc;
     alloc_point("batch plan (host)");
     BatchPlan *b = new (std::nothrow) BatchPlan();
@@ -1511,9 +1528,25 @@ static int batch_rows(const pargo_ctx *ctx, const pargo_tile *tiles, int ntiles)
     return strip_rows_of(work, 32);
 }
 
+// A caller's graph that takes a plan's launches reads the plan's device copy
+// at every replay: that copy is the plan's own from then on, neither written
+// for another plan nor freed before the context is destroyed.
+static void keep_for_capture(pargo_ctx *ctx, BatchPlan *b)
+{
+    if (b->captured) return;
+    ctx->batch_captured.push_back(ctx->batch_mem);
+    ctx->batch_mem = nullptr;
+    ctx->batch_mem_bytes = 0;  // the next plan gets memory of its own
+    b->captured = true;
+}
+
 static int run_batch(pargo_ctx *ctx, BatchPlan *b, int mode, int rows_per_strip)
 {
     const hipStream_t s = ctx->stream;
+    bool capturing = false;
+    const int rc = is_capturing(ctx, &capturing);
+    if (rc) return rc;
+    if (capturing && mode != PARGO_BATCH_PER_TILE) keep_for_capture(ctx, b);
     if (mode == PARGO_BATCH_PER_TILE) {
         LaunchCfg cfg{b->cpt, rows_per_strip};
         for (int t = 0; t < b->ntiles; t++) {
@@ -1531,9 +1564,7 @@ static int run_batch(pargo_ctx *ctx, BatchPlan *b, int mode, int rows_per_strip)
     // is worth the capture (about 60 us).  So is a run on a stream that the
     // caller is capturing: its launches go into the caller's graph (a graph
     // launched there would not).
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    PARGO_HIP(ctx, hipStreamIsCapturing(s, &capturing));
-    if (b->runs++ == 0 || capturing != hipStreamCaptureStatusNone) {
+    if (b->runs++ == 0 || capturing) {
         enqueue_batch(*b, s);
         return check_launch(ctx, "pargo_batch_slope_d8 (graph)");
     }

@@ -43,6 +43,7 @@ struct pargo_ctx {
     size_t batch_mem_bytes = 0;
     hipEvent_t batch_copied[2] = {nullptr, nullptr};  // each host copy's last upload
     int batch_slot = 0;
+    std::vector<void *> batch_captured;  // device copies of plans that callers' graphs hold
     int batch_cpt = 4;
     int batch_rows = 32;  // once batch_tuned; by the batch's size before
     int batch_tuned = 0;
@@ -55,6 +56,7 @@ struct pargo_ctx {
 namespace pargo {
 void free_batch_plan(pargo_ctx *ctx);
 void free_batch_mem(pargo_ctx *ctx);
+void free_captured_batch_mem(pargo_ctx *ctx);
 // Resolves ctx->noalloc_scratch with ctx->device current.
 int resolve_noalloc_scratch(pargo_ctx *ctx);
 }
