@@ -1,5 +1,5 @@
-// faults.h -- allocation-failure injection and the exception guard of the
-// C ABI (host code only; not part of the C ABI).
+// faults.h -- allocation- and launch-failure injection and the exception
+// guard of the C ABI (host code only; not part of the C ABI).
 //
 // PARGO_FAIL_ALLOC="<n>" (or "<n>:<tag>", the tag only making a new value)
 // makes the n-th allocation point the library reaches, counted from 1 since
@@ -9,6 +9,11 @@
 // walk n = 1, 2, ... over an entry point's allocations and check that each
 // failure is reported and leaves the context usable.  Unset (the normal
 // case), a point costs one getenv.
+//
+// PARGO_FAIL_LAUNCH="<n>" (or "<n>:<tag>") likewise makes the n-th launch of
+// a pass that empties a device queue fail: the queue is then left as the
+// launch before it filled it, which the call reports as PARGO_E_DEVICE and a
+// later call must not see.
 #pragma once
 
 #include <cstddef>
@@ -23,6 +28,9 @@ int fail(pargo_ctx *ctx, int code, const char *fmt, ...);
 
 // True when this allocation point is the one PARGO_FAIL_ALLOC selects.
 bool alloc_should_fail(const char *site);
+
+// True when this launch is the one PARGO_FAIL_LAUNCH selects.
+bool launch_should_fail(const char *site);
 
 // A host allocation point: throws std::bad_alloc when selected.
 inline void alloc_point(const char *site)

@@ -1009,14 +1009,26 @@ static void launch_t(const FocalParams &p, const LaunchCfg &cfg, bool vec, hipSt
     }
 }
 
-static void launch_fixup(const FocalParams &p, const FocalParams *tiles, int ntiles, bool do_slope, bool do_d8,
-                         int cpt, hipStream_t s, unsigned *items = nullptr)
+static hipError_t launch_fixup(const FocalParams &p, const FocalParams *tiles, int ntiles, bool do_slope, bool do_d8,
+                               int cpt, hipStream_t s, unsigned *items = nullptr)
 {
+    if (launch_should_fail("fixup pass")) return hipErrorLaunchFailure;
     dim3 block(256), grid(kFixupBlocks);
     const int width = 64 * cpt;
     if (do_slope && do_d8) hipLaunchKernelGGL((focal_fixup_kernel<true, true>), grid, block, 0, s, p, tiles, ntiles, width, items);
     else if (do_slope) hipLaunchKernelGGL((focal_fixup_kernel<true, false>), grid, block, 0, s, p, tiles, ntiles, width, items);
     else hipLaunchKernelGGL((focal_fixup_kernel<false, true>), grid, block, 0, s, p, tiles, ntiles, width, items);
+    return hipSuccess;
+}
+
+// The outcome of launches that fill the fixup queue and empty it again: after
+// a failure the queue may hold entries, which the next call clears.
+static int queue_launched(pargo_ctx *ctx, hipError_t e, const char *name)
+{
+    const int rc = e == hipSuccess ? check_launch(ctx, name)
+                                   : fail(ctx, PARGO_E_DEVICE, "%s: %s%s", name, hipGetErrorString(e), injected_note());
+    if (rc) ctx->fix_stale = true;
+    return rc;
 }
 
 // Slope mode of the kernels: 1 the Horn fast path (FD), 2 the other
@@ -1074,11 +1086,26 @@ static LaunchCfg default_cfg(int rows, int cols)
     return c;
 }
 
-// The fixup queue: two counters and kFixupCap strip entries, zeroed once at
-// allocation; every fixup launch leaves the counters at zero again.
+// Zeroes the two queue counters (a kernel rather than a memset, so that a
+// caller may capture the call in a HIP graph).
+__global__ void fixup_counters_reset(unsigned *c)
+{
+    c[0] = 0;
+    c[1] = 0;
+}
+
+// The fixup queue: two counters and kFixupCap strip entries, zeroed at
+// allocation and after a failed launch; every fixup launch leaves the
+// counters at zero again.
 static int ensure_fixup(pargo_ctx *ctx)
 {
-    if (ctx->fix_mem) return PARGO_OK;
+    if (ctx->fix_mem) {
+        if (!ctx->fix_stale) return PARGO_OK;
+        hipLaunchKernelGGL(fixup_counters_reset, dim3(1), dim3(1), 0, ctx->stream, (unsigned *)ctx->fix_mem);
+        const int rc = check_launch(ctx, "fixup queue reset");
+        if (!rc) ctx->fix_stale = false;
+        return rc;
+    }
     const size_t bytes = 64 * sizeof(unsigned) + (size_t)kFixupCap * sizeof(uint4);
     hipError_t e = dev_malloc(&ctx->fix_mem, bytes, "fixup queue");
     if (e != hipSuccess)
@@ -1117,14 +1144,6 @@ int resolve_noalloc_scratch(pargo_ctx *ctx)
                     ctx->device, hipGetErrorString(e));
     ctx->noalloc_scratch = ptr;
     return PARGO_OK;
-}
-
-// Zeroes the two queue counters (a kernel rather than a memset, so that a
-// caller may capture the call in a HIP graph).
-__global__ void fixup_counters_reset(unsigned *c)
-{
-    c[0] = 0;
-    c[1] = 0;
 }
 
 // Validates the request and fills the kernel parameters.
@@ -1239,10 +1258,9 @@ static int run_focal(pargo_ctx *ctx, const pargo_grid *g, const float *dem, int 
     }
     if (in_wave) p.fix_count = nullptr;
     launch_focal(p, cfg, vec, do_slope, do_d8, ctx->stream);
-    rc = check_launch(ctx, name);
+    rc = in_wave ? check_launch(ctx, name) : queue_launched(ctx, hipSuccess, name);
     if (rc || in_wave) return rc;
-    launch_fixup(p, nullptr, 1, do_slope, do_d8, cfg.cpt, ctx->stream);
-    return check_launch(ctx, name);
+    return queue_launched(ctx, launch_fixup(p, nullptr, 1, do_slope, do_d8, cfg.cpt, ctx->stream), name);
 }
 
 // ---- batches ------------------------------------------------------------
@@ -1356,11 +1374,23 @@ static int blocks_c(pargo_ctx *ctx, const BatchPlan &b)
 
 // The persistent sequence: batch kernel, fixup (which leaves the item queue
 // at zero again, as the plan's upload does at first).
-static void enqueue_batch(const BatchPlan &b, hipStream_t s)
+static hipError_t enqueue_batch(const BatchPlan &b, hipStream_t s)
 {
     if (b.cpt == 2) launch_batch_c<2>(b, s);
     else launch_batch_c<4>(b, s);
-    launch_fixup(b.h_tiles[0], b.d_tiles, b.ntiles, b.do_slope, b.do_d8, b.cpt, s, b.d_queue);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return launch_fixup(b.h_tiles[0], b.d_tiles, b.ntiles, b.do_slope, b.do_d8, b.cpt, s, b.d_queue);
+}
+
+// The outcome of a run's launches.  After a failure the item queue may not
+// stand at zero either, and the next run would skip items: without its key
+// the plan is built and uploaded anew.
+static int batch_launched(pargo_ctx *ctx, BatchPlan *b, hipError_t e, const char *name)
+{
+    const int rc = queue_launched(ctx, e, name);
+    if (rc) b->key.clear();
+    return rc;
 }
 
 static int is_capturing(pargo_ctx *ctx, bool *capturing)
@@ -1410,7 +1440,7 @@ static int build_batch(pargo_ctx *ctx, const pargo_tile *tiles, int ntiles, int 
     std::memcpy(key.data() + sizeof(pargo_tile) * (size_t)ntiles, extra, sizeof(extra));
     if (ctx->batch && ctx->batch->key == key) {
         *out = ctx->batch;
-        return PARGO_OK;
+        return ensure_fixup(ctx);
     }
     // A captured upload would read the host copy at every replay.  Asked
     // before anything is waited for or dropped, so that the caller's capture
@@ -1549,25 +1579,22 @@ static int run_batch(pargo_ctx *ctx, BatchPlan *b, int mode, int rows_per_strip)
     if (capturing && mode != PARGO_BATCH_PER_TILE) keep_for_capture(ctx, b);
     if (mode == PARGO_BATCH_PER_TILE) {
         LaunchCfg cfg{b->cpt, rows_per_strip};
-        for (int t = 0; t < b->ntiles; t++) {
+        hipError_t e = hipSuccess;
+        for (int t = 0; t < b->ntiles && e == hipSuccess; t++) {
             const FocalParams &p = b->h_tiles[t];
             launch_focal_h(p, cfg, p.vec != 0, b->do_slope, b->do_d8, b->sm, s);
-            launch_fixup(p, nullptr, 1, b->do_slope, b->do_d8, b->cpt, s);
+            e = launch_fixup(p, nullptr, 1, b->do_slope, b->do_d8, b->cpt, s);
         }
-        return check_launch(ctx, "pargo_batch_slope_d8 (per tile)");
+        return queue_launched(ctx, e, "pargo_batch_slope_d8 (per tile)");
     }
-    if (mode == PARGO_BATCH_PERSISTENT) {
-        enqueue_batch(*b, s);
-        return check_launch(ctx, "pargo_batch_slope_d8 (persistent)");
-    }
+    if (mode == PARGO_BATCH_PERSISTENT)
+        return batch_launched(ctx, b, enqueue_batch(*b, s), "pargo_batch_slope_d8 (persistent)");
     // The first run of a plan is launched as it is; a batch that is run again
     // is worth the capture (about 60 us).  So is a run on a stream that the
     // caller is capturing: its launches go into the caller's graph (a graph
     // launched there would not).
-    if (b->runs++ == 0 || capturing) {
-        enqueue_batch(*b, s);
-        return check_launch(ctx, "pargo_batch_slope_d8 (graph)");
-    }
+    if (b->runs++ == 0 || capturing)
+        return batch_launched(ctx, b, enqueue_batch(*b, s), "pargo_batch_slope_d8 (graph)");
     if (!b->exec) {
         // capture on a private stream so that a caller's legacy default
         // stream can be used for everything else
@@ -1575,15 +1602,16 @@ static int run_batch(pargo_ctx *ctx, BatchPlan *b, int mode, int rows_per_strip)
         PARGO_HIP(ctx, hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
         hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
         if (e == hipSuccess) {
-            enqueue_batch(*b, cs);
-            e = hipStreamEndCapture(cs, &b->graph);
+            e = enqueue_batch(*b, cs);
+            const hipError_t ended = hipStreamEndCapture(cs, &b->graph);
+            if (e == hipSuccess) e = ended;
         }
         if (e == hipSuccess) e = hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0);
         hipStreamDestroy(cs);
-        if (e != hipSuccess) return fail(ctx, PARGO_E_DEVICE, "capturing the batch graph: %s", hipGetErrorString(e));
+        if (e != hipSuccess) return batch_launched(ctx, b, e, "capturing the batch graph");
     }
-    PARGO_HIP(ctx, hipGraphLaunch(b->exec, s));
-    return PARGO_OK;
+    const hipError_t e = hipGraphLaunch(b->exec, s);
+    return e == hipSuccess ? PARGO_OK : batch_launched(ctx, b, e, "pargo_batch_slope_d8 (graph)");
 }
 
 }  // namespace pargo
@@ -1717,7 +1745,7 @@ static int batch_order(pargo_ctx *ctx, const pargo_tile *tiles, int ntiles, int 
             const pargo::FocalParams &p = b->h_tiles[t];
             e = hipEventRecord(ev[2 * t], ctx->stream);
             pargo::launch_focal_h(p, cfg, p.vec != 0, b->do_slope, b->do_d8, b->sm, ctx->stream);
-            pargo::launch_fixup(p, nullptr, 1, b->do_slope, b->do_d8, b->cpt, ctx->stream);
+            if (e == hipSuccess) e = pargo::launch_fixup(p, nullptr, 1, b->do_slope, b->do_d8, b->cpt, ctx->stream);
             if (e == hipSuccess) e = hipEventRecord(ev[2 * t + 1], ctx->stream);
         }
         if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -1729,7 +1757,7 @@ static int batch_order(pargo_ctx *ctx, const pargo_tile *tiles, int ntiles, int 
         }
         for (hipEvent_t x : ev)
             if (x) hipEventDestroy(x);
-        if (e != hipSuccess) return pargo::fail(ctx, PARGO_E_DEVICE, "timing the batch tiles: %s", hipGetErrorString(e));
+        if (e != hipSuccess) return pargo::queue_launched(ctx, e, "timing the batch tiles");
         ctx->batch_load = std::move(load);
     }
     ctx->batch_order = source;
