@@ -252,7 +252,10 @@ int pargo_d8_classify(pargo_ctx *ctx, const pargo_grid *grid, const double *d8, 
  * inflows to NoData; PARGO_SCA_CONVERGE gives the area that repeated sweeps
  * converge to (full D8 flow accumulation).  grid->cellsize is unused.
  * Working memory: the context's scratch grows to 6784 bytes per 64 x 32 tile
- * (3.3 bytes per cell) plus 256 bytes, kept until pargo_destroy. */
+ * (3.3 bytes per cell of a full tile), in rasters of at most 32 columns or 16
+ * rows to at most 3 bytes per cell of whole tiles as wide or high as the
+ * raster, plus 256 bytes; kept until pargo_destroy.  Grids of more than 2^24
+ * tiles (34 Gcells of full ones) are refused with PARGO_E_INVALID. */
 int pargo_sca_d8(pargo_ctx *ctx, const pargo_grid *grid, const uint8_t *flow, const uint32_t *nodata_mask,
                  int mode, double *sca_out);
 

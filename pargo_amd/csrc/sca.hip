@@ -70,6 +70,7 @@
 // DEM, whose paths are long.  One walk over the whole raster with a global
 // atomic or a static word read per hop (33 bytes of HBM traffic, up to 1336
 // hops in a row) took 4.24, 1.21 and 1.15 ms.
+#include <algorithm>
 #include <cmath>
 
 #include "internal.h"
@@ -139,7 +140,33 @@ struct ScaParams {
     int tiles_x, ntiles;
     int converge;
     double nodata;
+    int w, h, slots;  // NARROW: cells and slots a tile has memory for
 };
+
+// Memory of a raster that is one column (of at most 32 cells) or one row (of
+// at most 16) of tiles: at a full tile's 6784 bytes a raster of one column
+// would take 212 bytes a cell.  Such a raster keeps static words for the
+// cells a tile holds and slots for the sides that have a tile beyond them
+// only, 2.4 to 2.9 bytes a cell; its kernels (NARROW) are the same but for
+// the addresses.
+constexpr int kNarrowCols = kTileC / 2, kNarrowRows = kTileR / 2;
+template <bool NARROW>
+__device__ __forceinline__ unsigned slot_stride(const ScaParams &p) { return NARROW ? (unsigned)p.slots : (unsigned)kSlotStride; }
+// A perimeter cell's slot in memory; of the sides without a tile beyond them
+// none is asked for.
+template <bool NARROW>
+__device__ __forceinline__ unsigned mem_slot(const ScaParams &p, int r, int c)
+{
+    if (!NARROW) return (unsigned)slot_of(r, c);
+    return (unsigned)(p.tiles_x == 1 ? (r == 0 ? c : p.w + c) : (c == 0 ? r : p.h + r));
+}
+// Whether a perimeter cell has one (all of a full tile's have).
+template <bool NARROW>
+__device__ __forceinline__ bool has_slot(const ScaParams &p, int r, int c)
+{
+    if (!NARROW) return true;
+    return p.tiles_x == 1 ? (r == 0 || r == kTileR - 1) && c < p.w : (c == 0 || c == kTileC - 1) && r < p.h;
+}
 
 __device__ __forceinline__ unsigned npend_of(unsigned s) { return s & 15u; }
 __device__ __forceinline__ unsigned nsrc_of(unsigned s) { return (s >> 4) & 15u; }
@@ -422,6 +449,7 @@ union LocalShared {
     unsigned acc[kTileN];  // once the static words are formed
 };
 
+template <bool NARROW>
 __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
 {
     __shared__ LocalShared S;
@@ -440,7 +468,7 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
     if (inner) swar_words(p, S.swar, stw, r0, c0);
     else general_words(p, S.general, stw, r0, c0);
     __syncthreads();
-    const unsigned long long slot0 = (unsigned long long)tile * kSlotStride;
+    const unsigned long long slot0 = (unsigned long long)tile * slot_stride<NARROW>(p);
     // the pending inflows of this thread's perimeter cell from outside the tile
     const int pcell = tid < kSlots ? cell_of_slot(tid) : 0;
     unsigned ext = 0;
@@ -466,8 +494,13 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
     const unsigned next_ = (unsigned)__builtin_popcount(ext);
     // the static words go out as they are; the tile keeps them with the
     // awaited inflows from inside only
-    const uint4 words = *reinterpret_cast<const uint4 *>(stw + 8 * tid);
-    *reinterpret_cast<uint4 *>(p.st + (long long)tile * kTileN + 8 * tid) = words;
+    if constexpr (NARROW) {
+        for (int i = tid; i < kTileN; i += 256)
+            if ((i >> 6) < p.h && (i & 63) < p.w) p.st[((long long)tile * p.h + (i >> 6)) * p.w + (i & 63)] = stw[i];
+    } else {
+        const uint4 words = *reinterpret_cast<const uint4 *>(stw + 8 * tid);
+        *reinterpret_cast<uint4 *>(p.st + (long long)tile * kTileN + 8 * tid) = words;
+    }
     unsigned s[kTileN / 256];
 #pragma unroll
     for (int k = 0; k < kTileN / 256; k++) {
@@ -509,10 +542,19 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
         const unsigned slot = entry[i];
         unsigned t = (unsigned)cell_of_slot((int)slot);
         for (int n = 0; n < kTileN && t < kLeaves; n++) t = nxt[t];
-        p.link[slot0 + slot] = (uint8_t)(t >= kLeaves && t != kEnds ? t - kLeaves : 255u);
+        unsigned at = slot, exit = t >= kLeaves && t != kEnds ? t - kLeaves : 255u;
+        if constexpr (NARROW) {
+            const int in = cell_of_slot((int)slot);
+            at = mem_slot<NARROW>(p, in >> 6, in & 63);
+            if (exit != 255u) {
+                const int out = cell_of_slot((int)exit);
+                exit = mem_slot<NARROW>(p, out >> 6, out & 63);
+            }
+        }
+        p.link[slot0 + at] = (uint8_t)exit;
     }
     __syncthreads();
-    if (tid < kSlotStride) {
+    if (NARROW ? tid < kSlots && has_slot<NARROW>(p, pcell >> 6, pcell & 63) : tid < kSlotStride) {
         unsigned long long x = kExitNever;
         unsigned to = kNoExit;
         if (tid < kSlots) {
@@ -521,7 +563,7 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
             if (t >= kLeaves && t != kEnds) {
                 const int gr = r0 + (pcell >> 6) + k / 3 - 1, gc = c0 + (pcell & 63) + k % 3 - 1;
                 const int beside = (gr / kTileR) * p.tiles_x + gc / kTileC;
-                to = (unsigned)beside * kSlotStride + (unsigned)slot_of(gr % kTileR, gc % kTileC);
+                to = (unsigned)beside * slot_stride<NARROW>(p) + mem_slot<NARROW>(p, gr % kTileR, gc % kTileC);
                 if ((v >> kLocPend) == 0) {
                     const unsigned n = (v >> kLocExt) & 255u;
                     if ((v >> kLocBad) & 15u) x = kExitStart | (1ull << kExitBad);  // not done, whatever arrives
@@ -529,15 +571,17 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
                 }
             }
         }
-        p.exits[slot0 + tid] = x;
-        p.next[slot0 + tid] = to;
-        p.ext[slot0 + tid] = (uint8_t)ext;
+        const unsigned at = NARROW ? mem_slot<NARROW>(p, pcell >> 6, pcell & 63) : (unsigned)tid;
+        p.exits[slot0 + at] = x;
+        p.next[slot0 + at] = to;
+        p.ext[slot0 + at] = (uint8_t)ext;
     }
 }
 
 // Each exit's successor: the exit that the perimeter cell it enters leads
 // to, none if that one awaits nothing (it is not done whatever arrives) or
 // never completes.
+template <bool NARROW>
 __global__ __launch_bounds__(256) void sca_link_kernel(ScaParams p, unsigned n)
 {
     const unsigned i = blockIdx.x * 256u + threadIdx.x;
@@ -547,7 +591,7 @@ __global__ __launch_bounds__(256) void sca_link_kernel(ScaParams p, unsigned n)
     const unsigned slot = p.link[to];
     unsigned x = kNoExit;
     if (slot != 255u) {
-        x = to / kSlotStride * kSlotStride + slot;
+        x = to / slot_stride<NARROW>(p) * slot_stride<NARROW>(p) + slot;
         const unsigned pend = (unsigned)(p.exits[x] >> kExitPend) & 255u;
         if (pend == 0 || pend == 255u) x = kNoExit;
     }
@@ -596,6 +640,7 @@ __global__ __launch_bounds__(256) void sca_cross_kernel(ScaParams p, unsigned n)
     }
 }
 
+template <bool NARROW>
 __global__ __launch_bounds__(256) void sca_final_kernel(ScaParams p)
 {
     __shared__ unsigned long long acc[kTileN];
@@ -607,21 +652,27 @@ __global__ __launch_bounds__(256) void sca_final_kernel(ScaParams p)
     if (tid == 0) starts.n = 0;
     const int ty = tile / p.tiles_x, tx = tile - ty * p.tiles_x;
     const int r0 = ty * kTileR, c0 = tx * kTileC;
-    const uint4 words = *reinterpret_cast<const uint4 *>(p.st + (long long)tile * kTileN + 8 * tid);
+    uint4 words;
+    if constexpr (!NARROW) words = *reinterpret_cast<const uint4 *>(p.st + (long long)tile * kTileN + 8 * tid);
     const int pcell = tid < kSlots ? cell_of_slot(tid) : 0;
     // What arrives at this thread's perimeter cell from outside.  The words
     // of its first three inflows are all requested before one is looked at;
     // more than three drain only into a few corners.
-    const unsigned long long slot0 = (unsigned long long)tile * kSlotStride;
-    const unsigned ext = tid < kSlots ? p.ext[slot0 + tid] : 0u;
-    const unsigned pword = tid < kSlots ? p.st[(long long)tile * kTileN + pcell] : 0u;
+    const unsigned long long slot0 = (unsigned long long)tile * slot_stride<NARROW>(p);
+    auto static_word = [&](int i) -> unsigned {  // of cell i of the tile
+        if constexpr (!NARROW) return p.st[(long long)tile * kTileN + i];
+        return (i >> 6) < p.h && (i & 63) < p.w ? p.st[((long long)tile * p.h + (i >> 6)) * p.w + (i & 63)] : 0u;
+    };
+    const unsigned mine = NARROW ? mem_slot<NARROW>(p, pcell >> 6, pcell & 63) : (unsigned)tid;
+    const unsigned ext = tid < kSlots && has_slot<NARROW>(p, pcell >> 6, pcell & 63) ? p.ext[slot0 + mine] : 0u;
+    const unsigned pword = tid < kSlots ? static_word(pcell) : 0u;
     unsigned long long arrived = 0;
     if (ext) {
         auto word = [&](unsigned e) -> unsigned long long {  // of the lowest inflow in e
             const unsigned k = (unsigned)win_of_bit(__builtin_ctz(e));
             const unsigned gr = (unsigned)(r0 + (pcell >> 6) - 1) + k / 3u, gc = (unsigned)(c0 + (pcell & 63) - 1) + k % 3u;
-            return p.exits[(unsigned long long)((gr / kTileR) * (unsigned)p.tiles_x + gc / kTileC) * kSlotStride +
-                           (unsigned)slot_of((int)(gr % kTileR), (int)(gc % kTileC))];
+            return p.exits[(unsigned long long)((gr / kTileR) * (unsigned)p.tiles_x + gc / kTileC) * slot_stride<NARROW>(p) +
+                           mem_slot<NARROW>(p, (int)(gr % kTileR), (int)(gc % kTileC))];
         };
         auto arrival = [&](unsigned long long x) -> unsigned long long {
             if (((x >> kExitPend) & 255ull) != 0) return 0;  // never complete
@@ -639,7 +690,11 @@ __global__ __launch_bounds__(256) void sca_final_kernel(ScaParams p)
 #pragma unroll
         for (int q = 0; q < 3; q++) arrived += arrival(x[q]);
     }
-    *reinterpret_cast<uint4 *>(nxt + 8 * tid) = words;
+    if constexpr (NARROW) {
+        for (int i = tid; i < kTileN; i += 256) nxt[i] = (uint16_t)static_word(i);
+    } else {
+        *reinterpret_cast<uint4 *>(nxt + 8 * tid) = words;
+    }
     __syncthreads();
     unsigned s[kTileN / 256];
 #pragma unroll
@@ -762,6 +817,17 @@ bool sca_nodata_ok(double nodata)
     return true;
 }
 
+template <bool NARROW>
+void launch_sca(const ScaParams &p, unsigned n, hipStream_t s)
+{
+    const dim3 tiles(8 * (unsigned)((p.ntiles + 7) / 8)), threads(256);
+    constexpr unsigned per = 256u * kCrossPer;
+    hipLaunchKernelGGL(sca_local_kernel<NARROW>, tiles, threads, 0, s, p);
+    hipLaunchKernelGGL(sca_link_kernel<NARROW>, dim3((n + 255u) / 256u), threads, 0, s, p, n);
+    hipLaunchKernelGGL(sca_cross_kernel, dim3((n + per - 1) / per), threads, 0, s, p, n);
+    hipLaunchKernelGGL(sca_final_kernel<NARROW>, tiles, threads, 0, s, p);
+}
+
 }  // namespace
 
 }  // namespace pargo
@@ -814,22 +880,26 @@ extern "C" int pargo_sca_d8(pargo_ctx *ctx, const pargo_grid *g, const uint8_t *
     if (ntiles > (1ll << 24))
         return fail(ctx, PARGO_E_INVALID, "grid of %d x %d cells needs %lld tiles, more than 2^24", g->rows, g->cols,
                     ntiles);
-    // scratch: the last-cell flags, then per tile the static words (2 bytes
-    // per cell) and, per perimeter slot, the exit word, its successor, the
-    // entry's exit and its inflows from outside
+    pargo::ScaParams p{};
+    const bool narrow = g->cols <= pargo::kNarrowCols || g->rows <= pargo::kNarrowRows;
+    p.w = narrow ? std::min(g->cols, pargo::kTileC) : pargo::kTileC;
+    p.h = narrow ? std::min(g->rows, pargo::kTileR) : pargo::kTileR;
+    p.slots = !narrow ? pargo::kSlotStride : 2 * (tiles_x == 1 ? p.w : p.h);
+    // scratch: the last-cell flags, the exit words of the perimeter slots, the
+    // tiles' static words (2 bytes per cell, an even number of them) and, per
+    // slot again, its successor, the entry's exit and its inflows from outside
     constexpr size_t head = 256;
-    const size_t slots = (size_t)ntiles * pargo::kSlotStride;
-    rc = pargo::ensure_scratch(ctx, head + (size_t)ntiles * pargo::kTileN * sizeof(uint16_t) + slots * (8 + 4 + 1 + 1));
+    const size_t slots = (size_t)ntiles * p.slots, cells = ((size_t)ntiles * p.w * p.h + 1) & ~(size_t)1;
+    rc = pargo::ensure_scratch(ctx, head + cells * sizeof(uint16_t) + slots * (8 + 4 + 1 + 1));
     if (rc) return rc;
     char *scr = static_cast<char *>(ctx->scratch);
-    pargo::ScaParams p{};
     p.flow = flow;
     p.mask = nodata_mask;
     p.area = sca_out;
     p.last_done = reinterpret_cast<unsigned *>(scr);
     p.exits = reinterpret_cast<unsigned long long *>(scr + head);
     p.st = reinterpret_cast<uint16_t *>(p.exits + slots);
-    p.next = reinterpret_cast<unsigned *>(p.st + (size_t)ntiles * pargo::kTileN);
+    p.next = reinterpret_cast<unsigned *>(p.st + cells);
     p.link = reinterpret_cast<uint8_t *>(p.next + slots);
     p.ext = p.link + slots;
     p.pitch = pitch;
@@ -840,13 +910,8 @@ extern "C" int pargo_sca_d8(pargo_ctx *ctx, const pargo_grid *g, const uint8_t *
     p.ntiles = (int)ntiles;
     p.converge = mode == PARGO_SCA_CONVERGE;
     p.nodata = g->nodata;
-    const dim3 tiles(8 * (unsigned)((ntiles + 7) / 8)), threads(256);
-    const unsigned n = (unsigned)slots;
-    hipLaunchKernelGGL(pargo::sca_local_kernel, tiles, threads, 0, ctx->stream, p);
-    hipLaunchKernelGGL(pargo::sca_link_kernel, dim3((n + 255u) / 256u), threads, 0, ctx->stream, p, n);
-    constexpr unsigned per = 256u * pargo::kCrossPer;
-    hipLaunchKernelGGL(pargo::sca_cross_kernel, dim3((n + per - 1) / per), threads, 0, ctx->stream, p, n);
-    hipLaunchKernelGGL(pargo::sca_final_kernel, tiles, threads, 0, ctx->stream, p);
+    if (narrow) pargo::launch_sca<true>(p, (unsigned)slots, ctx->stream);
+    else pargo::launch_sca<false>(p, (unsigned)slots, ctx->stream);
     if (last_rule) hipLaunchKernelGGL(pargo::sca_last_cell_kernel, dim3(1), dim3(1), 0, ctx->stream, p);
     return pargo::check_launch(ctx, "pargo_sca_d8");
 }
