@@ -575,7 +575,10 @@ __device__ __forceinline__ void flag_around(const FillParams &p, int tile, unsig
     }
 }
 
-template <int RW>
+// FIRST: pass 0, which does nothing for a DEM that is refused (the host
+// learns it from the same words, passes later): the DEM is left as the init
+// kernel made it, and the later lists stay empty.
+template <int RW, bool FIRST>
 __global__ __launch_bounds__(64 * (kTH / RW), RW == 8 ? 5 : 3) void fill_pass_kernel(FillParams p, int pass)
 {
     __shared__ FillShared<RW> S;
@@ -588,11 +591,8 @@ __global__ __launch_bounds__(64 * (kTH / RW), RW == 8 ? 5 : 3) void fill_pass_ke
         const unsigned o = (unsigned)__shfl_up((int)end, off);
         if (lane >= off) end += o;
     }
-    // a DEM that is refused (the host learns it from the same words, passes
-    // later) is left as the init kernel made it: pass 0 does nothing, so the
-    // lists stay empty
-    const bool refused = pass == 0 && fill_refused(p.range[0], p.range[1], p.nodata);
-    const unsigned n = refused ? 0u : (unsigned)__builtin_amdgcn_readlane((int)end, kSub - 1);
+    unsigned n = (unsigned)__builtin_amdgcn_readlane((int)end, kSub - 1);
+    if (FIRST && fill_refused(p.range[0], p.range[1], p.nodata)) n = 0;
     if (blockIdx.x == 0 && threadIdx.x < kSub) {
         // the counters that pass + 1 fills (pass - 1 read them)
         p.count[((pass + 2) % 3) * kSetWords + lane * kSubStride] = 0;
@@ -713,10 +713,9 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     int per_cu = 0;
     const bool tall = ntiles >= pargo::kTallTiles;
     const int pass_threads = tall ? 128 : 256;
-    if ((tall ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pargo::fill_pass_kernel<16>, pass_threads, 0)
-              : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pargo::fill_pass_kernel<8>, pass_threads, 0)) !=
-            hipSuccess ||
-        per_cu < 1)
+    auto *const first_kernel = tall ? pargo::fill_pass_kernel<16, true> : pargo::fill_pass_kernel<8, true>;
+    auto *const pass_kernel = tall ? pargo::fill_pass_kernel<16, false> : pargo::fill_pass_kernel<8, false>;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pass_kernel, pass_threads, 0) != hipSuccess || per_cu < 1)
         per_cu = 4;
     const int pass_blocks = std::min(ntiles, cus * per_cu);
     // Passes are launched a batch ahead of the one whose outcome is waited
@@ -724,13 +723,9 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     // a batch); passes with nothing on their list, up to a batch of them at
     // the end, take 2 us each.
     auto launch = [&](int first) -> int {
-        for (int k = 0; k < kBatch; k++)
-            if (tall)
-                hipLaunchKernelGGL(pargo::fill_pass_kernel<16>, dim3(pass_blocks), dim3(pass_threads), 0, ctx->stream, p,
-                                   first + k);
-            else
-                hipLaunchKernelGGL(pargo::fill_pass_kernel<8>, dim3(pass_blocks), dim3(pass_threads), 0, ctx->stream, p,
-                                   first + k);
+        for (int k = first; k < first + kBatch; k++)
+            hipLaunchKernelGGL(k == 0 ? first_kernel : pass_kernel, dim3(pass_blocks), dim3(pass_threads), 0, ctx->stream, p,
+                               k);
         const int slot = first / kBatch & 1;
         PARGO_HIP(ctx, hipMemcpyAsync(static_cast<unsigned *>(ctx->report) + 4 * slot, scr, 3 * sizeof(unsigned),
                                       hipMemcpyDeviceToHost, ctx->stream));
