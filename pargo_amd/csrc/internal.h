@@ -79,6 +79,10 @@ hipError_t dev_malloc(void **ptr, size_t bytes, const char *site);
 // " (injected at <site>)" after an injected failure, else "" (clears it).
 const char *injected_note();
 
+// pargo_sca_d8 of a raster of few columns or rows (sca_narrow.hip).
+int sca_narrow(pargo_ctx *ctx, const pargo_grid *g, const uint8_t *flow, const uint32_t *nodata_mask, int mode,
+               double *sca_out);
+
 // Grows the context scratch to at least `bytes`.
 int ensure_scratch(pargo_ctx *ctx, size_t bytes);
 

@@ -140,31 +140,34 @@ struct ScaParams {
     int tiles_x, ntiles;
     int converge;
     double nodata;
-    int w, h, slots;  // NARROW: cells and slots a tile has memory for
+    int w, h, slots;  // with kNarrow: cells and slots a tile has memory for
 };
 
 // Memory of a raster that is one column (of at most 32 cells) or one row (of
 // at most 16) of tiles: at a full tile's 6784 bytes a raster of one column
 // would take 212 bytes a cell.  Such a raster keeps static words for the
 // cells a tile holds and slots for the sides that have a tile beyond them
-// only, 2.4 to 2.9 bytes a cell; its kernels (NARROW) are the same but for
-// the addresses.
+// only, 2.4 to 2.9 bytes a cell.  Its kernels are the same but for these
+// addresses, and are compiled into a code object of their own
+// (sca_narrow.hip): beside them in one object, the kernels of full tiles ran
+// 0.3 % slower (5003 x 7001 layer 397.0 -> 398.4 us).
+#ifdef PARGO_SCA_NARROW
+constexpr bool kNarrow = true;
+#else
+constexpr bool kNarrow = false;
+#endif
 constexpr int kNarrowCols = kTileC / 2, kNarrowRows = kTileR / 2;
-template <bool NARROW>
-__device__ __forceinline__ unsigned slot_stride(const ScaParams &p) { return NARROW ? (unsigned)p.slots : (unsigned)kSlotStride; }
 // A perimeter cell's slot in memory; of the sides without a tile beyond them
 // none is asked for.
-template <bool NARROW>
 __device__ __forceinline__ unsigned mem_slot(const ScaParams &p, int r, int c)
 {
-    if (!NARROW) return (unsigned)slot_of(r, c);
+    if (!kNarrow) return (unsigned)slot_of(r, c);
     return (unsigned)(p.tiles_x == 1 ? (r == 0 ? c : p.w + c) : (c == 0 ? r : p.h + r));
 }
 // Whether a perimeter cell has one (all of a full tile's have).
-template <bool NARROW>
 __device__ __forceinline__ bool has_slot(const ScaParams &p, int r, int c)
 {
-    if (!NARROW) return true;
+    if (!kNarrow) return true;
     return p.tiles_x == 1 ? (r == 0 || r == kTileR - 1) && c < p.w : (c == 0 || c == kTileC - 1) && r < p.h;
 }
 
@@ -449,7 +452,6 @@ union LocalShared {
     unsigned acc[kTileN];  // once the static words are formed
 };
 
-template <bool NARROW>
 __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
 {
     __shared__ LocalShared S;
@@ -468,7 +470,7 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
     if (inner) swar_words(p, S.swar, stw, r0, c0);
     else general_words(p, S.general, stw, r0, c0);
     __syncthreads();
-    const unsigned long long slot0 = (unsigned long long)tile * slot_stride<NARROW>(p);
+    const unsigned long long slot0 = (unsigned long long)tile * (kNarrow ? p.slots : kSlotStride);
     // the pending inflows of this thread's perimeter cell from outside the tile
     const int pcell = tid < kSlots ? cell_of_slot(tid) : 0;
     unsigned ext = 0;
@@ -494,7 +496,7 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
     const unsigned next_ = (unsigned)__builtin_popcount(ext);
     // the static words go out as they are; the tile keeps them with the
     // awaited inflows from inside only
-    if constexpr (NARROW) {
+    if constexpr (kNarrow) {
         for (int i = tid; i < kTileN; i += 256)
             if ((i >> 6) < p.h && (i & 63) < p.w) p.st[((long long)tile * p.h + (i >> 6)) * p.w + (i & 63)] = stw[i];
     } else {
@@ -543,18 +545,18 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
         unsigned t = (unsigned)cell_of_slot((int)slot);
         for (int n = 0; n < kTileN && t < kLeaves; n++) t = nxt[t];
         unsigned at = slot, exit = t >= kLeaves && t != kEnds ? t - kLeaves : 255u;
-        if constexpr (NARROW) {
+        if constexpr (kNarrow) {
             const int in = cell_of_slot((int)slot);
-            at = mem_slot<NARROW>(p, in >> 6, in & 63);
+            at = mem_slot(p, in >> 6, in & 63);
             if (exit != 255u) {
                 const int out = cell_of_slot((int)exit);
-                exit = mem_slot<NARROW>(p, out >> 6, out & 63);
+                exit = mem_slot(p, out >> 6, out & 63);
             }
         }
         p.link[slot0 + at] = (uint8_t)exit;
     }
     __syncthreads();
-    if (NARROW ? tid < kSlots && has_slot<NARROW>(p, pcell >> 6, pcell & 63) : tid < kSlotStride) {
+    if (kNarrow ? tid < kSlots && has_slot(p, pcell >> 6, pcell & 63) : tid < kSlotStride) {
         unsigned long long x = kExitNever;
         unsigned to = kNoExit;
         if (tid < kSlots) {
@@ -563,7 +565,8 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
             if (t >= kLeaves && t != kEnds) {
                 const int gr = r0 + (pcell >> 6) + k / 3 - 1, gc = c0 + (pcell & 63) + k % 3 - 1;
                 const int beside = (gr / kTileR) * p.tiles_x + gc / kTileC;
-                to = (unsigned)beside * slot_stride<NARROW>(p) + mem_slot<NARROW>(p, gr % kTileR, gc % kTileC);
+                to = (unsigned)beside * (unsigned)(kNarrow ? p.slots : kSlotStride) +
+                     mem_slot(p, gr % kTileR, gc % kTileC);
                 if ((v >> kLocPend) == 0) {
                     const unsigned n = (v >> kLocExt) & 255u;
                     if ((v >> kLocBad) & 15u) x = kExitStart | (1ull << kExitBad);  // not done, whatever arrives
@@ -571,7 +574,7 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
                 }
             }
         }
-        const unsigned at = NARROW ? mem_slot<NARROW>(p, pcell >> 6, pcell & 63) : (unsigned)tid;
+        const unsigned at = kNarrow ? mem_slot(p, pcell >> 6, pcell & 63) : (unsigned)tid;
         p.exits[slot0 + at] = x;
         p.next[slot0 + at] = to;
         p.ext[slot0 + at] = (uint8_t)ext;
@@ -581,7 +584,6 @@ __global__ __launch_bounds__(256) void sca_local_kernel(ScaParams p)
 // Each exit's successor: the exit that the perimeter cell it enters leads
 // to, none if that one awaits nothing (it is not done whatever arrives) or
 // never completes.
-template <bool NARROW>
 __global__ __launch_bounds__(256) void sca_link_kernel(ScaParams p, unsigned n)
 {
     const unsigned i = blockIdx.x * 256u + threadIdx.x;
@@ -591,7 +593,8 @@ __global__ __launch_bounds__(256) void sca_link_kernel(ScaParams p, unsigned n)
     const unsigned slot = p.link[to];
     unsigned x = kNoExit;
     if (slot != 255u) {
-        x = to / slot_stride<NARROW>(p) * slot_stride<NARROW>(p) + slot;
+        const unsigned per = (unsigned)(kNarrow ? p.slots : kSlotStride);
+        x = to / per * per + slot;
         const unsigned pend = (unsigned)(p.exits[x] >> kExitPend) & 255u;
         if (pend == 0 || pend == 255u) x = kNoExit;
     }
@@ -640,7 +643,6 @@ __global__ __launch_bounds__(256) void sca_cross_kernel(ScaParams p, unsigned n)
     }
 }
 
-template <bool NARROW>
 __global__ __launch_bounds__(256) void sca_final_kernel(ScaParams p)
 {
     __shared__ unsigned long long acc[kTileN];
@@ -653,26 +655,27 @@ __global__ __launch_bounds__(256) void sca_final_kernel(ScaParams p)
     const int ty = tile / p.tiles_x, tx = tile - ty * p.tiles_x;
     const int r0 = ty * kTileR, c0 = tx * kTileC;
     uint4 words;
-    if constexpr (!NARROW) words = *reinterpret_cast<const uint4 *>(p.st + (long long)tile * kTileN + 8 * tid);
+    if constexpr (!kNarrow) words = *reinterpret_cast<const uint4 *>(p.st + (long long)tile * kTileN + 8 * tid);
     const int pcell = tid < kSlots ? cell_of_slot(tid) : 0;
     // What arrives at this thread's perimeter cell from outside.  The words
     // of its first three inflows are all requested before one is looked at;
     // more than three drain only into a few corners.
-    const unsigned long long slot0 = (unsigned long long)tile * slot_stride<NARROW>(p);
+    const unsigned long long slot0 = (unsigned long long)tile * (kNarrow ? p.slots : kSlotStride);
     auto static_word = [&](int i) -> unsigned {  // of cell i of the tile
-        if constexpr (!NARROW) return p.st[(long long)tile * kTileN + i];
+        if constexpr (!kNarrow) return p.st[(long long)tile * kTileN + i];
         return (i >> 6) < p.h && (i & 63) < p.w ? p.st[((long long)tile * p.h + (i >> 6)) * p.w + (i & 63)] : 0u;
     };
-    const unsigned mine = NARROW ? mem_slot<NARROW>(p, pcell >> 6, pcell & 63) : (unsigned)tid;
-    const unsigned ext = tid < kSlots && has_slot<NARROW>(p, pcell >> 6, pcell & 63) ? p.ext[slot0 + mine] : 0u;
+    const unsigned mine = kNarrow ? mem_slot(p, pcell >> 6, pcell & 63) : (unsigned)tid;
+    const unsigned ext = tid < kSlots && has_slot(p, pcell >> 6, pcell & 63) ? p.ext[slot0 + mine] : 0u;
     const unsigned pword = tid < kSlots ? static_word(pcell) : 0u;
     unsigned long long arrived = 0;
     if (ext) {
         auto word = [&](unsigned e) -> unsigned long long {  // of the lowest inflow in e
             const unsigned k = (unsigned)win_of_bit(__builtin_ctz(e));
             const unsigned gr = (unsigned)(r0 + (pcell >> 6) - 1) + k / 3u, gc = (unsigned)(c0 + (pcell & 63) - 1) + k % 3u;
-            return p.exits[(unsigned long long)((gr / kTileR) * (unsigned)p.tiles_x + gc / kTileC) * slot_stride<NARROW>(p) +
-                           mem_slot<NARROW>(p, (int)(gr % kTileR), (int)(gc % kTileC))];
+            return p.exits[(unsigned long long)((gr / kTileR) * (unsigned)p.tiles_x + gc / kTileC) *
+                               (unsigned)(kNarrow ? p.slots : kSlotStride) +
+                           mem_slot(p, (int)(gr % kTileR), (int)(gc % kTileC))];
         };
         auto arrival = [&](unsigned long long x) -> unsigned long long {
             if (((x >> kExitPend) & 255ull) != 0) return 0;  // never complete
@@ -690,7 +693,7 @@ __global__ __launch_bounds__(256) void sca_final_kernel(ScaParams p)
 #pragma unroll
         for (int q = 0; q < 3; q++) arrived += arrival(x[q]);
     }
-    if constexpr (NARROW) {
+    if constexpr (kNarrow) {
         for (int i = tid; i < kTileN; i += 256) nxt[i] = (uint16_t)static_word(i);
     } else {
         *reinterpret_cast<uint4 *>(nxt + 8 * tid) = words;
@@ -765,6 +768,7 @@ __global__ void sca_last_cell_kernel(ScaParams p)
     p.area[(long long)r * p.pitch + c] = v;
 }
 
+#ifndef PARGO_SCA_NARROW
 // Reference D8 layer (double) to flow classes: NoData when
 // fabs(v - nodata) < 1e-6, valid when > 1e-6 (scaOperator.cpp:48,71), and
 // neither (NaN) marks a cell that takes no inflow.  A valid cell flows to
@@ -817,20 +821,63 @@ bool sca_nodata_ok(double nodata)
     return true;
 }
 
-template <bool NARROW>
-void launch_sca(const ScaParams &p, unsigned n, hipStream_t s)
-{
-    const dim3 tiles(8 * (unsigned)((p.ntiles + 7) / 8)), threads(256);
-    constexpr unsigned per = 256u * kCrossPer;
-    hipLaunchKernelGGL(sca_local_kernel<NARROW>, tiles, threads, 0, s, p);
-    hipLaunchKernelGGL(sca_link_kernel<NARROW>, dim3((n + 255u) / 256u), threads, 0, s, p, n);
-    hipLaunchKernelGGL(sca_cross_kernel, dim3((n + per - 1) / per), threads, 0, s, p, n);
-    hipLaunchKernelGGL(sca_final_kernel<NARROW>, tiles, threads, 0, s, p);
-}
+#endif
 
 }  // namespace
 
+#ifdef PARGO_SCA_NARROW
+int sca_narrow
+#else
+static int sca_full
+#endif
+    (pargo_ctx *ctx, const pargo_grid *g, const uint8_t *flow, const uint32_t *nodata_mask, int mode, double *sca_out)
+{
+    const int tiles_x = (g->cols + kTileC - 1) / kTileC;
+    const long long ntiles = (long long)tiles_x * ((g->rows + kTileR - 1) / kTileR);
+    ScaParams p{};
+    p.w = kNarrow ? std::min(g->cols, kTileC) : kTileC;
+    p.h = kNarrow ? std::min(g->rows, kTileR) : kTileR;
+    p.slots = !kNarrow ? kSlotStride : 2 * (tiles_x == 1 ? p.w : p.h);
+    // scratch: the last-cell flags, the exit words of the perimeter slots, the
+    // tiles' static words (2 bytes per cell, an even number of them) and, per
+    // slot again, its successor, the entry's exit and its inflows from outside
+    constexpr size_t head = 256;
+    const size_t slots = (size_t)ntiles * p.slots, cells = ((size_t)ntiles * p.w * p.h + 1) & ~(size_t)1;
+    const int rc = ensure_scratch(ctx, head + cells * sizeof(uint16_t) + slots * (8 + 4 + 1 + 1));
+    if (rc) return rc;
+    char *scr = static_cast<char *>(ctx->scratch);
+    p.flow = flow;
+    p.mask = nodata_mask;
+    p.area = sca_out;
+    p.last_done = reinterpret_cast<unsigned *>(scr);
+    p.exits = reinterpret_cast<unsigned long long *>(scr + head);
+    p.st = reinterpret_cast<uint16_t *>(p.exits + slots);
+    p.next = reinterpret_cast<unsigned *>(p.st + cells);
+    p.link = reinterpret_cast<uint8_t *>(p.next + slots);
+    p.ext = p.link + slots;
+    p.pitch = g->pitch ? g->pitch : g->cols;
+    p.rows = g->rows;
+    p.cols = g->cols;
+    p.mask_words = (g->cols + 31) / 32;
+    p.tiles_x = tiles_x;
+    p.ntiles = (int)ntiles;
+    p.converge = mode == PARGO_SCA_CONVERGE;
+    p.nodata = g->nodata;
+    const dim3 tiles(8 * (unsigned)((ntiles + 7) / 8)), threads(256);
+    const unsigned n = (unsigned)slots;
+    hipLaunchKernelGGL(sca_local_kernel, tiles, threads, 0, ctx->stream, p);
+    hipLaunchKernelGGL(sca_link_kernel, dim3((n + 255u) / 256u), threads, 0, ctx->stream, p, n);
+    constexpr unsigned per = 256u * kCrossPer;
+    hipLaunchKernelGGL(sca_cross_kernel, dim3((n + per - 1) / per), threads, 0, ctx->stream, p, n);
+    hipLaunchKernelGGL(sca_final_kernel, tiles, threads, 0, ctx->stream, p);
+    if (mode == PARGO_SCA_REFERENCE && g->rows >= 3 && g->cols >= 3)
+        hipLaunchKernelGGL(sca_last_cell_kernel, dim3(1), dim3(1), 0, ctx->stream, p);
+    return check_launch(ctx, "pargo_sca_d8");
+}
+
 }  // namespace pargo
+
+#ifndef PARGO_SCA_NARROW
 
 using pargo::fail;
 
@@ -874,44 +921,13 @@ extern "C" int pargo_sca_d8(pargo_ctx *ctx, const pargo_grid *g, const uint8_t *
                     g->nodata);
     int rc = pargo::bind(ctx);
     if (rc) return rc;
-    const bool last_rule = mode == PARGO_SCA_REFERENCE && g->rows >= 3 && g->cols >= 3;
     const int tiles_x = (g->cols + pargo::kTileC - 1) / pargo::kTileC;
     const long long ntiles = (long long)tiles_x * ((g->rows + pargo::kTileR - 1) / pargo::kTileR);
     if (ntiles > (1ll << 24))
         return fail(ctx, PARGO_E_INVALID, "grid of %d x %d cells needs %lld tiles, more than 2^24", g->rows, g->cols,
                     ntiles);
-    pargo::ScaParams p{};
     const bool narrow = g->cols <= pargo::kNarrowCols || g->rows <= pargo::kNarrowRows;
-    p.w = narrow ? std::min(g->cols, pargo::kTileC) : pargo::kTileC;
-    p.h = narrow ? std::min(g->rows, pargo::kTileR) : pargo::kTileR;
-    p.slots = !narrow ? pargo::kSlotStride : 2 * (tiles_x == 1 ? p.w : p.h);
-    // scratch: the last-cell flags, the exit words of the perimeter slots, the
-    // tiles' static words (2 bytes per cell, an even number of them) and, per
-    // slot again, its successor, the entry's exit and its inflows from outside
-    constexpr size_t head = 256;
-    const size_t slots = (size_t)ntiles * p.slots, cells = ((size_t)ntiles * p.w * p.h + 1) & ~(size_t)1;
-    rc = pargo::ensure_scratch(ctx, head + cells * sizeof(uint16_t) + slots * (8 + 4 + 1 + 1));
-    if (rc) return rc;
-    char *scr = static_cast<char *>(ctx->scratch);
-    p.flow = flow;
-    p.mask = nodata_mask;
-    p.area = sca_out;
-    p.last_done = reinterpret_cast<unsigned *>(scr);
-    p.exits = reinterpret_cast<unsigned long long *>(scr + head);
-    p.st = reinterpret_cast<uint16_t *>(p.exits + slots);
-    p.next = reinterpret_cast<unsigned *>(p.st + cells);
-    p.link = reinterpret_cast<uint8_t *>(p.next + slots);
-    p.ext = p.link + slots;
-    p.pitch = pitch;
-    p.rows = g->rows;
-    p.cols = g->cols;
-    p.mask_words = (g->cols + 31) / 32;
-    p.tiles_x = tiles_x;
-    p.ntiles = (int)ntiles;
-    p.converge = mode == PARGO_SCA_CONVERGE;
-    p.nodata = g->nodata;
-    if (narrow) pargo::launch_sca<true>(p, (unsigned)slots, ctx->stream);
-    else pargo::launch_sca<false>(p, (unsigned)slots, ctx->stream);
-    if (last_rule) hipLaunchKernelGGL(pargo::sca_last_cell_kernel, dim3(1), dim3(1), 0, ctx->stream, p);
-    return pargo::check_launch(ctx, "pargo_sca_d8");
+    return (narrow ? pargo::sca_narrow : pargo::sca_full)(ctx, g, flow, nodata_mask, mode, sca_out);
 }
+
+#endif
