@@ -172,6 +172,7 @@ int pargo_create(int device, pargo_ctx **out)
     pargo_ctx *ctx = pargo::alloc_should_fail("context") ? nullptr : new (std::nothrow) pargo_ctx();
     if (!ctx) return fail(nullptr, PARGO_E_NOMEM, "out of host memory%s", pargo::injected_note());
     ctx->device = device;
+    ctx->fail_launch = pargo::launch_to_fail();
     e = hipSetDevice(device);
     if (e != hipSuccess) {
         delete ctx;

@@ -11,32 +11,32 @@ namespace pargo {
 
 namespace {
 std::mutex g_mu;
-struct Points {
-    std::string seen;  // the variable's value the count refers to
-    long count = 0;    // points reached since `seen` was set
-};
-Points g_allocs, g_launches;
+std::string g_seen;     // the variable's value the count refers to
+long g_count = 0;       // allocation points reached since g_seen was set
 thread_local std::string t_site;
+}  // namespace
 
-bool selected(const char *variable, Points &points, const char *site)
+bool alloc_should_fail(const char *site)
 {
-    const char *v = std::getenv(variable);
+    const char *v = std::getenv("PARGO_FAIL_ALLOC");
     if (!v || !*v) return false;
     std::lock_guard<std::mutex> lock(g_mu);
-    if (points.seen != v) {
-        points.seen = v;
-        points.count = 0;
+    if (g_seen != v) {
+        g_seen = v;
+        g_count = 0;
     }
     const long n = std::strtol(v, nullptr, 10);
     if (n < 1) return false;
-    if (++points.count != n) return false;
+    if (++g_count != n) return false;
     t_site = site;
     return true;
 }
-}  // namespace
 
-bool alloc_should_fail(const char *site) { return selected("PARGO_FAIL_ALLOC", g_allocs, site); }
-bool launch_should_fail(const char *site) { return selected("PARGO_FAIL_LAUNCH", g_launches, site); }
+long launch_to_fail()
+{
+    const char *v = std::getenv("PARGO_FAIL_LAUNCH");
+    return v ? std::strtol(v, nullptr, 10) : 0;
+}
 
 const char *take_injected_site()
 {

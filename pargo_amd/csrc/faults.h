@@ -10,10 +10,10 @@
 // failure is reported and leaves the context usable.  Unset (the normal
 // case), a point costs one getenv.
 //
-// PARGO_FAIL_LAUNCH="<n>" (or "<n>:<tag>") likewise makes the n-th launch of
-// a pass that empties a device queue fail: the queue is then left as the
-// launch before it filled it, which the call reports as PARGO_E_DEVICE and a
-// later call must not see.
+// PARGO_FAIL_LAUNCH="<n>", read by pargo_create, makes the context's n-th
+// launch of a pass that empties a device queue fail: the queue is then left as
+// the launch before it filled it, which the call reports as PARGO_E_DEVICE and
+// a later call must not see.
 #pragma once
 
 #include <cstddef>
@@ -29,8 +29,8 @@ int fail(pargo_ctx *ctx, int code, const char *fmt, ...);
 // True when this allocation point is the one PARGO_FAIL_ALLOC selects.
 bool alloc_should_fail(const char *site);
 
-// True when this launch is the one PARGO_FAIL_LAUNCH selects.
-bool launch_should_fail(const char *site);
+// The number in PARGO_FAIL_LAUNCH (0: none is to fail).
+long launch_to_fail();
 
 // A host allocation point: throws std::bad_alloc when selected.
 inline void alloc_point(const char *site)

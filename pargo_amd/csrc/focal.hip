@@ -1009,10 +1009,10 @@ static void launch_t(const FocalParams &p, const LaunchCfg &cfg, bool vec, hipSt
     }
 }
 
-static hipError_t launch_fixup(const FocalParams &p, const FocalParams *tiles, int ntiles, bool do_slope, bool do_d8,
-                               int cpt, hipStream_t s, unsigned *items = nullptr)
+static hipError_t launch_fixup(pargo_ctx *ctx, const FocalParams &p, const FocalParams *tiles, int ntiles, bool do_slope,
+                               bool do_d8, int cpt, hipStream_t s, unsigned *items = nullptr)
 {
-    if (launch_should_fail("fixup pass")) return hipErrorLaunchFailure;
+    if (ctx->fail_launch > 0 && --ctx->fail_launch == 0) return hipErrorLaunchFailure;
     dim3 block(256), grid(kFixupBlocks);
     const int width = 64 * cpt;
     if (do_slope && do_d8) hipLaunchKernelGGL((focal_fixup_kernel<true, true>), grid, block, 0, s, p, tiles, ntiles, width, items);
@@ -1026,7 +1026,7 @@ static hipError_t launch_fixup(const FocalParams &p, const FocalParams *tiles, i
 static int queue_launched(pargo_ctx *ctx, hipError_t e, const char *name)
 {
     const int rc = e == hipSuccess ? check_launch(ctx, name)
-                                   : fail(ctx, PARGO_E_DEVICE, "%s: %s%s", name, hipGetErrorString(e), injected_note());
+                                   : fail(ctx, PARGO_E_DEVICE, "%s: %s", name, hipGetErrorString(e));
     if (rc) ctx->fix_stale = true;
     return rc;
 }
@@ -1260,7 +1260,7 @@ static int run_focal(pargo_ctx *ctx, const pargo_grid *g, const float *dem, int 
     launch_focal(p, cfg, vec, do_slope, do_d8, ctx->stream);
     rc = in_wave ? check_launch(ctx, name) : queue_launched(ctx, hipSuccess, name);
     if (rc || in_wave) return rc;
-    return queue_launched(ctx, launch_fixup(p, nullptr, 1, do_slope, do_d8, cfg.cpt, ctx->stream), name);
+    return queue_launched(ctx, launch_fixup(ctx, p, nullptr, 1, do_slope, do_d8, cfg.cpt, ctx->stream), name);
 }
 
 // ---- batches ------------------------------------------------------------
@@ -1374,13 +1374,13 @@ static int blocks_c(pargo_ctx *ctx, const BatchPlan &b)
 
 // The persistent sequence: batch kernel, fixup (which leaves the item queue
 // at zero again, as the plan's upload does at first).
-static hipError_t enqueue_batch(const BatchPlan &b, hipStream_t s)
+static hipError_t enqueue_batch(pargo_ctx *ctx, const BatchPlan &b, hipStream_t s)
 {
     if (b.cpt == 2) launch_batch_c<2>(b, s);
     else launch_batch_c<4>(b, s);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_fixup(b.h_tiles[0], b.d_tiles, b.ntiles, b.do_slope, b.do_d8, b.cpt, s, b.d_queue);
+    return launch_fixup(ctx, b.h_tiles[0], b.d_tiles, b.ntiles, b.do_slope, b.do_d8, b.cpt, s, b.d_queue);
 }
 
 // The outcome of a run's launches.  After a failure the item queue may not
@@ -1583,18 +1583,18 @@ static int run_batch(pargo_ctx *ctx, BatchPlan *b, int mode, int rows_per_strip)
         for (int t = 0; t < b->ntiles && e == hipSuccess; t++) {
             const FocalParams &p = b->h_tiles[t];
             launch_focal_h(p, cfg, p.vec != 0, b->do_slope, b->do_d8, b->sm, s);
-            e = launch_fixup(p, nullptr, 1, b->do_slope, b->do_d8, b->cpt, s);
+            e = launch_fixup(ctx, p, nullptr, 1, b->do_slope, b->do_d8, b->cpt, s);
         }
         return queue_launched(ctx, e, "pargo_batch_slope_d8 (per tile)");
     }
     if (mode == PARGO_BATCH_PERSISTENT)
-        return batch_launched(ctx, b, enqueue_batch(*b, s), "pargo_batch_slope_d8 (persistent)");
+        return batch_launched(ctx, b, enqueue_batch(ctx, *b, s), "pargo_batch_slope_d8 (persistent)");
     // The first run of a plan is launched as it is; a batch that is run again
-    // is worth the capture (about 60 us).  So is a run on a stream that the
-    // caller is capturing: its launches go into the caller's graph (a graph
-    // launched there would not).
+    // is worth the capture (about 60 us).  A run on a stream that the caller is
+    // capturing is launched as it is too: its launches go into the caller's
+    // graph (a graph launched there would not).
     if (b->runs++ == 0 || capturing)
-        return batch_launched(ctx, b, enqueue_batch(*b, s), "pargo_batch_slope_d8 (graph)");
+        return batch_launched(ctx, b, enqueue_batch(ctx, *b, s), "pargo_batch_slope_d8 (graph)");
     if (!b->exec) {
         // capture on a private stream so that a caller's legacy default
         // stream can be used for everything else
@@ -1602,7 +1602,7 @@ static int run_batch(pargo_ctx *ctx, BatchPlan *b, int mode, int rows_per_strip)
         PARGO_HIP(ctx, hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
         hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
         if (e == hipSuccess) {
-            e = enqueue_batch(*b, cs);
+            e = enqueue_batch(ctx, *b, cs);
             const hipError_t ended = hipStreamEndCapture(cs, &b->graph);
             if (e == hipSuccess) e = ended;
         }
@@ -1745,7 +1745,7 @@ static int batch_order(pargo_ctx *ctx, const pargo_tile *tiles, int ntiles, int 
             const pargo::FocalParams &p = b->h_tiles[t];
             e = hipEventRecord(ev[2 * t], ctx->stream);
             pargo::launch_focal_h(p, cfg, p.vec != 0, b->do_slope, b->do_d8, b->sm, ctx->stream);
-            if (e == hipSuccess) e = pargo::launch_fixup(p, nullptr, 1, b->do_slope, b->do_d8, b->cpt, ctx->stream);
+            if (e == hipSuccess) e = pargo::launch_fixup(ctx, p, nullptr, 1, b->do_slope, b->do_d8, b->cpt, ctx->stream);
             if (e == hipSuccess) e = hipEventRecord(ev[2 * t + 1], ctx->stream);
         }
         if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);

@@ -33,6 +33,7 @@ struct pargo_ctx {
     hipEvent_t report_event[2] = {nullptr, nullptr};  // recorded behind such a copy
     void *fix_mem = nullptr;  // focal fixup queue (counters + cell list)
     bool fix_stale = false;   // a launch failed that may have left entries in it
+    long fail_launch = 0;     // the fixup launch that is to fail, counted down (faults.h)
     // device address of the static fixup queue of pargo_slope_d8_noalloc on
     // this context's device (resolved once by pargo_create)
     void *noalloc_scratch = nullptr;

@@ -13,40 +13,30 @@ from tests.test_gpu_batch_plans import check, clear, expected
 
 pytestmark = pytest.mark.gpu
 
-_gen = [0]
+
+def failing_context(n):
+    """A context whose n-th launch of a queue-emptying pass fails."""
+    os.environ["PARGO_FAIL_LAUNCH"] = str(n)
+    try:
+        return _lib.Context(0)
+    finally:
+        del os.environ["PARGO_FAIL_LAUNCH"]
 
 
-class failing_launch:
-    """The n-th launch of a queue-emptying pass inside the block fails."""
-
-    def __init__(self, n=1):
-        self.n = n
-
-    def __enter__(self):
-        _gen[0] += 1
-        os.environ["PARGO_FAIL_LAUNCH"] = "%d:%d" % (self.n, _gen[0])
-
-    def __exit__(self, *exc):
-        os.environ.pop("PARGO_FAIL_LAUNCH", None)
-
-
-@pytest.mark.parametrize("mode", [batch.PERSISTENT, batch.GRAPH, batch.PER_TILE])
-@pytest.mark.parametrize("runs_before", [0, 1, 2])
+@pytest.mark.parametrize("mode,runs_before", [(batch.PERSISTENT, 0), (batch.PERSISTENT, 2), (batch.GRAPH, 0),
+                                              (batch.GRAPH, 1), (batch.PER_TILE, 0), (batch.PER_TILE, 1)])
 def test_batch_after_a_failed_fixup_launch(mode, runs_before):
     import torch
-    ctx = _lib.Context(0)
     # enough wave-rows that the waves take items from the queue
     dems = tiles(64, 91, 300, 800)
     ref = expected(dems)
+    # (the second run in graph mode captures the launches)
+    ctx = failing_context(64 * runs_before + 7 if mode == batch.PER_TILE else runs_before + 1)
     b = batch.Batch(dems, ctx=ctx)
     for _ in range(runs_before):
         b.run(mode)
-    with failing_launch(7 if mode == batch.PER_TILE else 1):
-        if mode == batch.GRAPH and runs_before == 2:
-            b.run(mode)  # a replay makes no launch of its own
-        else:
-            with pytest.raises(_lib.PargoError, match="injected at fixup pass"):
-                b.run(mode)
+    with pytest.raises(_lib.PargoError, match="launch failure"):
+        b.run(mode)
     for _ in range(3):
         clear(b)
         b.run(mode)
@@ -55,27 +45,32 @@ def test_batch_after_a_failed_fixup_launch(mode, runs_before):
     ctx.close()
 
 
-def test_rasters_and_batches_share_the_queue():
+@pytest.mark.parametrize("fails", ["batch", "raster"])
+def test_rasters_and_batches_share_the_queue(fails):
     # a batch whose strips for the exact pass stay in the queue, then a single
     # raster that uses it, and the other way round
     import torch
-    ctx = _lib.Context(0)
     dems = tiles(64, 92, 300, 800)
     big = torch.from_numpy(batch.tile_dem(3, 2049, 2050)).cuda()
     big[1000, 1000], big[5, 2040] = 3e13, -2e13
     refs, (rs, rc, _) = expected(dems), focal.slope_d8(big, 30.0, -9999.0)
+    ctx = failing_context(1 if fails == "batch" else 2)
     b = batch.Batch(dems, ctx=ctx)
-    for _ in range(2):
-        with failing_launch(), pytest.raises(_lib.PargoError, match="injected at fixup pass"):
+    if fails == "batch":
+        with pytest.raises(_lib.PargoError, match="launch failure"):
             b.run(batch.PERSISTENT)
-        s, c, _ = focal.slope_d8(big, 30.0, -9999.0, ctx=ctx)
-        torch.cuda.synchronize()
-        assert torch.equal(s, rs) and torch.equal(c, rc)
-        b.run(batch.GRAPH)
-        with failing_launch(), pytest.raises(_lib.PargoError, match="injected at fixup pass"):
+    else:
+        b.run(batch.PERSISTENT)
+        with pytest.raises(_lib.PargoError, match="launch failure"):
             focal.slope_d8(big, 30.0, -9999.0, ctx=ctx)
         clear(b)
-        b.run(batch.GRAPH)
+        b.run(batch.GRAPH)  # the plan of before
         torch.cuda.synchronize()
         check(b, refs)
+    s, c, _ = focal.slope_d8(big, 30.0, -9999.0, ctx=ctx)
+    clear(b)
+    b.run(batch.GRAPH)
+    torch.cuda.synchronize()
+    assert torch.equal(s, rs) and torch.equal(c, rc)
+    check(b, refs)
     ctx.close()

@@ -9,7 +9,7 @@ import pytest
 
 from oracle import pyoracle
 from pargo_amd import _lib, focal, synth
-from tests.test_gpu_launch_faults import failing_launch
+from tests.test_gpu_launch_faults import failing_context
 
 pytestmark = pytest.mark.gpu
 
@@ -51,12 +51,13 @@ def test_queue_and_wave_give_the_same_bits(method, dirtype):
     # the exact pass matters: without it (its launch failed) windows differ
     p = torch.zeros_like(s)
     q = torch.zeros_like(c)
-    L, ctx = _lib.lib(), _lib.default_context(0)
+    L, ctx = _lib.lib(), failing_context(1)
+    ctx.bind_stream()
     g = focal.grid_of(dem, 30.0, ND)
-    with failing_launch():
-        rc = L.pargo_slope_d8(ctx.h, ctypes.byref(g), _lib._ptr(dem), focal.get_slope_algorithm(method), 0, dirtype,
-                              _lib._ptr(p), _lib._ptr(q), None)
+    rc = L.pargo_slope_d8(ctx.h, ctypes.byref(g), _lib._ptr(dem), focal.get_slope_algorithm(method), 0, dirtype,
+                          _lib._ptr(p), _lib._ptr(q), None)
     torch.cuda.synchronize()
+    ctx.close()
     assert rc == _lib.PARGO_E_DEVICE
     differs = (bits(p) != bits(s)) | (q != c)
     near = torch.zeros_like(differs)
@@ -81,7 +82,7 @@ def test_noalloc_queue_gives_the_same_bits():
     z, _ = raster()
     dem = torch.from_numpy(z).cuda()
     ref = focal.slope_d8(dem, 30.0, ND, want_mask=True)
-    L, ctx = _lib.lib(), _lib.Context(0)  # a context without a queue of its own
+    L, ctx = _lib.lib(), failing_context(2)  # a context without a queue of its own
     ctx.bind_stream()
     g = focal.grid_of(dem, 30.0, ND)
     # twice, the second time on what an interrupted call left in the counters
@@ -89,8 +90,7 @@ def test_noalloc_queue_gives_the_same_bits():
         out = [torch.zeros_like(t) for t in ref]
         args = (ctx.h, ctypes.byref(g), _lib._ptr(dem), 0, 0, 256) + tuple(_lib._ptr(t) for t in out)
         if interrupted:
-            with failing_launch():
-                assert L.pargo_slope_d8_noalloc(*args) == _lib.PARGO_E_DEVICE
+            assert L.pargo_slope_d8_noalloc(*args) == _lib.PARGO_E_DEVICE
         ctx.check(L.pargo_slope_d8_noalloc(*args))
         torch.cuda.synchronize()
         for a, b in zip(out, ref):
