@@ -55,16 +55,15 @@
 // change.
 //
 // Measured at 16384^2 on the synthetic DEM: 6.1 ms (19.3 ms with nine-cell
-// windows swept over whole tiles, two launches per pass).  With four waves a
-// tile, 6.8 ms: 0.6 ms init, 6 ms in 32 passes, 525,000 visits of which half
-// change something and 3.3 waves on average load.  A visit that changes
-// nothing reads 26 KB at 5.1 TB/s (0.67 ms for all 131,072 tiles), which is
-// 2.2 ms of the passes; the rest is the evaluations (3.4 rounds a visit), the
-// rows written (4.8 GB) and the 15-20 us a pass of few tiles takes.  Also with four waves: occupancy (4 to
-// 6 waves per SIMD), a tiled layout of W and 16- or 64-row tiles changed nothing or lost
-// (16 rows 11.2 ms, 64 rows 8.9 ms against 7.2); putting a visit off when a
-// neighbour has changed during the pass saved no visits and took 56 passes
-// instead of 32.
+// windows swept over whole tiles, two launches per pass): 0.60 ms init and
+// 5.5 ms in 35 to 40 passes, 534,000 visits of which 54 % change an edge,
+// 2.5 rounds a visit.  A visit that changes nothing reads 26 KB at 5.1 TB/s
+// (0.67 ms for all 131,072 tiles), 2.2 ms of the passes; the rest is the
+// evaluations, the rows written (4.8 GB) and the 15-20 us a pass of few tiles
+// takes.  Measured with four waves a tile (6.8 to 7.2 ms): occupancy (4 to 6
+// waves per SIMD) and a tiled layout of W changed nothing, 16- and 64-row
+// tiles lost (11.2 and 8.9 ms), and putting a visit off when a neighbour has
+// changed during the pass saved no visits.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -78,12 +77,15 @@ namespace {
 constexpr int kTW = 64, kTH = 32;  // tile: 64 columns x 32 rows
 static_assert(kTW == 64, "a lane is a column of the tile");
 // From this many tiles on, a tile is held by two waves of 16 rows instead of
-// four of 8: fewer waves wait for each other at the round's barrier (eight
-// waves of 4 rows took 12.4 ms at 16384^2, four 6.8, two 6.1), but a wave's
-// chain of rows is longer, which a raster that does not fill the GPU many
-// times over waits for.  us, four waves / two: 1000^2 (512 tiles) 438 / 484,
-// 2048^2 678 / 734, 3000 x 4000 (5,922) 1014 / 1057, 5003 x 7001 (17,270)
-// 1785 / 1735, 8192^2 2827 / 2610, 16384^2 6989 / 6173.
+// four of 8 (eight waves of 4 rows took 12.4 ms at 16384^2, four 6.8, two
+// 6.1).  As many visits, but a change crosses fewer bands: 2.5 rounds a visit
+// instead of 3.4, with them 1.08 G VALU instructions instead of 1.43 and
+// 0.75 G scalar ones instead of 1.33, and of the wave cycles (6.7 G instead
+// of 12.9) 51 % wait instead of 60.  A wave's chain of rows is longer, though,
+// which a raster that does not fill the GPU many times over waits for.  us,
+// four waves / two: 1000^2 (512 tiles) 438 / 484, 2048^2 678 / 734,
+// 3000 x 4000 (5,922) 1014 / 1057, 5003 x 7001 (17,270) 1785 / 1735,
+// 8192^2 2827 / 2610, 16384^2 6989 / 6173.
 constexpr int kTallTiles = 16384;
 constexpr double kGap = 0.0005;    // pitRemoveOperator.cpp:36
 constexpr double kStart = 10000.0; // pitRemoveOperator.cpp:41
@@ -720,8 +722,8 @@ extern "C" int pargo_pit_remove(pargo_ctx *ctx, const pargo_grid *g, const float
     const int pass_blocks = std::min(ntiles, cus * per_cu);
     // Passes are launched a batch ahead of the one whose outcome is waited
     // for, so that the GPU does not idle while the host learns it (about 30 us
-    // a batch); passes with nothing on their list, up to a batch of them at
-    // the end, take 2 us each.
+    // a batch); passes with nothing on their list, 8 to 15 of them at the end,
+    // take 2 us each (4.5 with the grid of a large raster).
     auto launch = [&](int first) -> int {
         for (int k = first; k < first + kBatch; k++)
             hipLaunchKernelGGL(k == 0 ? first_kernel : pass_kernel, dim3(pass_blocks), dim3(pass_threads), 0, ctx->stream, p,

@@ -65,7 +65,7 @@
 // received, which is their area.
 //
 // Measured on the headline DEM's codes: 16384^2 in the reference mode 1.96 ms
-// (local 0.94, link 0.07, cross 0.12, final 0.88), 5003 x 7001 in the
+// (local 0.89, link 0.07, cross 0.12, final 0.87), 5003 x 7001 in the
 // converging mode 0.34 ms, and 0.11 ms for the codes of a filled 1501 x 2003
 // DEM, whose paths are long.  One walk over the whole raster with a global
 // atomic or a static word read per hop (33 bytes of HBM traffic, up to 1336
