@@ -102,7 +102,12 @@ int pargo_abi_version(void);
  * One stream at a time: a context's device state (fixup queue, scratch,
  * batch queue) is shared by everything queued through it, so a switch makes
  * the new stream wait (hipStreamWaitEvent) for the work already queued on
- * the old one.  Work for two streams that must overlap needs two contexts. */
+ * the old one.  Work for two streams that must overlap needs two contexts.
+ * A caller's graph that captured work of a context holds the device state the
+ * work uses: memory the context outgrows later is kept for it until
+ * pargo_destroy, and a replay is ordered with the context's other work like a
+ * call.  A call that would have to allocate while the stream is captured is
+ * refused with PARGO_E_DEVICE; run it once before. */
 int pargo_set_stream(pargo_ctx *ctx, void *hip_stream);
 void *pargo_own_stream(const pargo_ctx *ctx);
 int pargo_sync(pargo_ctx *ctx);
@@ -182,10 +187,8 @@ typedef struct {
  * (which takes the FP32-root path for them) and their D8 codes identical.
  * On a stream that the caller is capturing, a batch that was run once before
  * goes into the caller's graph, in every mode (a first run is refused with
- * PARGO_E_DEVICE and leaves the capture intact).  The device memory such a
- * graph reads stays its own until pargo_destroy, whatever runs on the context
- * meanwhile; a replay uses the context like a run, so it is ordered with the
- * context's other work and ends before pargo_destroy. */
+ * PARGO_E_DEVICE and leaves the capture intact).  The device copy of the plan
+ * that such a graph reads stays its own until pargo_destroy. */
 int pargo_batch_slope_d8(pargo_ctx *ctx, const pargo_tile *tiles, int ntiles, int method, int unit, int dirtype,
                          int mode);
 

@@ -65,10 +65,36 @@ const char *injected_note()
     return buf;
 }
 
+int is_capturing(pargo_ctx *ctx, bool *capturing)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    PARGO_HIP(ctx, hipStreamIsCapturing(ctx->stream, &status));
+    *capturing = status != hipStreamCaptureStatusNone;
+    return PARGO_OK;
+}
+
 int ensure_scratch(pargo_ctx *ctx, size_t bytes)
 {
-    if (ctx->scratch_bytes >= bytes) return PARGO_OK;
-    if (ctx->scratch) {
+    bool capturing = false;
+    const int rc = is_capturing(ctx, &capturing);
+    if (rc) return rc;
+    if (ctx->scratch_bytes >= bytes) {
+        ctx->scratch_captured |= capturing;
+        return PARGO_OK;
+    }
+    if (capturing)
+        return fail(ctx, PARGO_E_DEVICE, "a call that needs more scratch cannot be captured: run it once before");
+    if (ctx->scratch && ctx->scratch_captured) {
+        // a caller's graph reads and writes it at every replay
+        try {
+            ctx->captured_mem.push_back(ctx->scratch);
+        } catch (const std::bad_alloc &) {
+            return fail(ctx, PARGO_E_NOMEM, "out of host memory");
+        }
+        ctx->scratch = nullptr;
+        ctx->scratch_bytes = 0;
+        ctx->scratch_captured = false;
+    } else if (ctx->scratch) {
         // The old buffer may still be in use by queued work.
         hipError_t e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) return fail(ctx, PARGO_E_DEVICE, "hipStreamSynchronize: %s", hipGetErrorString(e));
@@ -210,7 +236,7 @@ int pargo_destroy(pargo_ctx *ctx)
         if (e) hipEventDestroy(e);
     pargo::free_batch_plan(ctx);
     pargo::free_batch_mem(ctx);
-    pargo::free_captured_batch_mem(ctx);
+    for (void *m : ctx->captured_mem) hipFree(m);
     if (ctx->fix_mem) hipFree(ctx->fix_mem);
     if (ctx->switch_event) hipEventDestroy(ctx->switch_event);
     if (ctx->own_stream) hipStreamDestroy(ctx->own_stream);

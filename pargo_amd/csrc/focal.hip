@@ -1308,12 +1308,6 @@ void free_batch_mem(pargo_ctx *ctx)
     ctx->batch_mem_bytes = 0;
 }
 
-void free_captured_batch_mem(pargo_ctx *ctx)
-{
-    for (void *m : ctx->batch_captured) hipFree(m);
-    ctx->batch_captured.clear();
-}
-
 template <int CPT, bool DO_SLOPE, int DO_D8, int SM>
 static int batch_blocks(pargo_ctx *ctx)
 {
@@ -1391,14 +1385,6 @@ static int batch_launched(pargo_ctx *ctx, BatchPlan *b, hipError_t e, const char
     const int rc = queue_launched(ctx, e, name);
     if (rc) b->key.clear();
     return rc;
-}
-
-static int is_capturing(pargo_ctx *ctx, bool *capturing)
-{
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    PARGO_HIP(ctx, hipStreamIsCapturing(ctx->stream, &status));
-    *capturing = status != hipStreamCaptureStatusNone;
-    return PARGO_OK;
 }
 
 // The device copy of the batch plan and two page-locked host copies, kept by
@@ -1564,7 +1550,7 @@ static int batch_rows(const pargo_ctx *ctx, const pargo_tile *tiles, int ntiles)
 static void keep_for_capture(pargo_ctx *ctx, BatchPlan *b)
 {
     if (b->captured) return;
-    ctx->batch_captured.push_back(ctx->batch_mem);
+    ctx->captured_mem.push_back(ctx->batch_mem);
     ctx->batch_mem = nullptr;
     ctx->batch_mem_bytes = 0;  // the next plan gets memory of its own
     b->captured = true;

@@ -29,6 +29,10 @@ struct pargo_ctx {
     // Small reusable device scratch owned by the context (grows on demand).
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
+    bool scratch_captured = false;  // a caller's graph holds its address
+    // device memory that callers' graphs hold and the context no longer uses
+    // (scratch it has outgrown, device copies of batch plans)
+    std::vector<void *> captured_mem;
     void *report = nullptr;  // page-locked host words that progress counters are copied to (64 bytes)
     hipEvent_t report_event[2] = {nullptr, nullptr};  // recorded behind such a copy
     void *fix_mem = nullptr;  // focal fixup queue (counters + cell list)
@@ -45,7 +49,6 @@ struct pargo_ctx {
     size_t batch_mem_bytes = 0;
     hipEvent_t batch_copied[2] = {nullptr, nullptr};  // each host copy's last upload
     int batch_slot = 0;
-    std::vector<void *> batch_captured;  // device copies of plans that callers' graphs hold
     int batch_cpt = 4;
     int batch_rows = 32;  // once batch_tuned; by the batch's size before
     int batch_tuned = 0;
@@ -58,7 +61,6 @@ struct pargo_ctx {
 namespace pargo {
 void free_batch_plan(pargo_ctx *ctx);
 void free_batch_mem(pargo_ctx *ctx);
-void free_captured_batch_mem(pargo_ctx *ctx);
 // Resolves ctx->noalloc_scratch with ctx->device current.
 int resolve_noalloc_scratch(pargo_ctx *ctx);
 }
@@ -84,7 +86,11 @@ const char *injected_note();
 int sca_narrow(pargo_ctx *ctx, const pargo_grid *g, const uint8_t *flow, const uint32_t *nodata_mask, int mode,
                double *sca_out);
 
-// Grows the context scratch to at least `bytes`.
+// Whether the caller is capturing the context's stream.
+int is_capturing(pargo_ctx *ctx, bool *capturing);
+
+// Grows the context scratch to at least `bytes` (refused while the caller
+// captures the stream).
 int ensure_scratch(pargo_ctx *ctx, size_t bytes);
 
 // Allocates the context's page-locked report words and their events: a device-to-host copy of
